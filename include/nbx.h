@@ -86,7 +86,9 @@ typedef struct nbx_params {
     int block_size;   /* threads per block of the update stage: 0 (= 256) or a multiple  */
                       /* of 64 in [64, 1024] (the reference's blockSize, main.cu:30)   */
     int force_waves;  /* waves per block of the force kernel: 2, 4 or 8; 0 = 4 in
-                         nbx_create, "keep the current choice" in nbx_set_params        */
+                         nbx_create, "keep the current choice" in nbx_set_params (up to
+                         5,120 groups of 64 bodies the waves of a block share one group,
+                         and their number follows from the groups)                      */
     int build_locked; /* 1: subtrees built by lock-based insertion (compare-and-swap on
                          child slots, Kernels.cu:138-241); 0: from the shared-digit
                          counts of neighbouring sorted keys, one store per slot.  Both

@@ -50,7 +50,7 @@
 //
 // The counting variant (COUNT) also records, per group, the child steps (one
 // step tests one child for the 64 lanes) and the frames of the walk.
-#include "nbx_device.h"
+#include "walk_split.h"
 
 namespace nbx {
 
@@ -235,7 +235,7 @@ __global__ void __launch_bounds__(64 * W) force_kernel(const float4 *__restrict_
         walk_group<KAHAN, COUNT, SOFT, BATCH>(g, threadIdx.x & 63, stk[threadIdx.x >> 6], fnode, fmeta, eps2, &st->fj);
 }
 
-// A group's weight in the split: its recorded child steps, within [1, 2^24].
+// A group's weight in the XCD split: its recorded child steps, within [1, 2^24].
 static __device__ inline int64_t group_cost(int32_t c) { return min(max(c, 1), 1 << 24); }
 
 // Before each force launch: stores the launch's job record and splits its
@@ -331,11 +331,162 @@ static void launch_w(const ForceArgs &a, hipStream_t s, int waves)
     else launch_one<KAHAN, COUNT, SOFT, BATCH, 4>(a, s);
 }
 
+// The same walk with the group's frames shared by the S waves of a workgroup
+// (walk_split.h), for launches of few groups.  Workgroup b walks one group; the
+// groups of an XCD are consecutive.  Every wave sums its own frames as above,
+// the compensated totals of the waves are added in wave order.  Bound by the
+// length of the longest group's chain of rounds (about 1,500 clocks each: the
+// block's trip to the L2, five child steps, the barrier).  Force kernel, one
+// wave per group against S waves: star + disk N = 2,000, 75 -> 18 us (S = 16);
+// 20,011-body sphere 338 -> 84 (16); 32,768-body disk 168 -> 37 (16); sphere
+// 65,536, 395 -> 161 (8); sphere 150,001 at theta 0.7, 240 -> 176 (8);
+// binary + disk 300,007 unsoftened at theta 0.3, 1089 -> 760 (4).
+// The register budget of eight waves per SIMD is worth a few reloads: with 94
+// scalar registers (seven waves) the same kernel was 5-15 % slower, with S = 16
+// 30 % (one workgroup per CU instead of two).
+template <bool KAHAN, bool SOFT, bool BATCH, int S>
+__global__ void __launch_bounds__(64 * S) __attribute__((amdgpu_waves_per_eu(8)))
+force_split_kernel(ForceJob jb, const float4 *__restrict__ fnode, const int2 *__restrict__ fmeta, float eps2,
+                   const DeviceState *st)
+{
+    __shared__ SplitStack<S> L;
+    __shared__ int s_stop;
+    static_assert(sizeof(L.stk) >= sizeof(float) * 3 * 64 * S, "the waves' sums meet in the stack's memory");
+    if (threadIdx.x == 0) s_stop = latched(st);  // one read: the workgroup stays or leaves as a whole
+    __syncthreads();
+    if (s_stop) return;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int g = xcd_swizzle(blockIdx.x, gridDim.x);
+    int first = g * 64, cnt_bodies = min(64, jb.n - first), sys = 0;
+    if (BATCH) {
+        const int4 gr = jb.groups[g];
+        first = gr.x;
+        cnt_bodies = gr.y;
+        sys = gr.z;
+    }
+    const bool valid = lane < cnt_bodies;
+    const int p = valid ? jb.gorder[first + lane] : 0;
+    const float4 me = valid ? jb.nodes4[p] : make_float4(0.f, 0.f, 0.f, 0.f);
+    const uint64_t live = __ballot(valid);
+
+    float sx = 0.f, sy = 0.f, sz = 0.f;  // compensated totals of this wave
+    float cx = 0.f, cy = 0.f, cz = 0.f;
+    float px = 0.f, py = 0.f, pz = 0.f;
+    auto step = [&](const float4 q, const float crit, const uint64_t mask) -> uint64_t {
+        const float dx = q.x - me.x;
+        const float dy = q.y - me.y;
+        const float dz = q.z - me.z;
+        const float d2 = fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, eps2)));
+        const uint64_t ok = __ballot(crit < d2);
+        uint64_t takem = mask & ok;
+        if (!SOFT) takem &= __ballot(d2 > 0.f);
+        const float ri = __builtin_amdgcn_rsqf(SOFT || d2 > 0.f ? d2 : 1.f);
+        float f = q.w * ri * (ri * ri);
+        f = __builtin_amdgcn_inverse_ballot_w64(takem) ? f : 0.f;
+        px = fmaf(f, dx, px);
+        py = fmaf(f, dy, py);
+        pz = fmaf(f, dz, pz);
+        return mask & ~ok;
+    };
+    const int2 rd = jb.frootm[sys];
+    const int rt = __builtin_amdgcn_readfirstlane(rd.x);
+    const uint64_t om = step(jb.froot4[sys], __int_as_float(__builtin_amdgcn_readfirstlane(rd.y)), live);
+    if (wave > 0) px = py = pz = 0.f;  // the root counts once
+    int t = 0;
+    const bool ok = split_walk<S>(L, wave, lane, make_uint4((unsigned)rt, 0u, (unsigned)om, (unsigned)(om >> 32)),
+                                  om != 0, [&](uint4 e, uint4 *out) -> int {
+        const int tag = __builtin_amdgcn_readfirstlane((int)e.x);
+        const int nch = tag & 15, off = tag >> 4;
+        float4 q[8];
+        int2 d[8];
+        load_block(fnode + off, fmeta + off, q, d);
+        // the mask after the block's loads: a wait for it in between would split them
+        asm volatile("" : "+v"(e.z), "+v"(e.w));
+        const uint64_t mask = ((uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)e.w) << 32) |
+                              (uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)e.z);
+        int k = 0;
+        asm volatile("" : "+s"(k));  // a scalar count
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            if (j >= nch) break;
+            const int tj = __builtin_amdgcn_readfirstlane(d[j].x);
+            const uint64_t o = step(q[j], __int_as_float(__builtin_amdgcn_readfirstlane(d[j].y)), mask);
+            if (o) {
+                if (lane == 0) out[k] = make_uint4((unsigned)tj, 0u, (unsigned)o, (unsigned)(o >> 32));
+                k = __builtin_amdgcn_readfirstlane(k + 1);
+            }
+        }
+        if (KAHAN && ++t == 8) {
+            kahan_add(sx, cx, px); kahan_add(sy, cy, py); kahan_add(sz, cz, pz);
+            px = py = pz = 0.f;
+            t = 0;
+        }
+        return k;
+    });
+    // the arguments that only the end needs are read again from the kernel's own
+    // argument block, so that they hold no scalar registers during the walk
+    const __attribute__((address_space(4))) ForceJob *kj =
+        (const __attribute__((address_space(4))) ForceJob *)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(kj));
+    if (!ok && lane == 0) atomicOr(kj->err, kErrStack);
+    if (KAHAN) {
+        kahan_add(sx, cx, px); kahan_add(sy, cy, py); kahan_add(sz, cz, pz);
+    } else {
+        sx = px; sy = py; sz = pz;
+    }
+    __syncthreads();  // the stack is free
+    float *red = reinterpret_cast<float *>(L.stk);
+    red[(3 * wave + 0) * 64 + lane] = sx;
+    red[(3 * wave + 1) * 64 + lane] = sy;
+    red[(3 * wave + 2) * 64 + lane] = sz;
+    __syncthreads();
+    if (wave == 0 && valid) {
+        sx = sy = sz = cx = cy = cz = 0.f;
+#pragma unroll
+        for (int w = 0; w < S; ++w) {
+            kahan_add(sx, cx, red[(3 * w + 0) * 64 + lane]);
+            kahan_add(sy, cy, red[(3 * w + 1) * 64 + lane]);
+            kahan_add(sz, cz, red[(3 * w + 2) * 64 + lane]);
+        }
+        const int i = kj->perm[p];
+        const float G = kj->G;
+        kj->ax[i] = G * sx;
+        kj->ay[i] = G * sy;
+        kj->az[i] = G * sz;
+    }
+}
+
+template <bool KAHAN, bool SOFT, bool BATCH>
+static void launch_split(const ForceArgs &a, hipStream_t s, int S)
+{
+    const int g = a.jb.ngroups;
+    if (S >= 16) force_split_kernel<KAHAN, SOFT, BATCH, 16><<<g, 1024, 0, s>>>(a.jb, a.fnode, a.fmeta, a.eps2, a.st);
+    else if (S >= 8) force_split_kernel<KAHAN, SOFT, BATCH, 8><<<g, 512, 0, s>>>(a.jb, a.fnode, a.fmeta, a.eps2, a.st);
+    else force_split_kernel<KAHAN, SOFT, BATCH, 4><<<g, 256, 0, s>>>(a.jb, a.fnode, a.fmeta, a.eps2, a.st);
+}
+
+// Waves per group.  As many as fill the device (256 CUs of 32 waves) about once,
+// 16 at most.  Each round costs a barrier and the hand-out of the frames, so once
+// the waves of one-wave groups fill the device by themselves the shared walk only
+// adds work: 4,096 groups (sphere of 262,144) 576 us with 4 waves per group
+// against 632 with one, 8,192 groups 1,129 against 1,031 (sphere) and 573 against
+// 600 (disk).  16 waves: 1,024 groups 176 us against 161 with 8; 313 groups 84
+// against 96.
+static int split_waves(int ngroups)
+{
+    return ngroups <= 640 ? 16 : ngroups <= 2560 ? 8 : ngroups <= 5120 ? 4 : 1;
+}
+
 template <bool BATCH>
 static void dispatch(const ForceArgs &a, hipStream_t s, bool kahan, int waves)
 {
     const bool soft = a.eps2 > 0.f;
-    if (a.jb.counts) {
+    const int split = a.jb.counts ? 1 : split_waves(a.jb.ngroups);
+    if (split > 1) {
+        if (kahan) soft ? launch_split<true, true, BATCH>(a, s, split) : launch_split<true, false, BATCH>(a, s, split);
+        else soft ? launch_split<false, true, BATCH>(a, s, split) : launch_split<false, false, BATCH>(a, s, split);
+    } else if (a.jb.counts) {
         if (soft) launch_w<false, true, true, BATCH>(a, s, waves);
         else launch_w<false, true, false, BATCH>(a, s, waves);
     } else if (kahan) {
