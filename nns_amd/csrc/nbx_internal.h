@@ -82,8 +82,7 @@ struct DeviceState {
     int seen;           // bits of err already reported by the host check (not moved to sticky)
     int nsub;           // subtrees found by the top-tree pass
     int ntop;           // top cells (excluding roots): ids [base0, base0 + ntop)
-    int log_next;       // adjoint: next free record of the node-term log
-    int log_count;      // adjoint: records written (sort length)
+    int log_count;      // adjoint: records of the node-term log (sort length)
     // Grid barrier of the top summary: arrivals of its workgroups and their
     // exits; the last workgroup to leave sets both back to 0.
     alignas(128) int tsync;
@@ -150,6 +149,14 @@ struct nbx_context {
     double *adj_ab = nullptr;    // [4 (m_max + 1)] per block: sum over ancestors of G/M and GM - G.X/M
     // node-term log: one record {node, float4} per child step with accepting lanes
     int64_t adj_cap = 0;         // records
+    int adj_nlogs = 1, adj_subcap = 0;  // parts of the log, records of each
+    // binned sums: ids per bin (log2; 0: sorted form), bins, records per tile
+    int adj_shift = 0, adj_nbins = 0, adj_tile = 0;
+    float4 *adj_own = nullptr;   // [n_max] the walk's own part of dL/dx, by sorted position
+    int *adj_next = nullptr;     // next free record of each part, then the work items of the binned sums
+    float4 *adj_sval = nullptr;  // binned sums: values in bin order (ids in adj_sk), tile rows, work items
+    uint16_t *adj_tab = nullptr;
+    int4 *adj_items = nullptr;
     uint32_t *adj_log_id = nullptr, *adj_sk = nullptr, *adj_tk = nullptr;
     float4 *adj_log_val = nullptr;
     int32_t *adj_sv = nullptr, *adj_tv = nullptr;
