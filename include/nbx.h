@@ -134,9 +134,9 @@ int nbx_compute_bounding_box(nbx_context *ctx, int *mutex, float *x, float *y, f
                              float *maxZ, int n, void *stream, float *elapsed_ms);
 
 /* buildTree (KernelsWrapper.cu:136-162, Kernels.cu:157-377): x, y, z and n must be those of
- * the last nbx_compute_bounding_box (NBX_ERR_INVALID otherwise).  Morton keys, stable radix
- * sort of (key, body), then lock-based insertion along the key digits (child slots
- * locked with -2 by compare-and-swap).  Fills child and *index.  Cell sums are left to
+ * the last nbx_compute_bounding_box (NBX_ERR_INVALID otherwise).  Morton keys, stable sort
+ * of (key, body), then the cells from the shared digits of neighbouring keys (or,
+ * build_locked, by lock-based insertion along the key digits).  Fills child and *index.  Cell sums are left to
  * nbx_centre_of_mass. */
 int nbx_build_tree(nbx_context *ctx, float *x, float *y, float *z, float *mass, int *count,
                    int *start, int *child, int *index, float *minX, float *maxX, float *minY,
@@ -178,7 +178,7 @@ int nbx_update(nbx_context *ctx, float *x, float *y, float *z, float *vx, float 
 int nbx_compute_keys(nbx_context *ctx, const float *x, const float *y, const float *z, int n,
                      int key_type, uint64_t *keys, void *stream, float *elapsed_ms);
 
-/* Stable ascending LSD radix sort of n 64-bit keys: sorted_keys and perm (perm[k] = index of
+/* Stable ascending sort of n 64-bit keys: sorted_keys and perm (perm[k] = index of
  * the k-th key).  Scratch comes from the context (n <= n_max). */
 int nbx_sort_keys(nbx_context *ctx, const uint64_t *keys, int n, uint64_t *sorted_keys,
                   int32_t *perm, void *stream, float *elapsed_ms);
@@ -199,11 +199,11 @@ int nbx_star_forces(nbx_context *ctx, const float *sx, const float *sy, const fl
                     const float *mass, float *ax, float *ay, float *az, int n, float g, void *stream,
                     float *elapsed_ms);
 
-/* The sort of nbx_sort_keys (stable ascending LSD radix sort of n 64-bit keys into
+/* The sort of nbx_sort_keys (stable ascending sort of n 64-bit keys into
  * sorted_keys and perm) without a context and without allocating: no counterpart in the
  * reference.  It is for callers that cannot allocate device memory -- code under HIP
  * graph capture, serving loops.  Its scratch is one static device array of the library
- * (12.5 MiB on every GPU it runs on, held until the process ends), found on the current
+ * (12 MiB on every GPU it runs on, held until the process ends), found on the current
  * device at the first call there; n is at most 1,048,576 (NBX_ERR_INVALID above, message
  * in nbx_last_error(NULL)).  keys, sorted_keys and perm are device arrays on the current
  * device; stream (NULL = the null stream) must belong to it.  Every call on one GPU

@@ -29,7 +29,7 @@ COMMON = [
     "-Wall", "-Wno-unused-function", "-I", os.path.join(ROOT, "include"),
 ]
 
-SOURCES = ["k_basic.hip", "k_radix.hip", "k_tree.hip", "k_force.hip", "k_adjoint.hip", "nbx_api.cpp", "nbx_batch.cpp",
+SOURCES = ["k_basic.hip", "k_radix.hip", "k_sort.hip", "k_tree.hip", "k_force.hip", "k_adjoint.hip", "nbx_api.cpp", "nbx_batch.cpp",
            "nbx_ics.cpp", "k_probe.hip", "nbx_static.hip"]
 
 

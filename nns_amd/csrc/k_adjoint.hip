@@ -864,8 +864,8 @@ void launch_vjp(nbx_context *c, hipStream_t s, const float *ux, const float *uy,
     } else {
         log_count_kernel<<<1, 1, 0, s>>>(c->st, c->adj_next, c->adj_subcap);
         uint32_t *tk = passes % 2 ? c->adj_log_id : c->adj_tk;  // the input keys are dead after the first pass
-        launch_radix_passes(c->adj_hist, s, c->adj_log_id, nullptr, (int)c->adj_cap, 0, passes, c->adj_sk, c->adj_sv,
-                            tk, c->adj_tv, nullptr, &c->st->log_count);
+        launch_radix_passes(c->adj_hist, s, c->adj_log_id, (int)c->adj_cap, passes, c->adj_sk, c->adj_sv, tk, c->adj_tv,
+                            &c->st->log_count);
         const int64_t waves = (c->adj_cap + 64 * kReduceTiles - 1) / (64 * kReduceTiles);
         log_reduce_kernel<<<(int)std::min<int64_t>((waves + 3) / 4, 65536), 256, 0, s>>>(
             c->adj_sk, c->adj_sv, c->adj_log_val, c->st, v.sentinel, c->adj_tgt);

@@ -148,14 +148,13 @@ __global__ void __launch_bounds__(256) bbox_fold_kernel(const float *__restrict_
     }
 }
 
-// Keys, and (x, y, z, m) packed as float4 for the one-line gather of the layout.
+// Keys of nbx_compute_keys (the build makes its own in the sort's first launch).
 // Hilbert keys map the Morton key through the state table in LDS; Morton keys
 // need neither the table nor the barrier after its fill.
 template <bool HILBERT>
 __global__ void __launch_bounds__(256) keys_kernel(
-    const float *__restrict__ x, const float *__restrict__ y, const float *__restrict__ z,
-    const float *__restrict__ mass, int n, const DeviceState *__restrict__ st,
-    uint64_t *__restrict__ keys, float4 *__restrict__ bodies4)
+    const float *__restrict__ x, const float *__restrict__ y, const float *__restrict__ z, int n,
+    const DeviceState *__restrict__ st, uint64_t *__restrict__ keys)
 {
     __shared__ uint8_t s_tab[HILBERT ? kHilbertTable : 1];
     if (HILBERT) {
@@ -168,7 +167,6 @@ __global__ void __launch_bounds__(256) keys_kernel(
         uint64_t k = morton_key(xi, yi, zi, ext);
         if (HILBERT) k = hilbert_top_lds(k & ~(1ull << 63), kKeyLevels, s_tab);
         keys[i] = k;
-        if (mass) bodies4[i] = make_float4(xi, yi, zi, mass[i]);
     }
 }
 
@@ -323,14 +321,14 @@ void launch_bbox(nbx_context *c, hipStream_t s, const float *x, const float *y, 
     bbox_fold_kernel<<<1, block, 0, s>>>(c->bbox_part, g, c->st, minX, maxX, minY, maxY, minZ, maxZ);
 }
 
-void launch_keys(nbx_context *c, hipStream_t s, const float *x, const float *y, const float *z, const float *mass,
-                 int n, int key_type, uint64_t *keys)
+void launch_keys(nbx_context *c, hipStream_t s, const float *x, const float *y, const float *z, int n, int key_type,
+                 uint64_t *keys)
 {
     const int block = 256;
     if (key_type == NBX_KEY_HILBERT)
-        keys_kernel<true><<<grid_for(n, block, 65536), block, 0, s>>>(x, y, z, mass, n, c->st, keys, c->bodies4);
+        keys_kernel<true><<<grid_for(n, block, 65536), block, 0, s>>>(x, y, z, n, c->st, keys);
     else
-        keys_kernel<false><<<grid_for(n, block, 65536), block, 0, s>>>(x, y, z, mass, n, c->st, keys, c->bodies4);
+        keys_kernel<false><<<grid_for(n, block, 65536), block, 0, s>>>(x, y, z, n, c->st, keys);
 }
 
 void launch_update(hipStream_t s, int block, const DeviceState *st, float *x, float *y, float *z, float *vx, float *vy,
@@ -420,20 +418,6 @@ __global__ void __launch_bounds__(256) bbox_batch_fold_kernel(int S, const int32
     ext[4 * s + 0] = v[0]; ext[4 * s + 1] = v[2]; ext[4 * s + 2] = v[4]; ext[4 * s + 3] = sp;
 }
 
-__global__ void __launch_bounds__(256) keys_batch_kernel(
-    const float *__restrict__ x, const float *__restrict__ y, const float *__restrict__ z,
-    const float *__restrict__ mass, int n, const int32_t *__restrict__ sys_of, const double *__restrict__ ext,
-    uint64_t *__restrict__ keys, float4 *__restrict__ bodies4)
-{
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += blockDim.x * gridDim.x) {
-        const int s = sys_of[i];
-        const double e[4] = {ext[4 * s], ext[4 * s + 1], ext[4 * s + 2], ext[4 * s + 3]};
-        const float xi = x[i], yi = y[i], zi = z[i];
-        keys[i] = morton_key(xi, yi, zi, e);
-        bodies4[i] = make_float4(xi, yi, zi, mass[i]);
-    }
-}
-
 void launch_batch_reset(nbx_batch *b, hipStream_t s)
 {
     reset_batch_kernel<<<grid_for(b->S, 256, 1024), 256, 0, s>>>(b->S, b->N, b->child, b->index, b->cell_level,
@@ -444,12 +428,6 @@ void launch_batch_bbox(nbx_batch *b, hipStream_t s)
 {
     bbox_batch_kernel<<<b->nchunk, 256, 0, s>>>(b->x, b->y, b->z, b->bchunk, b->bpart, b->st);
     bbox_batch_fold_kernel<<<(b->S + 255) / 256, 256, 0, s>>>(b->S, b->bchunk_off, b->bpart, b->mm, b->ext);
-}
-
-void launch_batch_keys(nbx_batch *b, hipStream_t s)
-{
-    keys_batch_kernel<<<grid_for(b->N, 256, 65536), 256, 0, s>>>(b->x, b->y, b->z, b->mass, b->N, b->sys_of,
-                                                                 b->ext, b->keys, b->bodies4);
 }
 
 }  // namespace nbx

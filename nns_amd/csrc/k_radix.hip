@@ -1,13 +1,13 @@
-// k_radix.hip -- stable LSD radix sort of (64- or 32-bit key, int32 index) pairs.
+// k_radix.hip -- stable LSD radix sort of (32-bit key, index) pairs with a
+// device-side count (the node-term log of the adjoint), and the scans of the tree build.
 //
 // Passes of kRadixBits = 8 bits.  Each pass is three launches over tiles of 2048
 // keys (4 waves x 8 items x 64 lanes; wave w owns the contiguous quarter w of the
 // tile, walked item by item so that lane order is element order):
-//   upsweep   per-tile digit histogram (LDS atomics) reads 8 B/key (64-bit keys)
+//   upsweep   per-tile digit histogram (LDS atomics) reads 4 B/key
 //   scan      exclusive scan of each digit row       ~1 KiB per tile
 //   downsweep stable rank, the tile reordered by digit in LDS, then written out
-//             digit run by digit run (coalesced)  reads 12 B/key, writes 12 B/key
-// (32-bit keys: 4 and 8 B/key).
+//             digit run by digit run (coalesced)  reads 8 B/key, writes 8 B/key
 // In the downsweep, ranks inside a wave come from a 64-lane match of the digit
 // built from kRadixBits ballots (no atomics, no intra-wave waits), so equal
 // digits keep their order; the upsweep needs counts only and takes them with
@@ -31,9 +31,8 @@ __device__ inline uint64_t match_digit(uint32_t digit, uint64_t live)
     return peers;
 }
 
-template <class K>
 __global__ void __launch_bounds__(kSortThreads) radix_upsweep(
-    const K *__restrict__ keys, int n, int shift, int ntiles, uint32_t *__restrict__ hist,
+    const uint32_t *__restrict__ keys, int n, int shift, int ntiles, uint32_t *__restrict__ hist,
     const int *__restrict__ n_dev)
 {
     __shared__ uint32_t cnt[kSortThreads / 64][kRadix];
@@ -127,11 +126,10 @@ __global__ void __launch_bounds__(256) scan_add_kernel(uint32_t *__restrict__ da
         if (base + j < total) data[base + j] += off;
 }
 
-template <class K>
 __global__ void __launch_bounds__(kSortThreads) radix_downsweep(
-    const K *__restrict__ kin, const int32_t *__restrict__ vin, int n, int shift, int ntiles,
-    const uint32_t *__restrict__ hist, const uint32_t *__restrict__ rowsum, K *__restrict__ kout,
-    int32_t *__restrict__ vout, int32_t *__restrict__ inv, const int *__restrict__ n_dev)
+    const uint32_t *__restrict__ kin, const int32_t *__restrict__ vin, int n, int shift, int ntiles,
+    const uint32_t *__restrict__ hist, const uint32_t *__restrict__ rowsum, uint32_t *__restrict__ kout,
+    int32_t *__restrict__ vout, const int *__restrict__ n_dev)
 {
     if (n_dev) n = min(n, *n_dev);
     if ((int64_t)blockIdx.x * kSortTile >= n) return;  // no keys in this tile
@@ -140,7 +138,7 @@ __global__ void __launch_bounds__(kSortThreads) radix_downsweep(
     __shared__ uint32_t dbase[kRadix];
     __shared__ uint32_t gdelta[kRadix];
     __shared__ uint32_t scan_sh[kSortThreads];
-    __shared__ K s_key[kSortTile];
+    __shared__ uint32_t s_key[kSortTile];
     __shared__ int32_t s_val[kSortTile];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     for (int k = tid; k < W * kRadix; k += kSortThreads) (&run[0][0])[k] = 0u;
@@ -164,7 +162,7 @@ __global__ void __launch_bounds__(kSortThreads) radix_downsweep(
     __syncthreads();
     const int64_t base = (int64_t)blockIdx.x * kSortTile + (int64_t)wave * (kSortItems * 64);
     const uint64_t lt = lanemask_lt(lane);
-    K key[kSortItems];
+    uint32_t key[kSortItems];
     int32_t val[kSortItems];
     uint32_t rank[kSortItems];
     uint32_t dig[kSortItems];
@@ -172,7 +170,7 @@ __global__ void __launch_bounds__(kSortThreads) radix_downsweep(
     for (int i = 0; i < kSortItems; ++i) {
         const int64_t e = base + i * 64 + lane;
         const bool valid = e < n;
-        key[i] = valid ? kin[e] : K(0);
+        key[i] = valid ? kin[e] : 0u;
         val[i] = valid ? (vin ? vin[e] : (int32_t)e) : 0;
         const uint32_t d = (uint32_t)((key[i] >> shift) & (kRadix - 1));
         dig[i] = d;
@@ -232,88 +230,35 @@ __global__ void __launch_bounds__(kSortThreads) radix_downsweep(
     const int64_t t0 = (int64_t)blockIdx.x * kSortTile;
     const int tn = (int)min((int64_t)kSortTile, (int64_t)n - t0);
     for (int j = tid; j < tn; j += kSortThreads) {
-        const K k = s_key[j];
+        const uint32_t k = s_key[j];
         const int32_t v = s_val[j];
         const uint32_t d = (uint32_t)((k >> shift) & (kRadix - 1));
         const uint32_t p = (uint32_t)j + gdelta[d];
         kout[p] = k;
         vout[p] = v;
-        if (inv) inv[v] = (int32_t)p;
     }
 }
 
-template <class K>
-void launch_radix_passes(uint32_t *hist, hipStream_t s, const K *keys_in, const int32_t *vals_in, int n,
-                         int first_shift, int npasses, K *keys_out, int32_t *vals_out, K *tmp_k,
-                         int32_t *tmp_v, int32_t *inv_out, const int *n_dev)
+void launch_radix_passes(uint32_t *hist, hipStream_t s, const uint32_t *keys_in, int n, int npasses, uint32_t *keys_out,
+                         int32_t *vals_out, uint32_t *tmp_k, int32_t *tmp_v, const int *n_dev)
 {
     if (n <= 0 || npasses <= 0) return;
     const int ntiles = (n + kSortTile - 1) / kSortTile;
-    const K *ki = keys_in;
-    const int32_t *vi = vals_in;
+    const uint32_t *ki = keys_in;
+    const int32_t *vi = nullptr;
     for (int p = 0; p < npasses; ++p) {
-        const int shift = first_shift + p * kRadixBits;
-        const bool last = (p == npasses - 1);
+        const int shift = p * kRadixBits;
         // alternate so that the last pass lands in keys_out / vals_out
         const bool to_out = ((npasses - 1 - p) % 2) == 0;
-        K *ko = to_out ? keys_out : tmp_k;
+        uint32_t *ko = to_out ? keys_out : tmp_k;
         int32_t *vo = to_out ? vals_out : tmp_v;
         uint32_t *rowsum = hist + (int64_t)ntiles * kRadix;  // kRadix totals after the rows
-        radix_upsweep<K><<<ntiles, kSortThreads, 0, s>>>(ki, n, shift, ntiles, hist, n_dev);
+        radix_upsweep<<<ntiles, kSortThreads, 0, s>>>(ki, n, shift, ntiles, hist, n_dev);
         radix_rows_scan<<<kRadix, 256, 0, s>>>(hist, ntiles, rowsum, n, n_dev);
-        radix_downsweep<K><<<ntiles, kSortThreads, 0, s>>>(ki, vi, n, shift, ntiles, hist, rowsum, ko, vo,
-                                                        last ? inv_out : nullptr, n_dev);
+        radix_downsweep<<<ntiles, kSortThreads, 0, s>>>(ki, vi, n, shift, ntiles, hist, rowsum, ko, vo, n_dev);
         ki = ko;
         vi = vo;
     }
-}
-
-template void launch_radix_passes<uint64_t>(uint32_t *, hipStream_t, const uint64_t *, const int32_t *, int, int, int,
-                                            uint64_t *, int32_t *, uint64_t *, int32_t *, int32_t *, const int *);
-template void launch_radix_passes<uint32_t>(uint32_t *, hipStream_t, const uint32_t *, const int32_t *, int, int, int,
-                                            uint32_t *, int32_t *, uint32_t *, int32_t *, int32_t *, const int *);
-
-// Batched form: after the 8 key passes, stable passes over the system index
-// (32-bit keys, one pass per 8 bits of it) group every system's bodies, in key
-// order, at [off[s], off[s+1]).
-__global__ void __launch_bounds__(256) system_key_kernel(int n, const int32_t *__restrict__ perm,
-                                                         const int32_t *__restrict__ sys_of,
-                                                         uint32_t *__restrict__ k2)
-{
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += blockDim.x * gridDim.x)
-        k2[k] = (uint32_t)sys_of[perm[k]];
-}
-
-__global__ void __launch_bounds__(256) gather_sorted_kernel(int n, const int32_t *__restrict__ perm,
-                                                            const uint64_t *__restrict__ keys,
-                                                            uint64_t *__restrict__ skeys,
-                                                            int32_t *__restrict__ pos)
-{
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += blockDim.x * gridDim.x) {
-        const int b = perm[k];
-        skeys[k] = keys[b];
-        pos[b] = k;
-    }
-}
-
-void launch_batch_sort(nbx_batch *b, hipStream_t s)
-{
-    const int n = b->N;
-    int g = (n + 255) / 256;
-    if (g > 65536) g = 65536;
-    // 1. stable sort of (key, body) over the 63 key bits below the constant top bit
-    launch_radix_passes(b->hist, s, b->keys, nullptr, n, 0, (kMortonSortBits + kRadixBits - 1) / kRadixBits,
-                        b->skeys, b->perm1, b->kbuf, b->vbuf, nullptr);
-    // 2. stable sort by system: 32-bit keys, one pass up to 256 systems, two up to 65536
-    int sys_bits = 0;
-    while ((1 << sys_bits) < b->S) ++sys_bits;
-    const int sys_passes = sys_bits > kRadixBits ? 2 : 1;
-    uint32_t *k2 = reinterpret_cast<uint32_t *>(b->k2);
-    system_key_kernel<<<g, 256, 0, s>>>(n, b->perm1, b->sys_of, k2);
-    launch_radix_passes(b->hist, s, k2, b->perm1, n, 0, sys_passes, reinterpret_cast<uint32_t *>(b->k2buf), b->perm,
-                        reinterpret_cast<uint32_t *>(b->kbuf), b->vbuf, nullptr);
-    // 3. keys in (system, key) order and the inverse permutation
-    gather_sorted_kernel<<<g, 256, 0, s>>>(n, b->perm, b->keys, b->skeys, b->pos);
 }
 
 // Exclusive scan of `total` uint32 in place by one workgroup of 1024 threads,
@@ -355,13 +300,6 @@ void launch_exclusive_scan_u32(uint32_t *data, int total, uint32_t *sums, hipStr
     scan_blocks_kernel<<<nb, 256, 0, s>>>(data, total, sums);
     scan_sums_kernel<<<1, 1024, 0, s>>>(sums, nb);
     scan_add_kernel<<<nb, 256, 0, s>>>(data, total, sums);
-}
-
-void launch_radix_sort(nbx_context *c, hipStream_t s, const uint64_t *keys_in, int n, uint64_t *keys_out,
-                       int32_t *perm_out, uint64_t *tmp_k, int32_t *tmp_v, int32_t *inv_out, int key_bits)
-{
-    launch_radix_passes(c->hist, s, keys_in, nullptr, n, 0, (key_bits + kRadixBits - 1) / kRadixBits, keys_out,
-                        perm_out, tmp_k, tmp_v, inv_out);
 }
 
 }  // namespace nbx

@@ -132,18 +132,70 @@ __global__ void __launch_bounds__(256) top_cells_kernel(Segs g, int nsamples, co
     }
 }
 
+// Group order of the force walk.  The walk gives each wave 64 consecutive
+// bodies of this order.  Key order has jumps (consecutive Morton keys can lie in
+// cells far apart), so bodies are ordered by the top kGroupLevels Hilbert digits
+// of their key instead, stably over key order (ties keep key order), each system
+// by itself.  The order changes which bodies share a wave, never a body's
+// interaction list.
+//
+// A cell's bodies are a range of this order too, and its children's ranges follow
+// each other in the order of their Hilbert digits, so the order is read off the
+// tree: in state s (a function of the cell's key digits) a child's range starts at its
+// cell's plus the counts of the children with smaller digits (its offset), and a
+// body's place is the sum of the offsets on its way up.  Below level kGroupLevels the
+// digit is the slot (state kPlain).  The build leaves the offsets of the top cells and
+// of the subtrees (top_wire_kernel, which has the child ranges in hand); here a
+// workgroup takes a subtree: one thread per cell for the offsets of its children, then
+// one per body for the sum.  No keys are made and nothing is sorted: the order takes
+// 20 us at N = 2,000, 31 at 1M and 98 at 4M, where Hilbert keys and four radix passes (13
+// launches) took 51, 138 and 245.  Placing the cells level by level instead took 34,
+// 74 and 258 us: few of a level's lanes have a cell.
+constexpr int kPlain = 12;
+
+// Digit of each slot and state of each child, a nibble per slot, by state.
+struct OrderTables {
+    uint32_t dig[kPlain + 1], next[kPlain + 1];
+};
+__device__ inline void order_tables_fill(OrderTables &o)
+{
+    const int t = threadIdx.x;
+    if (t <= kPlain) {
+        uint32_t dig = 0, next = 0;
+        for (int s = 0; s < 8; ++s) {
+            dig |= (uint32_t)(t < kPlain ? c_hil[t][s] : s) << (4 * s);
+            next |= (uint32_t)(t < kPlain ? c_dir[t][s] : kPlain) << (4 * s);
+        }
+        o.dig[t] = dig;
+        o.next[t] = next;
+    }
+}
+// State of the level-`to` cell of `key` from that of its level-`from` cell.
+__device__ inline int order_state(const OrderTables &o, uint64_t key, int state, int from, int to)
+{
+    if (to >= kGroupLevels) return kPlain;
+    for (int L = from; L < to; ++L) state = (int)(o.next[state] >> (4 * digit_at(key, L))) & 15;
+    return state;
+}
+
 // Wires every top cell (and every root): child ranges by digit L; a range of
 // one body is a leaf, of more than kSubtreeMax a top cell, otherwise a subtree
 // queued for the subtree build.  Eight lanes per entry, lane d for digit d: each
 // finds the end of its digit's range by one binary search over the cell's
 // range and takes its start from the lane before (the searches run side by
 // side, not one after another).  Thread 0 also sets *index past the top cells.
+// Every child's place in the group order is left relative to its parent's: {offset,
+// the parent's number among the top cells}, or {place, -1} under a root.
 __global__ void __launch_bounds__(256) top_wire_kernel(
     Segs g, int nsamples, const uint64_t *__restrict__ skeys, const int32_t *__restrict__ perm, int *child,
     int32_t *__restrict__ cell_level, const uint32_t *__restrict__ flag, const uint32_t *__restrict__ id,
     const int32_t *__restrict__ ta, const int32_t *__restrict__ tb, int4 *__restrict__ sub, int sub_max,
-    int base0, int m, int *index, int *__restrict__ start, DeviceState *st)
+    int base0, int m, int *index, int *__restrict__ start, int2 *__restrict__ top_place,
+    int2 *__restrict__ sub_place, DeviceState *st)
 {
+    __shared__ OrderTables tab;
+    order_tables_fill(tab);
+    __syncthreads();
     if (latched(st)) return;
     const int total = nsamples * kLevels;
     const int gt = blockIdx.x * blockDim.x + threadIdx.x;
@@ -190,6 +242,13 @@ __global__ void __launch_bounds__(256) top_wire_kernel(
     const int up = __shfl_up(db, 1, 8);
     const int da = d == 0 ? a : up;
     const int cnt = db - da;
+    const uint32_t dig = tab.dig[order_state(tab, skeys[a], 0, 0, L)];
+    int below = 0;
+    for (int o = 0; o < 8; ++o) {
+        const int w = __shfl(cnt, o, 8);
+        below += ((int)(dig >> (4 * o)) & 7) < ((int)(dig >> (4 * d)) & 7) ? w : 0;
+    }
+    const int2 place = t < total ? make_int2(below, (int)id[t]) : make_int2(a + below, -1);
     const int64_t slot = 8 * (int64_t)c + d;
     if (cnt == 0) {
         child[slot] = -1;
@@ -197,12 +256,18 @@ __global__ void __launch_bounds__(256) top_wire_kernel(
         child[slot] = perm[da];
     } else if (cnt > kSubtreeMax) {
         const int kk = samp_lo(g, s) + (da - lo + kSubtreeMax - 1) / kSubtreeMax;
-        child[slot] = base0 + (int)id[(L + 1) * nsamples + kk];
+        const int tc = (int)id[(L + 1) * nsamples + kk];
+        child[slot] = base0 + tc;
+        top_place[tc] = place;
     } else {
         child[slot] = -1;  // set by the subtree build
         const int i = atomicAdd(&st->nsub, 1);
-        if (i < sub_max) sub[i] = make_int4(da, db, L + 1, (int)slot);
-        else atomicOr(&st->err, kErrCapacity);
+        if (i < sub_max) {
+            sub[i] = make_int4(da, db, L + 1, (int)slot);
+            sub_place[i] = place;
+        } else {
+            atomicOr(&st->err, kErrCapacity);
+        }
     }
 }
 
@@ -935,8 +1000,8 @@ __global__ void __launch_bounds__(256) top_summary_kernel(SumOut o, Segs g, int 
 
 // ------------------------------------------------------------------ layout
 // Bodies in key order as float4 (x, y, z, m) at nodes4[0..n), made right after
-// the build for the summary; sorted[] (the reference's output of the sort
-// stage) in the sort stage; then the frame blocks of the force walk
+// the build for the summary; in the sort stage sorted[] (the reference's output of
+// that stage) with the group order, and the frame blocks of the force walk
 // (frame_layout_kernel).  The bodies are read in input order and stored at
 // their sorted positions pos[] (the sort's inverse permutation): random 16-byte
 // reads each fetch a whole line, random 16-byte stores only dirty their bytes.
@@ -946,13 +1011,6 @@ __global__ void __launch_bounds__(256) sorted_bodies_kernel(int n, const int32_t
 {
     if (latched(st)) return;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += blockDim.x * gridDim.x) nodes4[pos[i]] = bodies4[i];
-}
-
-__global__ void __launch_bounds__(256) sorted_index_kernel(int n, const int32_t *__restrict__ perm,
-                                                           int *__restrict__ sorted, const DeviceState *st)
-{
-    if (latched(st)) return;
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += blockDim.x * gridDim.x) sorted[k] = perm[k];
 }
 
 // Frame blocks.  Block b lists the non-empty children of one cell, compacted in
@@ -1093,10 +1151,10 @@ __device__ inline int2 chain_bottom_from(int c, int4 a, int4 b, int lev, int n, 
     }
 }
 
-// Ensemble: the system of a cell from its first sorted body, whose group key
-// (made before the layout) holds the system index above the Hilbert digits.
+// Ensemble: the system of a cell from its first sorted position (sorting leaves every
+// system's bodies in the system's own positions, so sys_of holds for both orders).
 struct SysInfo {
-    const uint64_t *gkey;
+    const int32_t *sys_of;
     const float *theta;
     const double *ext;
 };
@@ -1152,7 +1210,7 @@ __global__ void __launch_bounds__(256) frame_layout_kernel(
         double span;
         float th;
         if (BATCH) {
-            const int sys = item < nroot ? (int)item : (int)(si.gkey[nstart] >> (3 * kGroupLevels));
+            const int sys = item < nroot ? (int)item : si.sys_of[nstart];
             span = si.ext[4 * sys + 3];
             th = si.theta[sys];
         } else {
@@ -1180,34 +1238,122 @@ __global__ void __launch_bounds__(256) frame_layout_kernel(
     }
 }
 
-// Group order of the force walk.  The walk gives each wave 64 consecutive
-// bodies of this order.  Key order has jumps (consecutive Morton keys can lie in
-// cells far apart), so bodies are ordered by the top kGroupLevels Hilbert digits
-// of their key instead, stably over key order (ties keep key order); the
-// ensemble puts the system index above them.  The order changes which bodies
-// share a wave, never a body's interaction list.  A single system's keys
-// (3 kGroupLevels = 30 bits) are sorted as 32-bit keys.
-template <class K>
-__global__ void __launch_bounds__(256) group_keys_kernel(int n, const uint64_t *__restrict__ skeys,
-                                                         const int32_t *__restrict__ perm,
-                                                         const int32_t *__restrict__ sys_of,
-                                                         K *__restrict__ gkey, const DeviceState *st)
+// Also writes sorted[] (the reference's output of the sort stage).  A subtree of
+// more than kOrdCells cells (chains of one-child cells) keeps its cells' offsets in
+// `place`, one word per cell.
+constexpr int kOrdCells = 1024;
+__global__ void __launch_bounds__(256) group_order_kernel(Segs g, int base0, const uint64_t *__restrict__ skeys,
+                                                          const int4 *__restrict__ sub,
+                                                          const int4 *__restrict__ subcells,
+                                                          const int *__restrict__ child, const int *__restrict__ count,
+                                                          const int *__restrict__ start,
+                                                          const int32_t *__restrict__ cell_level,
+                                                          const int2 *__restrict__ top_place,
+                                                          const int2 *__restrict__ sub_place, int *place,
+                                                          const int32_t *__restrict__ perm, int *__restrict__ sorted,
+                                                          int32_t *__restrict__ gorder, const DeviceState *st)
 {
-    __shared__ uint8_t s_tab[kHilbertTable];
-    hilbert_table_fill(s_tab);
-    __syncthreads();
+    __shared__ uint16_t s_cnt[kOrdCells], s_off[kOrdCells], s_par[kOrdCells];
+    __shared__ uint16_t s_boff[kSubtreeMax], s_bpar[kSubtreeMax];  // bodies: offset, cell
+    __shared__ OrderTables tab;
+    static_assert(kSubtreeMax <= 2048, "offsets of 11 bits");
     if (latched(st)) return;
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += blockDim.x * gridDim.x) {
-        uint64_t h = hilbert_top_lds(skeys[k] & ~(1ull << 63), kGroupLevels, s_tab);
-        if (sys_of) h |= (uint64_t)sys_of[perm[k]] << (3 * kGroupLevels);
-        gkey[k] = (K)h;
+    const int tid = threadIdx.x, n = g.n;
+    const int nsub = __hip_atomic_load(&st->nsub, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const int ntop = __hip_atomic_load(&st->ntop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    order_tables_fill(tab);
+    __syncthreads();
+    // a place under a top cell or root: the offsets from there up
+    auto up = [&](int2 e) {
+        int p = e.x;
+        while (e.y >= 0) {
+            e = top_place[e.y];
+            p += e.x;
+        }
+        return p;
+    };
+    for (int job = blockIdx.x; job < nsub; job += gridDim.x) {
+        const int4 sc = subcells[job], jb = sub[job];
+        const int base = sc.x, ks = sc.y, L0 = sc.z, a = jb.x, cnt = jb.y - jb.x;
+        const bool lds = ks <= kOrdCells;
+        const int2 pl = sub_place[job];
+        if (lds)
+            for (int k = tid; k < ks; k += 256) s_cnt[k] = (uint16_t)count[base + k];
+        const int state0 = order_state(tab, skeys[a], 0, 0, L0);
+        const int p0 = up(pl);
+        __syncthreads();
+        for (int k = tid; k < ks; k += 256) {
+            const int c = base + k, first = start[c];
+            const int4 *row = reinterpret_cast<const int4 *>(child + 8 * (int64_t)c);
+            const int4 ra = row[0], rb = row[1];
+            const int state = order_state(tab, skeys[first], state0, L0, cell_level[c]);
+            const int v[8] = {ra.x, ra.y, ra.z, ra.w, rb.x, rb.y, rb.z, rb.w};
+            int w[8], dg[8];
+            const uint32_t dig = tab.dig[state];
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                w[s] = v[s] == -1 ? 0 : v[s] < n ? 1 : lds ? (int)s_cnt[v[s] - base] : count[v[s]];
+                dg[s] = (int)(dig >> (4 * s)) & 7;
+            }
+            int cur = first - a;
+#pragma unroll
+            for (int s = 0; s < 8; ++s) {
+                int off = 0;
+#pragma unroll
+                for (int o = 0; o < 8; ++o) off += dg[o] < dg[s] ? w[o] : 0;
+                if (v[s] != -1) {
+                    if (v[s] < n) {
+                        s_boff[cur] = (uint16_t)off;
+                        s_bpar[cur] = (uint16_t)k;
+                    } else if (lds) {
+                        s_off[v[s] - base] = (uint16_t)off;
+                        s_par[v[s] - base] = (uint16_t)k;
+                    } else {
+                        place[v[s]] = off | k << 11;
+                    }
+                }
+                cur += w[s];
+            }
+        }
+        __syncthreads();
+        for (int i = tid; i < cnt; i += 256) {
+            int p = p0 + s_boff[i];
+            for (int c = s_bpar[i]; c != 0;) {  // the subtree's root is its first cell
+                if (lds) {
+                    p += s_off[c];
+                    c = s_par[c];
+                } else {
+                    const int e = place[base + c];
+                    p += e & 2047;
+                    c = e >> 11;
+                }
+            }
+            gorder[p] = a + i;
+        }
+        __syncthreads();
     }
+    // bodies that hang from a top cell or a root themselves: eight lanes per cell
+    const int d = tid & 7;
+    for (int i = (int)(blockIdx.x * 256 + tid) >> 3; i < ntop + g.nseg; i += (int)(gridDim.x * 256) >> 3) {
+        const bool top = i < ntop;
+        const int c = top ? base0 + i : seg_root(g, i - ntop);
+        const int v = child[8 * (int64_t)c + d];
+        if (((__ballot(v >= 0 && v < n) >> (tid & 56)) & 0xff) == 0) continue;  // of the cell's lanes
+        const int a = top ? start[c] : seg_lo(g, i - ntop);
+        const int w = v == -1 ? 0 : v < n ? 1 : count[v];
+        const uint32_t dig = tab.dig[top ? order_state(tab, skeys[a], 0, 0, cell_level[c]) : 0];
+        int before = 0, below = 0;
+        for (int s = 0; s < 8; ++s) {
+            const int ws = __shfl(w, s, 8);
+            before += s < d ? ws : 0;
+            below += ((int)(dig >> (4 * s)) & 7) < ((int)(dig >> (4 * d)) & 7) ? ws : 0;
+        }
+        if (v >= 0 && v < n) gorder[up(top ? make_int2(below, i) : make_int2(a + below, -1))] = a + before;
+    }
+    for (int k = blockIdx.x * 256 + tid; k < n; k += gridDim.x * 256) sorted[k] = perm[k];
 }
 
 // ------------------------------------------------------------------ launchers
-// Radix passes of the group-order keys (Hilbert digits, then the system index).
-static int group_passes(int sys_bits) { return (3 * kGroupLevels + sys_bits + kRadixBits - 1) / kRadixBits; }
-
 static inline int capped_grid(int64_t work, int cap = 65536)
 {
     int64_t g = (work + 255) / 256;
@@ -1237,7 +1383,7 @@ static void build_tree(Segs g, int nsamples, int base0, int m, TreeScratch &ts, 
     const int wire = nsamples * kLevels + g.nseg;  // entries, 8 lanes each
     top_wire_kernel<<<(8 * wire + 255) / 256, 256, 0, s>>>(g, nsamples, skeys, perm, child, cell_level, ts.top_flag,
                                                         ts.top_id, ts.top_a, ts.top_b, ts.sub, ts.sub_max,
-                                                        base0, m, index, start, st);
+                                                        base0, m, index, start, ts.top_place, ts.sub_place, st);
     subtree_cells_kernel<<<capped_grid(64 * (int64_t)ts.sub_max, 4096), 256, 0, s>>>(ts.sub, ts.sub_max, ts.lcp,
                                                                                      ts.cbase, st);
     subtree_base_kernel<<<1, 1024, 0, s>>>(ts.cbase, ts.sub_max, base0, m, index, st);
@@ -1277,6 +1423,8 @@ bool alloc_tree_scratch(TreeScratch &ts, int n, int nseg, int samples)
            hipMalloc((void **)&ts.top_id, 4 * tt) == hipSuccess &&
            hipMalloc((void **)&ts.top_a, 4 * tt) == hipSuccess &&
            hipMalloc((void **)&ts.top_b, 4 * tt) == hipSuccess &&
+           hipMalloc((void **)&ts.top_place, sizeof(int2) * tt) == hipSuccess &&
+           hipMalloc((void **)&ts.sub_place, sizeof(int2) * (size_t)ts.sub_max) == hipSuccess &&
            hipMalloc((void **)&ts.sub, sizeof(int4) * (size_t)ts.sub_max) == hipSuccess &&
            hipMalloc((void **)&ts.subcells, sizeof(int4) * (size_t)ts.sub_max) == hipSuccess &&
            hipMalloc((void **)&ts.cbase, sizeof(uint32_t) * ((size_t)ts.sub_max + 1)) == hipSuccess &&
@@ -1286,7 +1434,7 @@ bool alloc_tree_scratch(TreeScratch &ts, int n, int nseg, int samples)
 void free_tree_scratch(TreeScratch &ts)
 {
     void *p[] = {ts.lcp, ts.top_flag, ts.top_id, ts.top_a, ts.top_b, ts.sub, ts.subcells, ts.scan_tmp,
-                 ts.cbase};
+                 ts.cbase, ts.top_place, ts.sub_place};
     for (void *q : p)
         if (q) hipFree(q);
     ts = TreeScratch{};
@@ -1309,15 +1457,22 @@ void launch_summarize(nbx_context *c, hipStream_t s)
     summarise_tree(g, c->n, samples_of(c->n), c->ts, c->st, s, o);
 }
 
+// sorted[] and gorder[] (place: scratch of one int per node, free until the frame layout).
+static void order_bodies(Segs g, int base0, const TreeScratch &ts, DeviceState *st, hipStream_t s,
+                         const uint64_t *skeys, const int *child, const int *count, const int *start,
+                         const int32_t *cell_level, int *place, const int32_t *perm, int *sorted, int32_t *gorder)
+{
+    group_order_kernel<<<job_grid(g.n), 256, 0, s>>>(g, base0, skeys, ts.sub, ts.subcells, child, count, start,
+                                                     cell_level, ts.top_place, ts.sub_place, place, perm, sorted, gorder,
+                                                     st);
+}
+
 void launch_layout(nbx_context *c, hipStream_t s, int *sorted)
 {
-    const int n = c->n;
-    sorted_index_kernel<<<capped_grid(n), 256, 0, s>>>(n, c->perm, sorted, c->st);
+    Segs g{nullptr, nullptr, 1, c->n, 0};
+    order_bodies(g, c->n, c->ts, c->st, s, c->skeys, c->child, c->count, c->start, c->cell_level, c->pblk, c->perm,
+                 sorted, c->gorder);
     launch_frame_layout(c, s);
-    static_assert(3 * kGroupLevels <= 32, "single-system group keys are 32-bit");
-    group_keys_kernel<uint32_t><<<capped_grid(n), 256, 0, s>>>(n, c->skeys, c->perm, nullptr, c->gkey, c->st);
-    launch_radix_passes(c->hist, s, c->gkey, nullptr, n, 0, group_passes(0), c->gkey2, c->gorder,
-                        reinterpret_cast<uint32_t *>(c->kbuf), c->vbuf, nullptr);
 }
 
 void launch_frame_layout(nbx_context *c, hipStream_t s)
@@ -1351,19 +1506,16 @@ void launch_batch_summarize(nbx_batch *b, hipStream_t s)
 
 void launch_batch_layout(nbx_batch *b, hipStream_t s)
 {
-    sorted_index_kernel<<<capped_grid(b->N), 256, 0, s>>>(b->N, b->perm, b->sorted, b->st);
-    group_keys_kernel<uint64_t><<<capped_grid(b->N), 256, 0, s>>>(b->N, b->skeys, b->perm, b->sys_of, b->gkey, b->st);
-    SysInfo si{b->gkey, b->theta, b->ext};
+    Segs g{b->off, b->samp_off, b->S, b->N, 1};
+    order_bodies(g, b->N + b->S, b->ts, b->st, s, b->skeys, b->child, b->count, b->start, b->cell_level, b->pblk,
+                 b->perm, b->sorted, b->gorder);
+    SysInfo si{b->sys_of, b->theta, b->ext};
     const int runs = (int)(((int64_t)b->m - b->N + kOffRun - 1) / kOffRun);
     frame_count_kernel<true><<<runs, 256, 0, s>>>(b->N, b->index, b->child, b->boff, b->bsum, b->st);
     launch_scan_one_block(b->bsum, runs, s);
     frame_layout_kernel<true><<<capped_grid(8 * (int64_t)(b->m - b->N)), 256, 0, s>>>(
         b->N, b->S, b->index, b->child, b->pos, b->cell_level, b->count, b->start, b->nodes4, b->fnode, b->fmeta, b->boff,
         b->bsum, b->froot4, b->frootm, b->pblk, b->bpar, 0.f, layout_eps2(b->p), si, b->st);
-    int sys_bits = 0;
-    while ((1 << sys_bits) < b->S) ++sys_bits;
-    launch_radix_passes(b->hist, s, b->gkey, nullptr, b->N, 0, group_passes(sys_bits), b->gkey2, b->gorder, b->kbuf,
-                        b->vbuf, nullptr);
 }
 
 }  // namespace nbx

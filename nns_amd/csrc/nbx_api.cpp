@@ -148,12 +148,10 @@ int nbx_create(const nbx_params *p, int n_max, int m_max, int device, nbx_contex
     }
     const size_t n = (size_t)n_max, m = (size_t)m_max;
     c->bbox_blocks = 1024;
-    c->hist_tiles = (n_max + nbx::kSortTile - 1) / nbx::kSortTile;
     bool ok = dalloc(&c->st, 1) == hipSuccess && dalloc(&c->bbox_part, 6 * (size_t)c->bbox_blocks) == hipSuccess &&
               dalloc(&c->keys, n) == hipSuccess && dalloc(&c->skeys, n) == hipSuccess &&
               dalloc(&c->kbuf, n) == hipSuccess && dalloc(&c->perm, n) == hipSuccess &&
               dalloc(&c->vbuf, n) == hipSuccess && dalloc(&c->pos, n) == hipSuccess &&
-              dalloc(&c->hist, (size_t)c->hist_tiles * nbx::kRadix + nbx::kRadix) == hipSuccess &&
               dalloc(&c->cell_level, m) == hipSuccess && dalloc(&c->sum64, m) == hipSuccess &&
               dalloc(&c->nodes4, m) == hipSuccess &&
               dalloc(&c->fnode, m + 8) == hipSuccess && dalloc(&c->fmeta, m + 8) == hipSuccess &&
@@ -163,7 +161,6 @@ int nbx_create(const nbx_params *p, int n_max, int m_max, int device, nbx_contex
               dalloc(&c->acc_scratch, 3 * n) == hipSuccess && dalloc(&c->bodies4, n) == hipSuccess &&
               dalloc(&c->star_part, (size_t)nbx::kStarPartBlocks * NBX_MAX_STARS * 3) == hipSuccess &&
               dalloc(&c->walk, 2 * ((n + 63) / 64)) == hipSuccess && dalloc(&c->gcost, (n + 63) / 64) == hipSuccess &&
-              dalloc(&c->gkey, n) == hipSuccess && dalloc(&c->gkey2, n) == hipSuccess &&
               dalloc(&c->gorder, n) == hipSuccess &&
               hipEventCreate(&c->ev0) == hipSuccess && hipEventCreate(&c->ev1) == hipSuccess;
     for (int k = 0; ok && k < 8; ++k) ok = hipEventCreate(&c->stage_ev[k]) == hipSuccess;
@@ -184,10 +181,9 @@ int nbx_destroy(nbx_context *c)
     if (!c) return NBX_OK;
     hipSetDevice(c->device);
     hipDeviceSynchronize();
-    void *bufs[] = {c->st, c->bbox_part, c->keys, c->skeys, c->kbuf, c->perm, c->vbuf, c->pos, c->hist,
+    void *bufs[] = {c->st, c->bbox_part, c->keys, c->skeys, c->kbuf, c->perm, c->vbuf, c->pos,
                     c->cell_level, c->sum64, c->nodes4, c->fnode, c->fmeta, c->boff, c->bsum, c->froot4, c->frootm, c->pblk, c->bpar, c->counts,
-                    c->acc_scratch, c->star_part, c->walk, c->gcost, c->bodies4, c->gkey, c->gkey2,
-                    c->gorder};
+                    c->acc_scratch, c->star_part, c->walk, c->gcost, c->bodies4, c->gorder};
     for (void *b : bufs)
         if (b) hipFree(b);
     nbx::free_tree_scratch(c->ts);
@@ -307,8 +303,8 @@ int nbx_build_tree(nbx_context *c, float *x, float *y, float *z, float *mass, in
     c->child = child; c->count = count; c->start = start; c->index = index;
     c->n = n; c->m = m;
     StageTimer t(c, s, elapsed_ms);
-    nbx::launch_keys(c, s, x, y, z, mass, n, NBX_KEY_MORTON, c->keys);
-    nbx::launch_radix_sort(c, s, c->keys, n, c->skeys, c->perm, c->kbuf, c->vbuf, c->pos, nbx::kMortonSortBits);
+    nbx::launch_sort_bodies(nbx::one_segment(n), x, y, z, mass, c->st->ext, c->keys, c->bodies4, c->skeys, c->perm,
+                            c->kbuf, c->vbuf, c->pos, s);
     nbx::launch_build(c, s, n, m, child, index);
     c->stage = 2;
     return t.finish();
@@ -409,7 +405,7 @@ int nbx_compute_keys(nbx_context *c, const float *x, const float *y, const float
     hipSetDevice(c->device);
     hipStream_t s = (hipStream_t)stream;
     StageTimer t(c, s, elapsed_ms);
-    nbx::launch_keys(c, s, x, y, z, nullptr, n, key_type, keys);
+    nbx::launch_keys(c, s, x, y, z, n, key_type, keys);
     return t.finish();
 }
 
@@ -423,7 +419,7 @@ int nbx_sort_keys(nbx_context *c, const uint64_t *keys, int n, uint64_t *sorted_
     hipSetDevice(c->device);
     hipStream_t s = (hipStream_t)stream;
     StageTimer t(c, s, elapsed_ms);
-    nbx::launch_radix_sort(c, s, keys, n, sorted_keys, perm, c->kbuf, c->vbuf, nullptr, 64);
+    nbx::launch_sort_keys(nbx::one_segment(n), keys, sorted_keys, perm, c->kbuf, c->vbuf, nullptr, s);
     return t.finish();
 }
 

@@ -46,7 +46,6 @@ void enqueue_step(nbx_batch *b, hipStream_t s, hipEvent_t *ev)
     mark(1);
     nbx::launch_batch_bbox(b, s);
     mark(2);
-    nbx::launch_batch_keys(b, s);
     nbx::launch_batch_sort(b, s);
     nbx::launch_batch_build(b, s);
     mark(3);
@@ -108,13 +107,15 @@ int nbx_batch_create(const nbx_params *p, int nsys, const int *sys_n, const floa
     b->force_waves = p->force_waves == 2 || p->force_waves == 8 ? p->force_waves : 4;
     std::vector<int32_t> off(nsys + 1, 0), sys_of(total), samp(nsys + 1, 0);
     std::vector<float> th(nsys, p->theta);
-    std::vector<int4> groups, chunks;
+    std::vector<int4> groups, chunks, sorts;
     std::vector<int32_t> choff(nsys + 1, 0);
     for (int s = 0; s < nsys; ++s) {
         off[s + 1] = off[s] + sys_n[s];
         for (int f = off[s]; f < off[s + 1]; f += nbx::kBboxChunk)
             chunks.push_back(make_int4(s, f, std::min(f + nbx::kBboxChunk, off[s + 1]), 0));
         choff[s + 1] = (int32_t)chunks.size();
+        for (int j = 0; j * nbx::kSortChunk < sys_n[s]; ++j) sorts.push_back(make_int4(off[s], off[s + 1], j, s));
+        b->longest = std::max(b->longest, sys_n[s]);
         for (int i = off[s]; i < off[s + 1]; ++i) sys_of[i] = s;
         if (sys_theta) th[s] = sys_theta[s];
         for (int g = 0; g < sys_n[s]; g += 64) groups.push_back(make_int4(off[s] + g, std::min(64, sys_n[s] - g), s, 0));
@@ -122,13 +123,12 @@ int nbx_batch_create(const nbx_params *p, int nsys, const int *sys_n, const floa
     }
     b->ngroups = (int)groups.size();
     b->nchunk = (int)chunks.size();
+    b->nsort = (int)sorts.size();
     const size_t N = total, M = m64, S = nsys;
-    const size_t tiles = (N + nbx::kSortTile - 1) / nbx::kSortTile;
     bool ok = dalloc(&b->st, 1) && dalloc(&b->off, S + 1) && dalloc(&b->sys_of, N) && dalloc(&b->theta, S) &&
               dalloc(&b->groups, groups.size()) && dalloc(&b->ext, 4 * S) && dalloc(&b->mm, 6 * S) &&
-              dalloc(&b->keys, N) && dalloc(&b->skeys, N) && dalloc(&b->kbuf, N) && dalloc(&b->k2, N) &&
-              dalloc(&b->k2buf, N) && dalloc(&b->perm, N) && dalloc(&b->perm1, N) && dalloc(&b->vbuf, N) &&
-              dalloc(&b->pos, N) && dalloc(&b->sorted, N) && dalloc(&b->hist, tiles * nbx::kRadix + nbx::kRadix) &&
+              dalloc(&b->keys, N) && dalloc(&b->skeys, N) && dalloc(&b->kbuf, N) && dalloc(&b->perm, N) && dalloc(&b->vbuf, N) &&
+              dalloc(&b->pos, N) && dalloc(&b->sorted, N) && dalloc(&b->sort_chunks, sorts.size()) &&
               dalloc(&b->child, 8 * M) && dalloc(&b->index, 1) && dalloc(&b->count, M) && dalloc(&b->start, M) &&
               dalloc(&b->cell_level, M) &&
               dalloc(&b->sum64, M) && dalloc(&b->nodes4, M) &&
@@ -136,7 +136,7 @@ int nbx_batch_create(const nbx_params *p, int nsys, const int *sys_n, const floa
               dalloc(&b->bsum, M / nbx::kOffRun + 2) && dalloc(&b->froot4, S) &&
               dalloc(&b->frootm, S) && dalloc(&b->pblk, M) && dalloc(&b->bpar, N) && dalloc(&b->counts, N) && dalloc(&b->acc_scratch, 3 * N) && dalloc(&b->bodies4, N) &&
               dalloc(&b->walk, 2 * groups.size()) && dalloc(&b->gcost, groups.size()) &&
-              dalloc(&b->gkey, N) && dalloc(&b->gkey2, N) && dalloc(&b->gorder, N) &&
+              dalloc(&b->gorder, N) &&
               dalloc(&b->samp_off, S + 1) && dalloc(&b->bchunk, chunks.size()) && dalloc(&b->bchunk_off, S + 1) &&
               dalloc(&b->bpart, 6 * chunks.size()) && nbx::alloc_tree_scratch(b->ts, (int)N, nsys, samp[nsys]);
     for (int k = 0; ok && k < 8; ++k) ok = hipEventCreate(&b->stage_ev[k]) == hipSuccess;
@@ -148,6 +148,7 @@ int nbx_batch_create(const nbx_params *p, int nsys, const int *sys_n, const floa
          hipMemcpy(b->groups, groups.data(), sizeof(int4) * groups.size(), hipMemcpyHostToDevice) == hipSuccess &&
          hipMemcpy(b->samp_off, samp.data(), 4 * (S + 1), hipMemcpyHostToDevice) == hipSuccess &&
          hipMemcpy(b->bchunk, chunks.data(), sizeof(int4) * chunks.size(), hipMemcpyHostToDevice) == hipSuccess &&
+         hipMemcpy(b->sort_chunks, sorts.data(), sizeof(int4) * sorts.size(), hipMemcpyHostToDevice) == hipSuccess &&
          hipMemcpy(b->bchunk_off, choff.data(), 4 * (S + 1), hipMemcpyHostToDevice) == hipSuccess &&
          hipDeviceSynchronize() == hipSuccess;
     if (!ok) {
@@ -165,9 +166,9 @@ int nbx_batch_destroy(nbx_batch *b)
     hipDeviceSynchronize();
     drop_graph(b);
     void *bufs[] = {b->st, b->off, b->sys_of, b->theta, b->groups, b->ext, b->mm, b->keys, b->skeys, b->kbuf,
-                    b->k2, b->k2buf, b->perm, b->perm1, b->vbuf, b->pos, b->sorted, b->hist, b->child, b->index,
+                    b->perm, b->vbuf, b->pos, b->sorted, b->sort_chunks, b->child, b->index,
                     b->count, b->start, b->cell_level, b->sum64, b->nodes4,
-                    b->fnode, b->fmeta, b->boff, b->bsum, b->froot4, b->frootm, b->pblk, b->bpar, b->counts, b->acc_scratch, b->samp_off, b->bodies4, b->gkey, b->gkey2, b->gorder, b->walk, b->gcost,
+                    b->fnode, b->fmeta, b->boff, b->bsum, b->froot4, b->frootm, b->pblk, b->bpar, b->counts, b->acc_scratch, b->samp_off, b->bodies4, b->gorder, b->walk, b->gcost,
                     b->bchunk, b->bchunk_off, b->bpart};
     for (void *q : bufs)
         if (q) hipFree(q);
@@ -301,7 +302,6 @@ int nbx_batch_autotune(nbx_batch *b, void *stream, int *waves_out)
     // tree of the current state, without the update
     nbx::launch_batch_reset(b, s);
     nbx::launch_batch_bbox(b, s);
-    nbx::launch_batch_keys(b, s);
     nbx::launch_batch_sort(b, s);
     nbx::launch_batch_build(b, s);
     nbx::launch_batch_summarize(b, s);

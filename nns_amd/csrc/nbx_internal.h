@@ -13,9 +13,7 @@ namespace nbx {
 constexpr int kKeyLevels = 21;
 constexpr double kMaskCoord = 2097151.0;
 
-// Radix sort: 8-bit digits, 256 threads x 8 items per tile.  (9-bit digits would
-// save a pass on a 63-bit Morton key, but their 512-way scatter is slower: 10
-// passes of 9 bits took longer than 12 of 8 at N = 4M.)
+// Radix sort of 32-bit keys: 8-bit digits, 256 threads x 8 items per tile.
 constexpr int kRadixBits = 8;
 constexpr int kRadix = 1 << kRadixBits;
 constexpr int kSortThreads = 256;
@@ -97,6 +95,8 @@ struct TreeScratch {
     uint8_t *lcp = nullptr;      // [n-1] common key digits of sorted neighbours
     uint32_t *top_flag = nullptr, *top_id = nullptr;  // [samples * kLevels]
     int32_t *top_a = nullptr, *top_b = nullptr;       // [samples * kLevels] body range of a top cell
+    int2 *top_place = nullptr;   // [samples * kLevels] place of each top cell in the group order, by its number
+    int2 *sub_place = nullptr;   // [sub_max] and of each subtree: {offset in the parent, parent's number or -1}
     int4 *sub = nullptr;         // {first, end, level, slot address}
     int4 *subcells = nullptr;    // {first cell id, cells, level, deepest level} of each subtree
     uint32_t *cbase = nullptr;   // [sub_max + 1] cells of each subtree, then their exclusive sum
@@ -131,8 +131,6 @@ struct nbx_context {
     int bbox_blocks = 0;
     uint64_t *keys = nullptr, *skeys = nullptr, *kbuf = nullptr;
     int32_t *perm = nullptr, *vbuf = nullptr, *pos = nullptr;
-    uint32_t *hist = nullptr;
-    int hist_tiles = 0;
     int32_t *cell_level = nullptr;
     double4 *sum64 = nullptr;    // [m_max] FP64 sums of each cell: mass, mass moments x, y, z
     float4 *nodes4 = nullptr;
@@ -167,7 +165,6 @@ struct nbx_context {
     float *acc_scratch = nullptr;
     double *star_part = nullptr;  // star forces: per-block partial pulls, kStarBlocks x NBX_MAX_STARS x 3
     float4 *bodies4 = nullptr;  // (x, y, z, m) of every body in input order
-    uint32_t *gkey = nullptr, *gkey2 = nullptr;  // group-order sort keys
     int32_t *gorder = nullptr;  // [n] sorted position of the j-th body of the force groups
     nbx::TreeScratch ts;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
@@ -211,9 +208,11 @@ struct nbx_batch {
     int4 *bchunk = nullptr;         // [nchunk] {system, first body, end, 0}
     int32_t *bchunk_off = nullptr;  // [S+1] first chunk of each system
     float *bpart = nullptr;         // [6 nchunk] partial extremes
-    uint64_t *keys = nullptr, *skeys = nullptr, *kbuf = nullptr, *k2 = nullptr, *k2buf = nullptr;
-    int32_t *perm = nullptr, *perm1 = nullptr, *vbuf = nullptr, *pos = nullptr, *sorted = nullptr;
-    uint32_t *hist = nullptr;
+    int nsort = 0;                  // sort chunks, and bodies of the largest system
+    int longest = 0;
+    int4 *sort_chunks = nullptr;    // [nsort] {first body and end of the system, chunk in it, system}
+    uint64_t *keys = nullptr, *skeys = nullptr, *kbuf = nullptr;
+    int32_t *perm = nullptr, *vbuf = nullptr, *pos = nullptr, *sorted = nullptr;
     int *child = nullptr, *index = nullptr, *count = nullptr, *start = nullptr;
     int32_t *cell_level = nullptr;
     double4 *sum64 = nullptr;    // [M] FP64 sums of each cell: mass, mass moments x, y, z
@@ -228,7 +227,6 @@ struct nbx_batch {
     int64_t *counts = nullptr;
     float *acc_scratch = nullptr;
     float4 *bodies4 = nullptr;
-    uint64_t *gkey = nullptr, *gkey2 = nullptr;
     int32_t *gorder = nullptr;
     int32_t *samp_off = nullptr;  // [S+1] first top-table sample of each system
     nbx::TreeScratch ts;
@@ -249,9 +247,8 @@ void launch_reset(nbx_context *c, hipStream_t s, int *mutex, float *x, float *y,
                   float *minY, float *maxY, float *minZ, float *maxZ, int n, int m);
 void launch_bbox(nbx_context *c, hipStream_t s, const float *x, const float *y, const float *z,
                  float *minX, float *maxX, float *minY, float *maxY, float *minZ, float *maxZ, int n);
-// Also packs (x, y, z, mass) into c->bodies4 when mass is given.
-void launch_keys(nbx_context *c, hipStream_t s, const float *x, const float *y, const float *z, const float *mass,
-                 int n, int key_type, uint64_t *keys);
+void launch_keys(nbx_context *c, hipStream_t s, const float *x, const float *y, const float *z, int n, int key_type,
+                 uint64_t *keys);
 // Does nothing once the error latch of st is raised (st may be null: always runs).
 void launch_update(hipStream_t s, int block, const DeviceState *st, float *x, float *y, float *z, float *vx, float *vy,
                    float *vz, const float *ax, const float *ay, const float *az, int n, float dt, float d);
@@ -262,25 +259,38 @@ void launch_star_forces(nbx_context *c, hipStream_t s, const float *sx, const fl
                         const float *sm, float *sax, float *say, float *saz, int ns, const float *x, const float *y,
                         const float *z, const float *mass, float *ax, float *ay, float *az, int n, float g);
 
+// launchers (k_sort.hip)
+constexpr int kSortChunk = 4096;  // pairs sorted in LDS by one workgroup
+// Segments of a sort: one of n pairs (chunks null), or a table of chunks {segment
+// first, end, index of the chunk within it, system}.
+struct SortSegs {
+    const int4 *chunks;
+    int nchunks, n;
+    int longest;  // pairs of the longest segment
+};
+inline SortSegs one_segment(int n) { return SortSegs{nullptr, (n + kSortChunk - 1) / kSortChunk, n, n}; }
+// Stable ascending sort of the pairs (key, index) of every segment: keys_in (not
+// modified) into keys_out / perm_out, the inverse permutation to inv_out when not
+// null.  tmp_k / tmp_v: scratch of n elements.
+void launch_sort_keys(const SortSegs &g, const uint64_t *keys_in, uint64_t *keys_out, int32_t *perm_out,
+                      uint64_t *tmp_k, int32_t *tmp_v, int32_t *inv_out, hipStream_t s);
+// The same over the Morton keys of the bodies, made on the way (ext: 4 doubles per
+// system) and written to keys in input order, with (x, y, z, mass) to bodies4.
+void launch_sort_bodies(const SortSegs &g, const float *x, const float *y, const float *z, const float *mass,
+                        const double *ext, uint64_t *keys, float4 *bodies4, uint64_t *keys_out, int32_t *perm_out,
+                        uint64_t *tmp_k, int32_t *tmp_v, int32_t *inv_out, hipStream_t s);
+
 // launchers (k_radix.hip)
-// Sorts keys_in (not modified) by their low key_bits bits into keys_out / perm_out (stable);
-// writes the inverse permutation to inv_out when not null.  tmp_k / tmp_v: scratch of n
-// elements.  Morton keys need 63 bits (bit 63 is set in every key).
-void launch_radix_sort(nbx_context *c, hipStream_t s, const uint64_t *keys_in, int n, uint64_t *keys_out,
-                       int32_t *perm_out, uint64_t *tmp_k, int32_t *tmp_v, int32_t *inv_out, int key_bits);
-constexpr int kMortonSortBits = 63;
 // exclusive scan of total <= 2^20 values; sums: scratch of 1024 values
 void launch_exclusive_scan_u32(uint32_t *data, int total, uint32_t *sums, hipStream_t s);
 // The same in one launch of one workgroup (short arrays).
 void launch_scan_one_block(uint32_t *data, int total, hipStream_t s);
-// npasses passes of kRadixBits bits from bit first_shift; vals_in == nullptr means 0, 1, 2, ...
-// n_dev (nullable): device-side count; only the first min(n, *n_dev) keys are sorted
-// (grids are sized for n).  tmp_k may alias keys_in when npasses is odd.  K: uint64_t
-// or uint32_t.
-template <class K>
-void launch_radix_passes(uint32_t *hist, hipStream_t s, const K *keys_in, const int32_t *vals_in, int n,
-                         int first_shift, int npasses, K *keys_out, int32_t *vals_out, K *tmp_k,
-                         int32_t *tmp_v, int32_t *inv_out, const int *n_dev = nullptr);
+// Stable radix sort of the 32-bit keys and their indices: npasses passes of
+// kRadixBits bits from bit 0, into keys_out / vals_out.  n_dev: device-side count;
+// only the first min(n, *n_dev) keys are sorted (grids are sized for n).  tmp_k may
+// alias keys_in when npasses is odd.
+void launch_radix_passes(uint32_t *hist, hipStream_t s, const uint32_t *keys_in, int n, int npasses, uint32_t *keys_out,
+                         int32_t *vals_out, uint32_t *tmp_k, int32_t *tmp_v, const int *n_dev);
 
 // launchers (k_tree.hip)
 void launch_build(nbx_context *c, hipStream_t s, int n, int m, int *child, int *index);
@@ -305,10 +315,9 @@ void launch_force(nbx_context *c, hipStream_t s, float *ax, float *ay, float *az
                   int64_t *walk = nullptr);
 void launch_force_waves(nbx_context *c, hipStream_t s, float *ax, float *ay, float *az, float g, int waves);
 
-// batched form (k_basic.hip, k_radix.hip, k_tree.hip, k_force.hip)
+// batched form (k_basic.hip, k_sort.hip, k_tree.hip, k_force.hip)
 void launch_batch_reset(nbx_batch *b, hipStream_t s);
 void launch_batch_bbox(nbx_batch *b, hipStream_t s);
-void launch_batch_keys(nbx_batch *b, hipStream_t s);
 void launch_batch_sort(nbx_batch *b, hipStream_t s);
 void launch_batch_build(nbx_batch *b, hipStream_t s);
 void launch_batch_summarize(nbx_batch *b, hipStream_t s);

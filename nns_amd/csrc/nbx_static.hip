@@ -1,9 +1,9 @@
 // nbx_static.hip -- nbx_sort_keys_static: the stable key sort of nbx_sort_keys
 // for callers that cannot allocate device memory (code under HIP graph capture,
 // serving loops): no context, no hipMalloc, no hipFree.  Its scratch -- the
-// ping-pong keys and values of the radix passes and the digit histograms -- is
-// one file-scope device array, `scratch`, of kStaticSortMax keys' worth
-// (12.5 MiB), which every GPU the library runs on holds until the process ends.
+// second keys and values of the merge passes -- is one file-scope device array,
+// `scratch`, of kStaticSortMax keys' worth (12 MiB), which every GPU the library runs
+// on holds until the process ends.
 //
 // Host code never passes `scratch` itself to a kernel: on the host the name is
 // a stand-in, not a device address.  The first call on a device, with that
@@ -13,8 +13,8 @@
 //
 // All calls on one GPU share that GPU's array, whose contents are those of the
 // last call: calls that overlap on one GPU (two streams, two host threads) race.
-// Nothing in the array needs to start at zero: each radix pass writes every
-// histogram entry it later reads.
+// Nothing in the array needs to start at zero: a pass reads only what the pass
+// before it wrote.
 #include <mutex>
 
 #include "nbx_internal.h"
@@ -24,9 +24,7 @@ namespace {
 constexpr int kStaticSortMax = 1 << 20;  // keys per call
 constexpr size_t kTmpKeyBytes = sizeof(uint64_t) * (size_t)kStaticSortMax;
 constexpr size_t kTmpValBytes = sizeof(int32_t) * (size_t)kStaticSortMax;
-constexpr size_t kHistBytes =
-    sizeof(uint32_t) * ((size_t)(kStaticSortMax / nbx::kSortTile) * nbx::kRadix + nbx::kRadix);
-constexpr size_t kScratchBytes = kTmpKeyBytes + kTmpValBytes + kHistBytes;
+constexpr size_t kScratchBytes = kTmpKeyBytes + kTmpValBytes;
 static_assert(kTmpKeyBytes % 256 == 0 && kTmpValBytes % 256 == 0, "sub-buffers stay 256-byte aligned");
 
 constexpr int kMaxDevices = 64;
@@ -80,10 +78,8 @@ extern "C" int nbx_sort_keys_static(const uint64_t *keys, int n, uint64_t *sorte
     }
     uint64_t *tmp_k = reinterpret_cast<uint64_t *>(base);
     int32_t *tmp_v = reinterpret_cast<int32_t *>(base + kTmpKeyBytes);
-    uint32_t *hist = reinterpret_cast<uint32_t *>(base + kTmpKeyBytes + kTmpValBytes);
-    // 8 passes of 8 bits: the same launches as nbx_sort_keys over 64-bit keys
-    nbx::launch_radix_passes<uint64_t>(hist, (hipStream_t)stream, keys, nullptr, n, 0, 64 / nbx::kRadixBits,
-                                       sorted_keys, perm, tmp_k, tmp_v, nullptr);
+    // the same launches as nbx_sort_keys
+    nbx::launch_sort_keys(nbx::one_segment(n), keys, sorted_keys, perm, tmp_k, tmp_v, nullptr, (hipStream_t)stream);
     e = hipGetLastError();
     if (e != hipSuccess) {
         nbx::set_create_error(std::string("nbx_sort_keys_static: kernel launch: ") + hipGetErrorString(e));
