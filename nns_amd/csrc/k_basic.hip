@@ -200,7 +200,7 @@ __global__ void __launch_bounds__(1024) update_kernel(
 // The terms are evaluated in FP64.  Bodies: one thread each, the sum over the
 // stars added once to the FP32 acceleration the tree walk wrote.  Stars: each
 // block reduces its bodies' pulls per star (wave shuffles, then LDS) to one
-// partial per (block, star); star_final_kernel adds the partials in block
+// partial per (block, star); star_final_kernel adds the partials in a fixed
 // order and the star-star terms: no atomics, the same sums on every run.
 constexpr int kStarThreads = 256;
 
@@ -260,17 +260,28 @@ __global__ void __launch_bounds__(kStarThreads) star_bodies_kernel(
     }
 }
 
-__global__ void __launch_bounds__(64) star_final_kernel(
+// One workgroup per star: its threads add the block partials in strides, then meet by
+// shuffles and LDS (one thread adding them in turn took 27 us for 128 partials).
+__global__ void __launch_bounds__(kStarThreads) star_final_kernel(
     const float *__restrict__ sx, const float *__restrict__ sy, const float *__restrict__ sz,
     const float *__restrict__ sm, int ns, float *__restrict__ sax, float *__restrict__ say, float *__restrict__ saz,
     double G, double eps2, const double *__restrict__ part, int nblocks, const DeviceState *st)
 {
-    if (latched(st)) return;
-    const int s = threadIdx.x;
-    if (s >= ns) return;
+    __shared__ double red[kStarThreads / 64][3];
+    if (latched(st)) return;  // one value for the whole launch: nothing in it raises the latch
+    const int s = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    double b[3] = {0.0, 0.0, 0.0};
+    for (int k = tid; k < nblocks; k += kStarThreads)  // Interaction.cpp:120-123: the bodies
+        for (int c = 0; c < 3; ++c) b[c] += part[((int64_t)k * NBX_MAX_STARS + s) * 3 + c];
+    for (int c = 0; c < 3; ++c) {
+        b[c] = wave_sum_f64(b[c]);
+        if (lane == 0) red[wave][c] = b[c];
+    }
+    __syncthreads();
+    if (tid) return;
     const double qx = sx[s], qy = sy[s], qz = sz[s];
     double gx = 0.0, gy = 0.0, gz = 0.0;
-    for (int t = 0; t < ns; ++t) {  // Interaction.cpp:113-118: every other star
+    for (int t = 0; t < ns; ++t) {  // :113-118: every other star
         if (t == s) continue;
         const double dx = (double)sx[t] - qx, dy = (double)sy[t] - qy, dz = (double)sz[t] - qz;
         const double d2 = dx * dx + dy * dy + dz * dz;
@@ -279,9 +290,8 @@ __global__ void __launch_bounds__(64) star_final_kernel(
         const double w = (double)sm[t] / (r2 * sqrt(r2));
         gx += w * dx; gy += w * dy; gz += w * dz;
     }
-    for (int b = 0; b < nblocks; ++b) {  // :120-123: the bodies, block partials in order
-        const double *p = part + ((int64_t)b * NBX_MAX_STARS + s) * 3;
-        gx += p[0]; gy += p[1]; gz += p[2];
+    for (int w = 0; w < kStarThreads / 64; ++w) {
+        gx += red[w][0]; gy += red[w][1]; gz += red[w][2];
     }
     sax[s] = (float)(G * gx);
     say[s] = (float)(G * gy);
@@ -352,7 +362,7 @@ void launch_star_forces(nbx_context *c, hipStream_t s, const float *sx, const fl
     const int blocks = n > 0 ? grid_for(n, kStarThreads, kStarPartBlocks) : 1;
     star_bodies_kernel<<<blocks, kStarThreads, 0, s>>>(sx, sy, sz, sm, ns, x, y, z, mass, ax, ay, az, n, (double)g,
                                                        eps2, c->star_part, c->st);
-    star_final_kernel<<<1, 64, 0, s>>>(sx, sy, sz, sm, ns, sax, say, saz, (double)g, eps2, c->star_part, blocks,
+    star_final_kernel<<<ns, kStarThreads, 0, s>>>(sx, sy, sz, sm, ns, sax, say, saz, (double)g, eps2, c->star_part, blocks,
                                        c->st);
 }
 

@@ -11,7 +11,7 @@
 // own L2, so a fence or atomic at device scope costs a trip past L2; those are
 // kept to a handful per subtree:
 //   1. top cells -- cells holding more than kSubtreeMax bodies -- are found
-//      from the sorted keys by binary search (one thread per sample of
+//      from the sorted keys by searches (one thread per sample of
 //      kSubtreeMax bodies) and wired with their child ranges;
 //   2. every child range of a top cell with 2..kSubtreeMax bodies is a subtree
 //      built by ONE wave from the shared-digit counts of neighbouring keys:
@@ -56,79 +56,117 @@ __device__ inline int seg_of_sample(const Segs &g, int k)
 
 __device__ inline uint64_t prefix_of(uint64_t key, int L) { return key >> (63 - 3 * L); }
 
-// First index in [lo, hi) whose level-L prefix is >= P (keys sorted).
-__device__ inline int lower_prefix(const uint64_t *k, int lo, int hi, uint64_t P, int L)
+// One step of a search for the first index in [lo, hi) where a predicate that
+// holds up to it fails: three probes, a quarter of the range left.  Searches over
+// sorted keys are chains of dependent loads (an L2 round trip each), so halving the
+// steps is worth the two extra loads.
+struct Quarter {
+    int m[3];
+};
+__device__ inline Quarter quarter_probes(int lo, int hi)
 {
-    while (lo < hi) {
-        int mid = lo + ((hi - lo) >> 1);
-        if (prefix_of(k[mid], L) < P) lo = mid + 1; else hi = mid;
-    }
-    return lo;
+    const int len = hi - lo;
+    return Quarter{{lo + (len >> 2), lo + (len >> 1), lo + (int)((3 * (int64_t)len) >> 2)}};
 }
-__device__ inline int upper_prefix(const uint64_t *k, int lo, int hi, uint64_t P, int L)
+__device__ inline void quarter_step(int &lo, int &hi, const Quarter &q, bool p0, bool p1, bool p2)
 {
-    while (lo < hi) {
-        int mid = lo + ((hi - lo) >> 1);
-        if (prefix_of(k[mid], L) <= P) lo = mid + 1; else hi = mid;
+    const int l = p2 ? q.m[2] + 1 : p1 ? q.m[1] + 1 : p0 ? q.m[0] + 1 : lo;
+    hi = !p0 ? q.m[0] : !p1 ? q.m[1] : !p2 ? q.m[2] : hi;
+    lo = l;
+}
+// The run [a, b) of keys around position q of [lo, hi) that share its first L digits,
+// both ends searched at once.
+__device__ inline void prefix_run(const uint64_t *k, int lo, int q, int hi, int L, int &a, int &b)
+{
+    const uint64_t P = prefix_of(k[q], L);
+    int la = lo, ha = q, lb = q + 1, hb = hi;
+    while (la < ha || lb < hb) {
+        const bool ua = la < ha, ub = lb < hb;
+        const Quarter x = quarter_probes(la, ua ? ha : la), y = quarter_probes(ub ? lb : q, ub ? hb : q);
+        uint64_t kx[3], ky[3];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            kx[i] = k[x.m[i]];
+            ky[i] = k[y.m[i]];
+        }
+        if (ua) quarter_step(la, ha, x, prefix_of(kx[0], L) < P, prefix_of(kx[1], L) < P, prefix_of(kx[2], L) < P);
+        if (ub) quarter_step(lb, hb, y, prefix_of(ky[0], L) <= P, prefix_of(ky[1], L) <= P, prefix_of(ky[2], L) <= P);
     }
-    return lo;
+    a = la;
+    b = lb;
 }
 // First index in [lo, hi) whose digit L is >= d (all keys share the first L digits).
 __device__ inline int lower_digit(const uint64_t *k, int lo, int hi, int d, int L)
 {
     while (lo < hi) {
-        int mid = lo + ((hi - lo) >> 1);
-        if (digit_at(k[mid], L) < d) lo = mid + 1; else hi = mid;
+        const Quarter x = quarter_probes(lo, hi);
+        const uint64_t k0 = k[x.m[0]], k1 = k[x.m[1]], k2 = k[x.m[2]];
+        quarter_step(lo, hi, x, digit_at(k0, L) < d, digit_at(k1, L) < d, digit_at(k2, L) < d);
     }
     return lo;
 }
 
-// lcp[k] = number of leading key digits shared by sorted keys k and k+1 (21 if equal).
-__global__ void __launch_bounds__(256) lcp_kernel(int n, const uint64_t *__restrict__ skeys,
-                                                  uint8_t *__restrict__ lcp, DeviceState *st)
+// After the sort, in one launch: the top cells (the first `tb` workgroups), then lcp
+// and the key-ordered bodies.
+//
+// Top cells: one lane per (sample q, level L); q is every kSubtreeMax-th sorted
+// position of a segment.  The level-L cell through q is [a, b), found by a search
+// over the segment; it is a top cell when it holds more than kSubtreeMax bodies, and
+// q owns it when no earlier sample lies in it.  The levels of a sample are searched
+// side by side, not one after another.  The table is level-major (entry
+// L * nsamples + k), so the scan of its flags numbers the top cells level by level:
+// the cells of level L are the ids base0 + [id[L * nsamples], id[(L + 1) * nsamples]).
+//
+// lcp[k]: the number of leading key digits shared by sorted keys k and k+1 (21 if
+// equal).
+//
+// Bodies in key order as float4 (x, y, z, m) at nodes4[0..n), for the summary: read in
+// input order and stored at their sorted positions pos[] (the sort's inverse
+// permutation): random 16-byte reads each fetch a whole line, random 16-byte stores
+// only dirty their bytes.
+__global__ void __launch_bounds__(256) after_sort_kernel(Segs g, int nsamples, int tb,
+                                                         const uint64_t *__restrict__ skeys,
+                                                         uint32_t *__restrict__ flag, uint32_t *__restrict__ id,
+                                                         int32_t *__restrict__ ta, int32_t *__restrict__ tend,
+                                                         uint8_t *__restrict__ lcp, const int32_t *__restrict__ pos,
+                                                         const float4 *__restrict__ bodies4,
+                                                         float4 *__restrict__ nodes4, DeviceState *st)
 {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
+    const int tid = threadIdx.x;
+    if (blockIdx.x == 0 && tid == 0) {
         st->nsub = 0;
         st->ntop = 0;
     }
-    for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n - 1; k += blockDim.x * gridDim.x) {
-        const uint64_t x = (skeys[k] ^ skeys[k + 1]) & ~(1ull << 63);
-        lcp[k] = x == 0 ? (uint8_t)kKeyLevels : (uint8_t)((62 - (63 - __clzll((long long)x))) / 3);
-    }
-}
-
-// Top cells: one lane per (sample q, level L); q is every kSubtreeMax-th sorted
-// position of a segment.  The level-L cell through q is [a, b), found by two
-// binary searches over the segment; it is a top cell when it holds more than
-// kSubtreeMax bodies, and q owns it when no earlier sample lies in it.  The
-// levels of a sample are searched side by side, not one after another.  The
-// table is level-major (entry L * nsamples + k), so the scan of its flags
-// numbers the top cells level by level: the cells of level L are the ids
-// base0 + [id[L * nsamples], id[(L + 1) * nsamples]).
-__global__ void __launch_bounds__(256) top_cells_kernel(Segs g, int nsamples, const uint64_t *__restrict__ skeys,
-                                                        uint32_t *__restrict__ flag, uint32_t *__restrict__ id,
-                                                        int32_t *__restrict__ ta, int32_t *__restrict__ tb,
-                                                        const DeviceState *st)
-{
     if (latched(st)) return;
-    const int gt = blockIdx.x * blockDim.x + threadIdx.x;
-    const int k = gt >> 5, L = gt & 31;
-    if (k >= nsamples || L >= kLevels) return;
-    const int e = L * nsamples + k;
-    flag[e] = 0u;
-    id[e] = 0u;
-    if (L == 0) return;  // the root is wired separately
-    const int s = seg_of_sample(g, k);
-    const int lo = seg_lo(g, s), hi = seg_hi(g, s);
-    const int q = lo + (k - samp_lo(g, s)) * kSubtreeMax;
-    const uint64_t P = prefix_of(skeys[q], L);
-    const int a = lower_prefix(skeys, lo, q + 1, P, L);
-    const int b = upper_prefix(skeys, q, hi, P, L);
-    if (b - a > kSubtreeMax && (q - kSubtreeMax < a || q == lo)) {
-        flag[e] = 1u;
-        id[e] = 1u;
-        ta[e] = a;
-        tb[e] = b;
+    if ((int)blockIdx.x < tb) {
+        const int gt = blockIdx.x * 256 + tid;
+        const int k = gt >> 5, L = gt & 31;
+        if (k >= nsamples || L >= kLevels) return;
+        const int e = L * nsamples + k;
+        if (L == 0) {  // the root is wired separately
+            flag[e] = id[e] = 0u;
+            return;
+        }
+        const int s = seg_of_sample(g, k);
+        const int lo = seg_lo(g, s), hi = seg_hi(g, s);
+        const int q = lo + (k - samp_lo(g, s)) * kSubtreeMax;
+        int a, b;
+        prefix_run(skeys, lo, q, hi, L, a, b);
+        const bool top = b - a > kSubtreeMax && (q - kSubtreeMax < a || q == lo);
+        flag[e] = id[e] = top ? 1u : 0u;
+        if (top) {
+            ta[e] = a;
+            tend[e] = b;
+        }
+        return;
+    }
+    const int stride = (int)(gridDim.x - tb) * 256;
+    for (int k = (int)(blockIdx.x - tb) * 256 + tid; k < g.n; k += stride) {
+        nodes4[pos[k]] = bodies4[k];
+        if (k < g.n - 1) {
+            const uint64_t x = (skeys[k] ^ skeys[k + 1]) & ~(1ull << 63);
+            lcp[k] = x == 0 ? (uint8_t)kKeyLevels : (uint8_t)((62 - (63 - __clzll((long long)x))) / 3);
+        }
     }
 }
 
@@ -999,20 +1037,6 @@ __global__ void __launch_bounds__(256) top_summary_kernel(SumOut o, Segs g, int 
 }
 
 // ------------------------------------------------------------------ layout
-// Bodies in key order as float4 (x, y, z, m) at nodes4[0..n), made right after
-// the build for the summary; in the sort stage sorted[] (the reference's output of
-// that stage) with the group order, and the frame blocks of the force walk
-// (frame_layout_kernel).  The bodies are read in input order and stored at
-// their sorted positions pos[] (the sort's inverse permutation): random 16-byte
-// reads each fetch a whole line, random 16-byte stores only dirty their bytes.
-__global__ void __launch_bounds__(256) sorted_bodies_kernel(int n, const int32_t *__restrict__ pos,
-                                                            const float4 *__restrict__ bodies4,
-                                                            float4 *__restrict__ nodes4, const DeviceState *st)
-{
-    if (latched(st)) return;
-    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += blockDim.x * gridDim.x) nodes4[pos[i]] = bodies4[i];
-}
-
 // Frame blocks.  Block b lists the non-empty children of one cell, compacted in
 // slot order, as the records [off(b), off(b) + k_b) of the packed arrays:
 // fnode[off(b) + k] = (x, y, z, m) of the child and fmeta[off(b) + k] its
@@ -1362,23 +1386,26 @@ static inline int capped_grid(int64_t work, int cap = 65536)
 }
 
 
-// Workgroups of a job loop (subtree build, locked insertion, subtree summary):
-// about one per subtree (a subtree averages about 256 bodies), at least
-// kBuildBlocks.  With many jobs per workgroup the stride balances them worse:
-// at N = 48.8M, 16384 summary workgroups took 3.50 ms against 3.30 ms for a
-// shared job counter.
+// Workgroups of a job loop (subtree build, locked insertion, subtree summary, group
+// order): a few per subtree (a subtree averages about 256 bodies) up to kBuildBlocks,
+// which leaves about one each at 4M bodies, and about one per subtree above.  With
+// many jobs per workgroup the stride balances them worse: at N = 48.8M, 16384 summary
+// workgroups took 3.50 ms against 3.30 ms for a shared job counter.  Workgroups that
+// find no job still have to be dispatched: at N = 2,000, 16384 of them cost each of these
+// kernels several microseconds.
 static int job_grid(int nbodies)
 {
-    return std::min(1 << 20, std::max(kBuildBlocks, nbodies / 256));
+    return std::min(1 << 20, std::max({256, std::min(kBuildBlocks, nbodies / 64), nbodies / 256}));
 }
 
 static void build_tree(Segs g, int nsamples, int base0, int m, TreeScratch &ts, DeviceState *st, hipStream_t s,
-                       int n, const uint64_t *skeys, const int32_t *perm, const uint64_t *keys, int *child,
-                       int *index, int32_t *cell_level, int *start, bool locked)
+                       int n, const uint64_t *skeys, const int32_t *perm, const uint64_t *keys,
+                       const int32_t *pos, const float4 *bodies4, float4 *nodes4, int *child, int *index,
+                       int32_t *cell_level, int *start, bool locked)
 {
-    lcp_kernel<<<capped_grid(n), 256, 0, s>>>(n, skeys, ts.lcp, st);
-    top_cells_kernel<<<(32 * nsamples + 255) / 256, 256, 0, s>>>(g, nsamples, skeys, ts.top_flag, ts.top_id, ts.top_a,
-                                                             ts.top_b, st);
+    const int tb = (32 * nsamples + 255) / 256;
+    after_sort_kernel<<<tb + capped_grid(n), 256, 0, s>>>(g, nsamples, tb, skeys, ts.top_flag, ts.top_id, ts.top_a,
+                                                          ts.top_b, ts.lcp, pos, bodies4, nodes4, st);
     launch_exclusive_scan_u32(ts.top_id, nsamples * kLevels, ts.scan_tmp, s);
     const int wire = nsamples * kLevels + g.nseg;  // entries, 8 lanes each
     top_wire_kernel<<<(8 * wire + 255) / 256, 256, 0, s>>>(g, nsamples, skeys, perm, child, cell_level, ts.top_flag,
@@ -1444,9 +1471,8 @@ void launch_build(nbx_context *c, hipStream_t s, int n, int m, int *child, int *
 {
     if (n <= 0) return;
     Segs g{nullptr, nullptr, 1, n, 0};
-    build_tree(g, samples_of(n), n, m, c->ts, c->st, s, n, c->skeys, c->perm, c->keys, child, index, c->cell_level,
-               c->start, c->p.build_locked != 0);
-    sorted_bodies_kernel<<<capped_grid(n), 256, 0, s>>>(n, c->pos, c->bodies4, c->nodes4, c->st);
+    build_tree(g, samples_of(n), n, m, c->ts, c->st, s, n, c->skeys, c->perm, c->keys, c->pos, c->bodies4, c->nodes4,
+               child, index, c->cell_level, c->start, c->p.build_locked != 0);
 }
 
 void launch_summarize(nbx_context *c, hipStream_t s)
@@ -1491,9 +1517,8 @@ void launch_frame_layout(nbx_context *c, hipStream_t s)
 void launch_batch_build(nbx_batch *b, hipStream_t s)
 {
     Segs g{b->off, b->samp_off, b->S, b->N, 1};
-    build_tree(g, b->ts.samples_max, b->N + b->S, b->m, b->ts, b->st, s, b->N, b->skeys, b->perm, b->keys, b->child,
-               b->index, b->cell_level, b->start, b->p.build_locked != 0);
-    sorted_bodies_kernel<<<capped_grid(b->N), 256, 0, s>>>(b->N, b->pos, b->bodies4, b->nodes4, b->st);
+    build_tree(g, b->ts.samples_max, b->N + b->S, b->m, b->ts, b->st, s, b->N, b->skeys, b->perm, b->keys, b->pos,
+               b->bodies4, b->nodes4, b->child, b->index, b->cell_level, b->start, b->p.build_locked != 0);
 }
 
 void launch_batch_summarize(nbx_batch *b, hipStream_t s)
