@@ -343,32 +343,13 @@ __global__ void __launch_bounds__(256) subtree_cells_kernel(const int4 *__restri
     }
 }
 
-// One workgroup of 1024 threads: 16 counts per thread per pass.
 __global__ void __launch_bounds__(1024) subtree_base_kernel(uint32_t *__restrict__ cbase, int sub_max, int base0,
                                                             int m, int *index, DeviceState *st)
 {
     __shared__ uint32_t sh[16];
     if (latched(st)) return;
     const int nsub = min(__hip_atomic_load(&st->nsub, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), sub_max);
-    constexpr int V = 16;
-    uint32_t carry = 0;
-    for (int t0 = 0; t0 < nsub; t0 += V * (int)blockDim.x) {
-        const int i0 = t0 + V * (int)threadIdx.x;
-        uint32_t v[V], s = 0;
-#pragma unroll
-        for (int u = 0; u < V; ++u) {
-            v[u] = i0 + u < nsub ? cbase[i0 + u] : 0u;
-            s += v[u];
-        }
-        uint32_t tot;
-        uint32_t run = carry + block_exclusive_scan(s, sh, &tot);
-#pragma unroll
-        for (int u = 0; u < V; ++u) {
-            if (i0 + u < nsub) cbase[i0 + u] = run;
-            run += v[u];
-        }
-        carry += tot;
-    }
+    const uint32_t carry = scan_in_place(cbase, nsub, sh);
     if (threadIdx.x == 0) {
         cbase[nsub] = carry;  // so that subtree j has cbase[j + 1] - cbase[j] cells for every j
         const int64_t end = (int64_t)base0 + st->ntop + carry;
@@ -561,7 +542,7 @@ __global__ void __launch_bounds__(256) subtree_insert_kernel(
     }
 }
 
-// Subtree build, without locks or atomics on child slots.  One wave builds one
+// Subtree build, without locks or atomics on child slots.  One workgroup builds one
 // subtree [a, b) of sorted bodies whose root is at level L0 (a child range of
 // a top cell, 2..kSubtreeMax bodies).  With l[i] the number of key digits that
 // local bodies i and i+1 share (l[cnt-1] = L0 - 1 at the subtree's edge) and
@@ -569,179 +550,179 @@ __global__ void __launch_bounds__(256) subtree_insert_kernel(
 // more bodies that share L digits, L = L0..21, and body i starts exactly the
 // cells of levels P_i < L <= l[i].  Numbering cells by first body, then level,
 //     id(i, L) = base + cs[i] + (L - P_i - 1),   cs = exclusive sum of max(0, l[i] - P_i),
-// gives every cell its id from one prefix sum (base from one atomicAdd).
+// gives every cell its id from one prefix sum (base from subtree_base_kernel).
 // The parent of cell (i, L), L > L0, is (i, L-1) when L-1 > P_i; otherwise the
-// level-P_i cell that holds bodies i-1 and i, which starts at
-//     s_i = 1 + the last j < i-1 with l[j] < P_i   (0 if none),
-// a previous-smaller-value query answered by binary lifting over a table of
-// range minima of l in LDS.  The deepest cell of body i is (i, l[i]) when
-// l[i] > P_i, else the same (s_i, P_i).  A child takes the slot of its key
-// digit at the parent's level; in a level-21 bucket (equal keys) the bodies
-// take slots 0, 1, ... in sorted order, which is ascending index order.
-// Each slot thus has exactly one writer: the wave sets the slots of its cells
-// to -1, waits for those stores, and every cell and body stores itself into
-// its parent.  Every id and slot is range-checked before its store.
-constexpr int kLiftLevels = 10;  // 2^kLiftLevels >= kSubtreeMax
+// level-P_i cell that holds bodies i-1 and i, which starts at the first body s_i
+// that shares P_i digits with body i, found by a search over the keys in LDS.  The
+// deepest cell of body i is (i, l[i]) when l[i] > P_i, else the same (s_i, P_i).
+// A child takes the slot of its key digit at the parent's level; in a level-21
+// bucket (equal keys) the bodies take slots 0, 1, ... in sorted order, which is
+// ascending index order.  Each slot thus has exactly one writer: every cell and body
+// stores itself into its parent's slot in LDS, and the slots go out in one
+// contiguous store per cell.  Every id and slot is range-checked before its store.
+//
+// Latency bounds it: a chain of loads, a scan, a search and stores per subtree.  So
+// a thread has at most four bodies (one wave with up to sixteen, a table of
+// range minima for s_i and the slots stored to memory twice, empty and filled:
+// 2,000 bodies 22 us, now 10; 150,000: 36 and 13.5; 1M:
+// 48 and 30; 4M: 104 and 88), and, as in the summary, the subtrees of a launch are those that fit its
+// POOL of slots and not one of BELOW bytes; with REST also those that fit none,
+// whose slots are stored to memory directly.
+constexpr int kBuildSmall = 12672, kBuildSmallT = 128;  // 12 workgroups of 128 threads share a CU
+constexpr int kBuildPool = 26752;                       // six of 256; 1,024 bodies with 515 cells
+__host__ __device__ constexpr int build_bytes(int ks, int nb) { return 32 * ks + 10 * nb + 32; }
 // Workgroups stride over the jobs.  With about one job each at N = 4M (16,400
 // subtrees), the dispatcher starts a new workgroup wherever one has finished,
 // which balances subtrees of 2 to 1024 bodies better than a few jobs per
-// resident workgroup (0.141 ms with 4096 workgroups, 0.103 ms with 16384).
+// resident workgroup (with one wave each, 0.141 ms with 4096 workgroups, 0.103 ms
+// with 16384).
 constexpr int kBuildBlocks = 16384;
 
-__device__ inline int wave_exclusive_sum(int v, int *total)
+__device__ inline int shared_digits(uint64_t a, uint64_t b)  // of two keys, 21 if equal
 {
-    const int lane = threadIdx.x & 63;
-    int x = v;
-    for (int o = 1; o < 64; o <<= 1) {
-        const int y = __shfl_up(x, o);
-        if (lane >= o) x += y;
-    }
-    *total = __shfl(x, 63);
-    return x - v;
+    const uint64_t x = (a ^ b) & ~(1ull << 63);
+    return x == 0 ? kKeyLevels : (__clzll((long long)x) - 1) / 3;
 }
 
-__global__ void __launch_bounds__(64) subtree_build_kernel(
-    int m, const uint64_t *__restrict__ skeys, const int32_t *__restrict__ perm, const uint8_t *__restrict__ lcp,
-    int *__restrict__ child, int base0, const uint32_t *__restrict__ cbase, int32_t *__restrict__ cell_level,
-    int *__restrict__ start, const int4 *__restrict__ sub, int sub_max, int4 *__restrict__ subcells,
-    DeviceState *st)
+template <int T, int POOL, int BELOW>
+__global__ void __launch_bounds__(T, 6) subtree_build_kernel(
+    int m, const uint64_t *__restrict__ skeys, const int32_t *__restrict__ perm, int *__restrict__ child, int base0,
+    const uint32_t *__restrict__ cbase, int32_t *__restrict__ cell_level, int *__restrict__ start,
+    const int4 *__restrict__ sub, int sub_max, int4 *__restrict__ subcells, DeviceState *st)
 {
-    constexpr int C = kSubtreeMax / 64;                   // bodies per lane at most
-    __shared__ uint8_t s_min[kLiftLevels][kSubtreeMax];  // s_min[j][x] = min of l over [x, x + 2^j)
-    __shared__ uint16_t s_cs[kSubtreeMax];                 // cs[i] (ids relative to base)
-    if (latched(st)) return;
-    const int lane = threadIdx.x;
+    constexpr bool REST = POOL == kBuildPool;
+    constexpr int C = 4, W = T / 64;  // bodies per thread at most; waves
+    static_assert(!REST || (C * T >= kSubtreeMax && build_bytes(0, kSubtreeMax) <= POOL), "the keys fit without the slots");
+    __shared__ int s_stop, s_cnt[C][W], s_deep[W];
+    __shared__ __align__(16) unsigned char s_pool[POOL];
+    if (threadIdx.x == 0) s_stop = latched(st);  // one read: this launch raises the latch itself
+    __syncthreads();
+    if (s_stop) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nsub = min(__hip_atomic_load(&st->nsub, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), sub_max);
     const int top = base0 + __hip_atomic_load(&st->ntop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (int job = blockIdx.x; job < nsub; job += gridDim.x) {
         const int4 jb = sub[job];
         const uint32_t cb0 = cbase[job], cb1 = cbase[job + 1];
-        const int base = top + (int)cb0;  // ids reserved by subtree_base_kernel
+        const int base = top + (int)cb0, ks = (int)(cb1 - cb0);  // ids reserved by subtree_base_kernel
         const int a = jb.x, cnt = jb.y - jb.x, L0 = jb.z, slot = jb.w;
-        if (cnt < 2 || cnt > kSubtreeMax || L0 < 1 || L0 > kKeyLevels) {
-            if (lane == 0) {
+        const bool fits = ks >= 0 && ks < 65536 && cnt <= C * T && build_bytes(ks, cnt) <= POOL;
+        if (fits ? BELOW > 0 && cnt <= 4 * kBuildSmallT && build_bytes(ks, cnt) <= BELOW : !REST) continue;
+        if (cnt < 2 || cnt > kSubtreeMax || L0 < 1 || L0 > kKeyLevels || ks < 1 || ks > 65535 ||
+            (int64_t)base + ks > (int64_t)m) {
+            if (tid == 0) {
                 atomicOr(&st->err, kErrCapacity);
                 subcells[job] = make_int4(0, 0, L0, L0 - 1);
             }
             continue;
         }
-        // every global load of the job is issued before the first wait: l[]
-        // (lane-strided), then the lane's own chunk [i0, i1) of keys and bodies
-        const int chunk = (cnt + 63) >> 6;
-        const int i0 = min(cnt, lane * chunk), i1 = min(cnt, i0 + chunk);
-        int lv[C];
+        uint64_t *key = (uint64_t *)s_pool;
+        int *cslots = (int *)(s_pool + ((10 * cnt + 15) & ~15));
+        uint16_t *cs = (uint16_t *)(key + cnt);  // cs[i] (ids relative to base)
+        int *gslots = child + 8 * (int64_t)base;
         uint64_t kq[C];
         int pq[C];
 #pragma unroll
         for (int q = 0; q < C; ++q) {
-            const int i = lane + 64 * q;
-            lv[q] = i < cnt - 1 ? (int)lcp[a + i] : L0 - 1;
+            const int i = tid + T * q;
+            if (i >= cnt) break;
+            kq[q] = skeys[a + i];
+            pq[q] = perm[a + i];
         }
-#pragma unroll
-        for (int q = 0; q < C; ++q) {
-            const bool in = i0 + q < i1;
-            kq[q] = in ? skeys[a + i0 + q] : 0ull;
-            pq[q] = in ? perm[a + i0 + q] : 0;
-        }
+        const int4 none = make_int4(-1, -1, -1, -1);
+        for (int k = tid; k < 2 * ks; k += T) (fits ? (int4 *)cslots : (int4 *)gslots)[k] = none;
 #pragma unroll
         for (int q = 0; q < C; ++q)
-            if (lane + 64 * q < cnt) s_min[0][lane + 64 * q] = (uint8_t)lv[q];
+            if (tid + T * q < cnt) key[tid + T * q] = kq[q];
+        if (!fits) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
         __syncthreads();
-        int mine = 0, deep = L0;
+        int l[C], P[C], run[C], deep = L0;
 #pragma unroll
         for (int q = 0; q < C; ++q) {
-            const int i = i0 + q;
-            if (i >= i1) break;
-            const int P = i == 0 ? L0 - 1 : (int)s_min[0][i - 1];
-            const int l = s_min[0][i];
-            mine += max(0, l - P);
-            deep = max(deep, l);
+            const int i = tid + T * q;
+            l[q] = i < cnt - 1 ? shared_digits(kq[q], key[i + 1]) : L0 - 1;
+            P[q] = i > 0 && i < cnt ? shared_digits(key[i - 1], kq[q]) : L0 - 1;
+            run[q] = i < cnt ? max(0, l[q] - P[q]) : 0;
+            deep = max(deep, l[q]);
         }
-        int ks;
-        int run = wave_exclusive_sum(mine, &ks);
+#pragma unroll
+        for (int q = 0; q < C; ++q) {
+            const int own = run[q];
+            for (int o = 1; o < 64; o <<= 1) {
+                const int y = __shfl_up(run[q], o);
+                if (lane >= o) run[q] += y;
+            }
+            if (lane == 63) s_cnt[q][wave] = run[q];
+            run[q] -= own;
+        }
         for (int o = 32; o > 0; o >>= 1) deep = max(deep, __shfl_xor(deep, o));
+        if (lane == 0) s_deep[wave] = deep;
+        __syncthreads();
+        int total = 0;
 #pragma unroll
-        for (int q = 0; q < C; ++q) {
-            const int i = i0 + q;
-            if (i >= i1) break;
-            const int P = i == 0 ? L0 - 1 : (int)s_min[0][i - 1];
-            s_cs[i] = (uint16_t)run;
-            run += max(0, (int)s_min[0][i] - P);
-        }
-        if (ks < 1 || ks > 65535 || ks != (int)(cb1 - cb0) || (int64_t)base + ks > (int64_t)m) {
-            if (lane == 0) {
+        for (int q = 0; q < C; ++q)
+#pragma unroll
+            for (int w = 0; w < W; ++w) {
+                if (w == wave) run[q] += total;
+                total += s_cnt[q][w];
+            }
+        for (int w = 0; w < W; ++w) deep = max(deep, s_deep[w]);
+#pragma unroll
+        for (int q = 0; q < C; ++q)
+            if (tid + T * q < cnt) cs[tid + T * q] = (uint16_t)run[q];
+        __syncthreads();
+        if (total != ks) {  // uniform: the counts of subtree_cells_kernel do not hold
+            if (tid == 0) {
                 atomicOr(&st->err, kErrCapacity);
                 subcells[job] = make_int4(0, 0, L0, L0 - 1);
             }
             __syncthreads();
             continue;
         }
-        // range-minimum table over the cnt - 1 shared-digit counts
-        for (int j = 1; j < kLiftLevels && (1 << j) <= cnt - 1; ++j) {
-            __syncthreads();
-            const int h = 1 << (j - 1);
-            for (int x = lane; x + (1 << j) <= cnt - 1; x += 64)
-                s_min[j][x] = (uint8_t)min((int)s_min[j - 1][x], (int)s_min[j - 1][x + h]);
-        }
-        // empty slots, cell levels and starts
-        int *cslots = child + 8 * (int64_t)base;
-        for (int k = lane; k < 8 * ks; k += 64) cslots[k] = -1;
-#pragma unroll
-        for (int q = 0; q < C; ++q) {
-            const int i = i0 + q;
-            if (i >= i1) break;
-            const int P = i == 0 ? L0 - 1 : (int)s_min[0][i - 1];
-            const int l = s_min[0][i];
-            for (int L = P + 1; L <= l; ++L) {
-                const int c = base + (int)s_cs[i] + (L - P - 1);
-                cell_level[c] = L;
-                start[c] = a + i;
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
-        __syncthreads();
         // every cell (but the root) and every body into its parent's slot
         bool bad = false;
+        const auto put = [&](int par, int d, int v) {
+            if (par < 0 || par >= ks || d >= 8) bad = true;
+            else if (fits) cslots[8 * par + d] = v;
+            else gslots[8 * (int64_t)par + d] = v;
+        };
 #pragma unroll
         for (int q = 0; q < C; ++q) {
-            const int i = i0 + q;
-            if (i >= i1) break;
-            const int P = i == 0 ? L0 - 1 : (int)s_min[0][i - 1];
-            const int l = s_min[0][i];
-            const uint64_t key = kq[q];
-            const int own = (int)s_cs[i] - P - 1;  // id(i, L) - base = own + L
-            // start of the level-P run through i (only used for i >= 1)
-            int s = 0;
+            const int i = tid + T * q;
+            if (i >= cnt) break;
+            const int own = run[q] - P[q] - 1;  // id(i, L) - base = own + L
+            int s = 0, up = 0;                  // start of the level-P run through i >= 1, its id - base
             if (i >= 1) {
-                int p = i - 1;
-                for (int j = kLiftLevels - 1; j >= 0; --j) {
-                    const int w = 1 << j;
-                    if (p - w >= 0 && (int)s_min[j][p - w] >= P) p -= w;
+                const uint64_t want = prefix_of(kq[q], P[q]);
+                int hi = i - 1;
+                while (s < hi) {
+                    const Quarter z = quarter_probes(s, hi);
+                    const uint64_t k0 = key[z.m[0]], k1 = key[z.m[1]], k2 = key[z.m[2]];
+                    quarter_step(s, hi, z, prefix_of(k0, P[q]) < want, prefix_of(k1, P[q]) < want,
+                                 prefix_of(k2, P[q]) < want);
                 }
-                s = p;
+                const int Ps = s == 0 ? L0 - 1 : shared_digits(key[s - 1], key[s]);
+                up = (int)cs[s] - Ps - 1 + P[q];
             }
-            const int Ps = s == 0 ? L0 - 1 : (int)s_min[0][s - 1];
-            const int up = (int)s_cs[s] - Ps - 1 + P;  // id(s, P) - base
-            for (int L = max(P + 1, L0 + 1); L <= l; ++L) {
-                const int par = L - 1 > P ? own + L - 1 : up;
-                const int d = digit_at(key, L - 1);
-                if (par < 0 || par >= ks) { bad = true; continue; }
-                child[8 * ((int64_t)base + par) + d] = base + own + L;
+            for (int L = P[q] + 1; L <= l[q]; ++L) {
+                const int c = own + L;
+                if (c < 0 || c >= ks) { bad = true; break; }
+                cell_level[base + c] = L;
+                start[base + c] = a + i;
+                if (L > L0) put(L - 1 > P[q] ? c - 1 : up, digit_at(kq[q], L - 1), base + c);
             }
-            const int D = max(P, l);
-            const int par = l > P ? own + l : up;
-            const int d = D < kKeyLevels ? digit_at(key, D) : (l > P ? 0 : i - s);
-            if (par < 0 || par >= ks || d >= 8) { bad = true; continue; }
-            child[8 * ((int64_t)base + par) + d] = pq[q];
+            const int D = max(P[q], l[q]);
+            put(l[q] > P[q] ? own + l[q] : up, D < kKeyLevels ? digit_at(kq[q], D) : l[q] > P[q] ? 0 : i - s, pq[q]);
         }
-        if (__ballot(bad) && lane == 0) atomicOr(&st->err, kErrBucket);
-        if (lane == 0) {
+        if (bad) atomicOr(&st->err, kErrBucket);
+        if (tid == 0) {
             child[slot] = base;
             subcells[job] = make_int4(base, ks, L0, deep);
         }
-        // one wave per workgroup: its LDS operations are in order, so the next
-        // job may overwrite the tables without waiting for these stores
-        __builtin_amdgcn_wave_barrier();
+        __syncthreads();
+        if (fits)
+            for (int k = tid; k < 2 * ks; k += T) ((int4 *)gslots)[k] = ((const int4 *)cslots)[k];
+        __syncthreads();  // the next job overwrites the pool
     }
 }
 
@@ -750,6 +731,17 @@ struct CellSum {
     double ms, mx, my, mz;
     int cnt, first;
 };
+
+// The slots v[] of the level-21 bucket c in ascending index order, the stable key order.
+__device__ inline void order_bucket(int *child, int c, int *v)
+{
+    for (int i = 1; i < 8; ++i) {
+        int a = v[i], j = i - 1;
+        while (j >= 0 && (v[j] == -1 || (a != -1 && v[j] > a))) { v[j + 1] = v[j]; --j; }
+        v[j + 1] = a;
+    }
+    for (int s = 0; s < 8; ++s) child[8 * (int64_t)c + s] = v[s];
+}
 
 // Sums the children of c in slot order; a level-21 bucket first puts its
 // bodies (equal keys) in ascending index order, the stable key order.  The
@@ -765,26 +757,16 @@ struct CellSum {
 // subtrees (more would cost occupancy: 4 needs 90 registers against 59), 4 for
 // the top cells.  CURSOR: the build has given every cell its first sorted body
 // (first >= 0), which the summary then neither reads for the children nor
-// stores again.  LCNT: the counts of the cells [lbase, ...) of a subtree are
-// in LDS at lcnt (every cell child of a subtree cell is one of them).
-template <int B, bool CURSOR, bool LCNT>
-__device__ inline CellSum sum_cell(int c, int first, bool bucket, int n, int *child, const int *lslots,
-                                   const float4 *bodies4, const float4 *sorted4, const int32_t *pos,
-                                   const double4 *sum64, const int *count, const int *start,
-                                   const uint16_t *lcnt, int lbase)
+// stores again.
+template <int B, bool CURSOR>
+__device__ inline CellSum sum_cell(int c, int first, bool bucket, int n, int *child, const float4 *bodies4,
+                                   const float4 *sorted4, const int32_t *pos, const double4 *sum64,
+                                   const int *count, const int *start)
 {
     int v[8];
-    const int *src = lslots ? lslots : child + 8 * (int64_t)c;
 #pragma unroll
-    for (int s = 0; s < 8; ++s) v[s] = src[s];
-    if (bucket) {
-        for (int i = 1; i < 8; ++i) {
-            int a = v[i], j = i - 1;
-            while (j >= 0 && (v[j] == -1 || (a != -1 && v[j] > a))) { v[j + 1] = v[j]; --j; }
-            v[j + 1] = a;
-        }
-        for (int s = 0; s < 8; ++s) child[8 * (int64_t)c + s] = v[s];
-    }
+    for (int s = 0; s < 8; ++s) v[s] = child[8 * (int64_t)c + s];
+    if (bucket) order_bucket(child, c, v);
     CellSum r{0.0, 0.0, 0.0, 0.0, 0, 0x7fffffff};
     int cur = first;
 #pragma unroll
@@ -800,7 +782,7 @@ __device__ inline CellSum sum_cell(int c, int first, bool bucket, int n, int *ch
             cx[t] = cs.y;
             cy[t] = cs.z;
             cz[t] = cs.w;
-            kc[t] = LCNT ? (v[s0 + t] >= n ? lcnt[v[s0 + t] - lbase] : 0) : count[q];
+            kc[t] = count[q];
             kf[t] = CURSOR ? 0 : start[q];
         }
 #pragma unroll
@@ -855,99 +837,209 @@ struct SumOut {
     int cursor;              // cell starts known before the summary
 };
 
-// lev: the cell's level when the caller has it (else -1); lslots: an LDS copy of
-// its slots (else nullptr); with LCNT, lcnt holds the subtree's counts in LDS
-// from lbase and gets this cell's count too, and lfirst is the cell's first
-// sorted body (staged by the caller; with CURSOR only).
-// B: slots whose loads go together; CURSOR: o.cursor (sum_cell).
-template <int B, bool CURSOR, bool LCNT = false>
-__device__ inline void summarise(const SumOut &o, int c, DeviceState *st, bool single_root, int root_first = 0,
-                                 int lev = -1, const int *lslots = nullptr, uint16_t *lcnt = nullptr, int lbase = 0,
-                                 int lfirst = -1)
+__device__ inline void store_cell(const SumOut &o, int c, const CellSum &r, DeviceState *st)
 {
-    const bool bucket = !single_root && (lev >= 0 ? lev : o.cell_level[c]) == kKeyLevels;
-    const int first = !CURSOR ? -1 : single_root ? root_first : LCNT ? lfirst : o.start[c];
-    const CellSum r = sum_cell<B, CURSOR, LCNT>(c, first, bucket, o.n, o.child, lslots, o.bodies4, o.nodes4, o.pos, o.sum64,
-                                  o.count, o.start, lcnt, lbase);
     if (r.cnt > 0 && !(r.ms > 0.0)) atomicOr(&st->err, kErrNonFinite);
-    const double gx = r.mx / r.ms, gy = r.my / r.ms, gz = r.mz / r.ms;
-    const float fx = (float)gx, fy = (float)gy, fz = (float)gz, fm = (float)r.ms;
-    if (single_root) {
-        st->root64[0] = r.ms; st->root64[1] = gx; st->root64[2] = gy; st->root64[3] = gz;
-        st->root4 = make_float4(fx, fy, fz, fm);
-        return;
-    }
+    const float fx = (float)(r.mx / r.ms), fy = (float)(r.my / r.ms), fz = (float)(r.mz / r.ms), fm = (float)r.ms;
     o.sum64[c] = make_double4(r.ms, r.mx, r.my, r.mz);
     if (o.cx) {
         o.cx[c] = fx; o.cy[c] = fy; o.cz[c] = fz; o.mass[c] = fm;
     }
     o.count[c] = r.cnt;
-    if (LCNT) lcnt[c - lbase] = (uint16_t)r.cnt;  // a subtree holds at most kSubtreeMax bodies
-    if (!CURSOR) o.start[c] = r.first;
+    if (!o.cursor) o.start[c] = r.first;
     o.nodes4[c] = make_float4(fx, fy, fz, fm);
+}
+
+// lev: the cell's level when the caller has it (else -1).
+// B: slots whose loads go together; CURSOR: o.cursor (sum_cell).
+template <int B, bool CURSOR>
+__device__ inline void summarise(const SumOut &o, int c, DeviceState *st, bool single_root, int root_first = 0,
+                                 int lev = -1)
+{
+    const bool bucket = !single_root && (lev >= 0 ? lev : o.cell_level[c]) == kKeyLevels;
+    const int first = !CURSOR ? -1 : single_root ? root_first : o.start[c];
+    const CellSum r = sum_cell<B, CURSOR>(c, first, bucket, o.n, o.child, o.bodies4, o.nodes4, o.pos, o.sum64,
+                                          o.count, o.start);
+    if (!single_root) {
+        store_cell(o, c, r, st);
+        return;
+    }
+    if (r.cnt > 0 && !(r.ms > 0.0)) atomicOr(&st->err, kErrNonFinite);
+    const double gx = r.mx / r.ms, gy = r.my / r.ms, gz = r.mz / r.ms;
+    st->root64[0] = r.ms; st->root64[1] = gx; st->root64[2] = gy; st->root64[3] = gz;
+    st->root4 = make_float4((float)gx, (float)gy, (float)gz, (float)r.ms);
 }
 
 // Subtree summary: workgroup w sums subtrees w, w + gridDim.x, ...: with as many
 // workgroups as subtrees, about, the dispatcher hands each free slot of a CU
 // the next workgroup, a job queue with no shared counter.  The cells of a
-// subtree are the contiguous ids [base, base + ks), summed deepest
-// level first with a barrier between levels.  A subtree of up to kSumLdsCells
-// cells first copies its cells' levels and slots into LDS (one coalesced read),
-// and keeps the count of every cell it has summed there, so a level costs the
-// reads of the children's FP64 sums and bodies and the stores only.
-constexpr int kSumLdsCells = 512;
+// subtree are the contiguous ids [base, base + ks), its bodies the sorted range
+// [a, a + nb), and a cell waits for the level below it: a chain of up to 20 steps
+// that sets the time at every size (a subtree has 5 to 15 levels of few cells).  So
+// the subtree first comes into LDS, every load issued before the first wait, and its
+// cells are listed by level; the levels then run from the deepest up on LDS alone,
+// four lanes per cell, one for each of its four sums; and the centres, the divisions
+// and every store follow at the end, all cells side by side.  A cell's record holds
+// its slots until it is summed, then its sums.  (Sums and bodies read from memory and
+// results stored level by level: 2,000 bodies 32 us, now 11; 150,000: 43 and
+// 17; 1M: 86 and 43; 4M: 311 and 141.)
+//
+// What a subtree needs of LDS varies (a mean of 9 KB, at most some 43), and the
+// subtrees a CU holds at once are what hides their chains.  A launch takes those that
+// fit its POOL and, with BELOW > 0, do not fit a pool of BELOW bytes; with REST, the
+// subtrees that fit no pool too, which are summed in memory.
+constexpr int kSumSmall = 9920, kSumSmallT = 128;  // 16 workgroups of 128 threads share a CU
+constexpr int kSumPool = 40672;                    // four of 256; 1,024 bodies with 620 cells
+constexpr int kSumCells = 3;                       // cells a thread stages at most, and four bodies
 constexpr int kSubSumBatch = 2;
-template <bool CURSOR>
-__global__ void __launch_bounds__(256) subtree_summary_kernel(SumOut o, const int4 *__restrict__ subcells,
-                                                              DeviceState *st)
+__device__ inline bool sum_fits(int ks, int nb, int threads, int pool)
 {
-    __shared__ int s_job;
-    // 19,972 bytes of LDS (20 KB as allocated): eight workgroups of 256 threads
-    // fit a CU's 160 KB
-    __shared__ uint8_t s_lev[kSumLdsCells];
-    __shared__ int s_slot[8 * kSumLdsCells];
-    __shared__ uint16_t s_cnt[kSumLdsCells];  // counts of the subtree's summed cells
-    __shared__ int s_first[kSumLdsCells];     // first sorted body of each cell (CURSOR)
-    static_assert(kSubtreeMax < 65536 && kKeyLevels < 256, "counts and levels fit the LDS types");
+    return 39 * ks + 16 * nb + 72 <= pool && ks <= kSumCells * threads && nb <= 4 * threads;
+}
+
+template <bool CURSOR, int T, int POOL, int BELOW>
+__global__ void __launch_bounds__(T, POOL == kSumSmall ? 8 : 4) subtree_summary_kernel(
+    SumOut o, const int4 *__restrict__ sub, int sub_max, const int4 *__restrict__ subcells, DeviceState *st)
+{
+    constexpr bool REST = POOL == kSumPool;
+    static_assert(!REST || kSubtreeMax <= 4 * T, "a thread stages four bodies");
+    __shared__ int s_stop, s_hist[kLevels], s_from[kLevels + 1];
+    __shared__ __align__(32) unsigned char s_pool[POOL];
     const int tid = threadIdx.x;
-    const int nsub = __hip_atomic_load(&st->nsub, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    int next = blockIdx.x;
-    for (;;) {
-        // One read of the latch per job, by thread 0, published with the job:
-        // the workgroup continues or leaves as a whole (a zero cell mass raises
-        // the latch from inside this launch).
-        if (tid == 0) s_job = latched(st) ? nsub : next;
-        next += gridDim.x;
+    const int nsub = min(__hip_atomic_load(&st->nsub, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), sub_max);
+    for (int job = blockIdx.x; job < nsub; job += gridDim.x) {
+        const int4 sc = subcells[job], jb = sub[job];
+        const int base = sc.x, ks = sc.y, L0 = sc.z, a = jb.x, nb = jb.y - jb.x;
+        const bool fits = sum_fits(ks, nb, T, POOL);
+        if (fits ? BELOW > 0 && sum_fits(ks, nb, kSumSmallT, BELOW) : !REST) continue;
+        // One read of the latch per job, by thread 0, published to the workgroup,
+        // which continues or leaves as a whole (a zero cell mass raises the latch
+        // from inside this launch).
+        if (tid == 0) s_stop = latched(st);
+        if (tid < kLevels) s_hist[tid] = 0;
         __syncthreads();
-        const int job = s_job;
-        __syncthreads();
-        if (job >= nsub) break;
-        const int4 sc = subcells[job];
-        const int base = sc.x, ks = sc.y, L0 = sc.z;
-        const bool lds = ks <= kSumLdsCells;
-        if (lds) {
-            for (int k = tid; k < ks; k += blockDim.x) {
-                s_lev[k] = (uint8_t)o.cell_level[base + k];
-                if (CURSOR) s_first[k] = o.start[base + k];
-            }
-            for (int k = tid; k < 8 * ks; k += blockDim.x) s_slot[k] = o.child[8 * (int64_t)base + k];
-            __syncthreads();
-        }
-        if (lds) {  // levels, slots and the counts of summed cells in LDS
-            for (int L = sc.w; L >= L0; --L) {
-                for (int k = tid; k < ks; k += blockDim.x)
-                    if (s_lev[k] == L)
-                        summarise<kSubSumBatch, CURSOR, true>(o, base + k, st, false, 0, L, s_slot + 8 * k, s_cnt,
-                                                              base, CURSOR ? s_first[k] : -1);
-                __syncthreads();
-            }
-        } else {
+        if (s_stop) break;
+        if (!fits) {
             for (int L = sc.w; L >= L0; --L) {
                 for (int k = tid; k < ks; k += blockDim.x)
                     if (o.cell_level[base + k] == L) summarise<kSubSumBatch, CURSOR>(o, base + k, st, false, 0, L);
                 __syncthreads();
             }
+            continue;
         }
+        // Slots in LDS, 16 bits each, the empty ones left out: a cell's number in the
+        // subtree; `none` after the last; and for a body `one`, or with no cursor
+        // 0x8000 | its position.  The entries `one` and `none` of cnt[] hold 1 and 0.
+        const uint32_t one = ks, none = ks + 1;
+        double4 *rec = (double4 *)s_pool;
+        float4 *body = (float4 *)(rec + ks + 2);
+        uint16_t *cnt = (uint16_t *)(body + nb), *first = cnt + ks + 2, *list = first + ks;
+        uint8_t *lev = (uint8_t *)(list + ks);
+        float4 bv[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (tid + T * u < nb) bv[u] = o.nodes4[a + tid + T * u];
+#pragma unroll
+        for (int u = 0; u < kSumCells; ++u) {
+            const int k = tid + T * u;
+            if (k >= ks) break;
+            const int4 *c4 = (const int4 *)(o.child + 8 * ((int64_t)base + k));
+            const int4 va = c4[0], vb = c4[1];
+            const int lv = o.cell_level[base + k], fv = CURSOR ? o.start[base + k] - a : 0;
+            int v[8] = {va.x, va.y, va.z, va.w, vb.x, vb.y, vb.z, vb.w};
+            if (!CURSOR && lv == kKeyLevels) order_bucket(o.child, base + k, v);
+            uint64_t lo = none * 0x0001000100010001ull, hi = lo;
+#pragma unroll
+            for (int t = 7; t >= 0; --t) {
+                const int ch = v[t];
+                const bool isb = ch >= 0 && ch < o.n, in = isb || (ch > base && ch - base < ks);
+                const uint64_t w = !isb ? (uint32_t)(ch - base)
+                                        : CURSOR ? one : 0x8000u | ((uint32_t)(o.pos[ch] - a) & 0x3ffu);
+                hi = in ? hi << 16 | lo >> 48 : hi;
+                lo = in ? lo << 16 | w : lo;
+            }
+            *(ulonglong2 *)&rec[k] = make_ulonglong2(lo, hi);
+            lev[k] = (uint8_t)lv;
+            first[k] = (uint16_t)fv;
+            cnt[k] = (uint16_t)atomicAdd(&s_hist[lv], 1);  // for now, its number in its level
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (tid + T * u < nb) body[tid + T * u] = bv[u];
+        if (tid < 2) {
+            rec[ks + tid] = make_double4(0.0, 0.0, 0.0, 0.0);
+            cnt[ks + tid] = tid == 0;
+        }
+        __syncthreads();
+        if (tid < 64) {
+            int x = tid < kLevels ? s_hist[tid] : 0;
+            for (int d = 1; d < 32; d <<= 1) {
+                const int y = __shfl_up(x, d);
+                if (tid >= d) x += y;
+            }
+            if (tid < kLevels) s_from[tid + 1] = x;
+            if (tid == 0) s_from[0] = 0;
+        }
+        __syncthreads();
+        for (int k = tid; k < ks; k += T) list[s_from[lev[k]] + cnt[k]] = (uint16_t)k;
+        __syncthreads();
+        const int q = tid & 3;  // this lane's sum: mass, moments x, y, z
+        for (int L = sc.w; L >= L0; --L) {
+            const int to = s_from[L + 1];
+            for (int i = s_from[L] + (tid >> 2); i < to; i += T / 4) {
+                const int k = list[i];
+                const ulonglong2 slots = *(const ulonglong2 *)&rec[k];
+                int at_first = nb, all = CURSOR ? (int)first[k] : 0;
+                const int f0 = all;
+                double sum = 0.0;
+                for (int half = 0; half < 2; ++half) {
+                    const uint64_t wq = half ? slots.y : slots.x;
+                    if ((uint32_t)(wq & 0xffffu) == none) break;
+                    bool isb[4];
+                    int at[4];  // a child's first body
+                    double cs[4];
+                    float bm[4], br[4];
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        const uint32_t w = (uint32_t)(wq >> (16 * t)) & 0xffffu;
+                        isb[t] = CURSOR ? w == one : w >= 0x8000u;
+                        const uint32_t c = !CURSOR && isb[t] ? one : w;
+                        const int kc = cnt[c];
+                        cs[t] = ((const double *)rec)[4 * c + q];
+                        if (CURSOR) {
+                            at[t] = all;
+                        } else {
+                            at[t] = isb[t] ? (int)(w & 0x3ffu) : c < one ? (int)first[c] : nb;
+                            at_first = min(at_first, at[t]);
+                        }
+                        all += kc;
+                    }
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        const int e = min(at[t], nb - 1);
+                        bm[t] = body[e].w;
+                        br[t] = ((const float *)body)[4 * e + ((q + 3) & 3)];  // the mass itself for lane 0
+                    }
+#pragma unroll
+                    for (int t = 0; t < 4; ++t) {
+                        const float r = q ? br[t] : 1.0f;
+                        const double v = __dmul_rn((double)bm[t], (double)r);
+                        sum = __dadd_rn(sum, isb[t] ? v : cs[t]);
+                    }
+                }
+                ((double *)rec)[4 * k + q] = sum;
+                if (q == 0) {
+                    cnt[k] = (uint16_t)(all - f0);
+                    if (!CURSOR) first[k] = (uint16_t)at_first;
+                }
+            }
+            __syncthreads();
+        }
+        for (int k = tid; k < ks; k += T) {
+            const double4 r = rec[k];
+            store_cell(o, base + k, CellSum{r.x, r.y, r.z, r.w, (int)cnt[k], a + (int)first[k]}, st);
+        }
+        __syncthreads();  // the next job overwrites the pool
     }
 }
 
@@ -1398,6 +1490,13 @@ static int job_grid(int nbodies)
     return std::min(1 << 20, std::max({256, std::min(kBuildBlocks, nbodies / 64), nbodies / 256}));
 }
 
+// From this many bodies on, the subtrees of a launch go to two pools of LDS by size:
+// there are then several rounds of workgroups, and the small ones leave room for more at
+// once.  Below, nearly all are resident together and a second launch only costs its 4 to
+// 5 us.  Summary, one pool and two: 43 and 50 us at 1M, 162 and 141 at 4M, 366 and 286 at
+// 7.5M bodies in 512 systems; build: 30 and 37, 89 and 88, 207 and 177.
+constexpr int kSumTwoPools = 1 << 21, kBuildTwoPools = 1 << 22;
+
 static void build_tree(Segs g, int nsamples, int base0, int m, TreeScratch &ts, DeviceState *st, hipStream_t s,
                        int n, const uint64_t *skeys, const int32_t *perm, const uint64_t *keys,
                        const int32_t *pos, const float4 *bodies4, float4 *nodes4, int *child, int *index,
@@ -1418,22 +1517,39 @@ static void build_tree(Segs g, int nsamples, int base0, int m, TreeScratch &ts, 
         subtree_insert_kernel<<<job_grid(g.n), 256, 0, s>>>(n, m, skeys, perm, keys, ts.lcp, child, base0,
                                                                 ts.cbase, cell_level, ts.sub, ts.sub_max,
                                                                 ts.subcells, st);
-    else
-        subtree_build_kernel<<<job_grid(g.n), 64, 0, s>>>(m, skeys, perm, ts.lcp, child, base0, ts.cbase, cell_level,
-                                                         start, ts.sub, ts.sub_max, ts.subcells, st);
+    else if (g.n < kBuildTwoPools) {
+        subtree_build_kernel<256, kBuildPool, 0><<<job_grid(g.n), 256, 0, s>>>(m, skeys, perm, child, base0, ts.cbase, cell_level,
+                                                                         start, ts.sub, ts.sub_max, ts.subcells, st);
+    } else {
+        subtree_build_kernel<256, kBuildPool, kBuildSmall><<<job_grid(g.n), 256, 0, s>>>(m, skeys, perm, child, base0, ts.cbase,
+                                                                         cell_level, start, ts.sub, ts.sub_max,
+                                                                         ts.subcells, st);
+        subtree_build_kernel<kBuildSmallT, kBuildSmall, 0><<<job_grid(g.n), kBuildSmallT, 0, s>>>(m, skeys, perm, child, base0, ts.cbase, cell_level,
+                                                                         start, ts.sub, ts.sub_max, ts.subcells, st);
+    }
 }
 
+template <bool CURSOR>
+static void summarise_tree(Segs g, int base0, int nsamples, TreeScratch &ts, DeviceState *st, hipStream_t s,
+                           const SumOut &o)
+{
+    const int grid = job_grid(g.n);
+    if (g.n < kSumTwoPools) {
+        subtree_summary_kernel<CURSOR, 256, kSumPool, 0><<<grid, 256, 0, s>>>(o, ts.sub, ts.sub_max, ts.subcells, st);
+    } else {
+        subtree_summary_kernel<CURSOR, 256, kSumPool, kSumSmall><<<grid, 256, 0, s>>>(o, ts.sub, ts.sub_max, ts.subcells, st);
+        subtree_summary_kernel<CURSOR, kSumSmallT, kSumSmall, 0><<<grid, kSumSmallT, 0, s>>>(o, ts.sub, ts.sub_max, ts.subcells, st);
+    }
+    top_summary_kernel<CURSOR><<<kTopBlocks, 256, 0, s>>>(o, g, base0, nsamples, ts.top_id, st);
+}
 // base0: the first top cell's id; nsamples: the top table's samples.
 static void summarise_tree(Segs g, int base0, int nsamples, TreeScratch &ts, DeviceState *st, hipStream_t s,
                            const SumOut &o)
 {
-    if (o.cursor) {
-        subtree_summary_kernel<true><<<job_grid(g.n), 256, 0, s>>>(o, ts.subcells, st);
-        top_summary_kernel<true><<<kTopBlocks, 256, 0, s>>>(o, g, base0, nsamples, ts.top_id, st);
-    } else {
-        subtree_summary_kernel<false><<<job_grid(g.n), 256, 0, s>>>(o, ts.subcells, st);
-        top_summary_kernel<false><<<kTopBlocks, 256, 0, s>>>(o, g, base0, nsamples, ts.top_id, st);
-    }
+    if (o.cursor)
+        summarise_tree<true>(g, base0, nsamples, ts, st, s, o);
+    else
+        summarise_tree<false>(g, base0, nsamples, ts, st, s, o);
 }
 
 static inline int samples_of(int n) { return (n + kSubtreeMax - 1) / kSubtreeMax; }
