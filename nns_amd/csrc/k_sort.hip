@@ -5,8 +5,9 @@
 // (merge_pass_kernel), every workgroup producing kMergeTile consecutive outputs.
 // Both steps take the left element of equal keys first, so the order is stable.
 // A sort of n pairs is 1 + ceil(log2(n / kSortChunk)) launches, where eight radix
-// passes of 8 bits were 24.  Keys and permutation on one MI355X, radix -> merge:
-// N = 2,000, 95 -> 16 us; 20,011, 127 -> 45; 150,001, 132 -> 71; 1,000,003, 172 -> 127;
+// passes of 8 bits were 24; up to 17 chunks are merged in one launch (rank_merge_kernel).
+// Keys and permutation on one MI355X, radix -> merge:
+// N = 2,000, 95 -> 16 us; 20,011, 127 -> 31; 150,001, 132 -> 71; 1,000,003, 172 -> 127;
 // 4,194,304, 388 -> 370 (and its Morton keys are made on the way, 37 us less); 8.4 M,
 // 737 -> 753.  Chunks of 8,192 pairs take 36 us against 29 at N = 8,192 and 131
 // against 127 at 1M (one workgroup per CU instead of three), chunks of 2,048 139.
@@ -92,7 +93,9 @@ struct SortSource {
 // workgroup (coalesced) and handed to the threads, eight consecutive pairs each, through
 // LDS; each thread sorts its eight, then runs of 8, 16, ... are merged in LDS.
 // Bound by the LDS round trips of the merges (nine rounds of a split search and
-// eight steps each, about 2 us a round): 20 us for one chunk, 102 us for 4M bodies.
+// eight steps each, about 2 us a round, which wait on instruction issue as much as on the
+// LDS: a four-way search took 24, the eight steps as a bitonic network in registers
+// 28): 20 us for one chunk, 102 us for 4M bodies.
 template <bool BODIES>
 __global__ void __launch_bounds__(kChunkThreads) chunk_sort_kernel(SortSource src, const int4 *__restrict__ chunks,
                                                                    int n, uint64_t *__restrict__ kout,
@@ -258,6 +261,102 @@ __global__ void __launch_bounds__(kMergeThreads) merge_pass_kernel(const uint64_
     }
 }
 
+// All merges in one launch, for few pairs in segments of few chunks: a pair's place
+// is its position in its own chunk plus, for every other chunk of the segment, the
+// number of its keys that come before (in an earlier chunk equal keys too).  Every 64th key
+// of every chunk is staged in LDS.  The 64 consecutive pairs of a wave bracket each
+// other: the places of the first and the last in a chunk are found by two ballots over
+// 64 keys each, and the others search between them, four chunks side by side.  Bound by
+// the chain of loads, about 7 us per four chunks, where each doubling of the runs costs a
+// launch of 8 us; every wave meets every chunk, so the work grows with the square of the
+// chunks.  Sort of n pairs, merge passes and this: n = 8,192, 29.4 and 28.9 us;
+// 20,000, 44 and 30; 36,864, 53 and 35; 69,632 (17 chunks), 61 and 48; 150,000, 84 and
+// 114; an ensemble of 7.5M pairs in chunks by at most 16, 419 and 673.
+constexpr int kRankThreads = 256, kRankWidth = 4;
+constexpr int kRankChunks = 17, kRankPairs = 1 << 17;
+
+__device__ inline bool comes_before(uint64_t q, uint64_t k, bool earlier) { return q < k || (earlier && q == k); }
+__device__ inline uint64_t lane_key(uint64_t k, int lane)
+{
+    return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(k >> 32), lane) << 32 |
+           (uint32_t)__builtin_amdgcn_readlane((int)k, lane);
+}
+
+__global__ void __launch_bounds__(kRankThreads) rank_merge_kernel(const uint64_t *__restrict__ kin,
+                                                                  const int32_t *__restrict__ vin,
+                                                                  const int4 *__restrict__ chunks, int n,
+                                                                  uint64_t *__restrict__ kout,
+                                                                  int32_t *__restrict__ vout,
+                                                                  int32_t *__restrict__ inv)
+{
+    constexpr int kSub = kSortChunk / kRankThreads, kEach = kSortChunk / 64;
+    __shared__ uint64_t s_key[kRankChunks * kEach];
+    const int4 ck = chunk_of(chunks, n, blockIdx.x / kSub);
+    const int lane = threadIdx.x & 63;
+    const int own = (int)(blockIdx.x % kSub) * kRankThreads + (int)threadIdx.x;
+    const int len = ck.y - ck.x, z = ck.z, e = z * kSortChunk + own;
+    if (e - (int)threadIdx.x >= len) return;  // the workgroup as a whole
+    const int nc = (len + kSortChunk - 1) / kSortChunk;
+    const uint64_t *seg = kin + ck.x;
+    const uint64_t k = seg[min(e, len - 1)];
+    for (int i = threadIdx.x; i < nc * kEach && i * 64 < len; i += kRankThreads) s_key[i] = seg[64 * i];
+    __syncthreads();
+    if (e - lane >= len) return;
+    const uint64_t kf = lane_key(k, 0), kl = lane_key(k, 63);
+    int to = ck.x + own;
+    for (int i = 0; i < nc - 1; i += kRankWidth) {
+        int from[kRankWidth], lo[kRankWidth], hi[kRankWidth], cf[kRankWidth], cl[kRankWidth], have[kRankWidth];
+        bool earlier[kRankWidth];
+        uint64_t q[kRankWidth], r[kRankWidth];
+#pragma unroll
+        for (int u = 0; u < kRankWidth; ++u) {
+            const int o = min(i + u, nc - 2), c = o + (o >= z);
+            earlier[u] = c < z;
+            from[u] = c * kSortChunk;
+            have[u] = i + u < nc - 1 ? min(kSortChunk, len - from[u]) : 0;
+            q[u] = s_key[c * kEach + lane];
+        }
+#pragma unroll
+        for (int u = 0; u < kRankWidth; ++u) {
+            const bool in = lane * 64 < have[u];
+            cf[u] = __popcll(__ballot(in && comes_before(q[u], kf, earlier[u])));
+            cl[u] = __popcll(__ballot(in && comes_before(q[u], kl, earlier[u])));
+            // the place lies past sample c - 1, and not past sample c
+            q[u] = seg[from[u] + min(64 * max(cf[u] - 1, 0) + lane, max(have[u] - 1, 0))];
+            r[u] = seg[from[u] + min(64 * max(cl[u] - 1, 0) + lane, max(have[u] - 1, 0))];
+        }
+        int width = 0;
+#pragma unroll
+        for (int u = 0; u < kRankWidth; ++u) {
+            const int bf = 64 * (cf[u] - 1), bl = 64 * (cl[u] - 1);
+            const int pf = __popcll(__ballot(bf + lane < have[u] && comes_before(q[u], kf, earlier[u])));
+            const int pl = __popcll(__ballot(bl + lane < have[u] && comes_before(r[u], kl, earlier[u])));
+            lo[u] = cf[u] ? bf + pf : 0;
+            hi[u] = cl[u] ? bl + pl : 0;
+            width = max(width, hi[u] - lo[u]);
+        }
+        for (int w = width; w > 0; w >>= 1) {  // an interval of w halves to w / 2 at most
+#pragma unroll
+            for (int u = 0; u < kRankWidth; ++u) q[u] = seg[from[u] + min((lo[u] + hi[u]) >> 1, max(have[u] - 1, 0))];
+#pragma unroll
+            for (int u = 0; u < kRankWidth; ++u) {
+                const int mid = (lo[u] + hi[u]) >> 1;
+                const bool up = lo[u] < hi[u] && comes_before(q[u], k, earlier[u]);
+                hi[u] = up ? hi[u] : mid;
+                lo[u] = up ? mid + 1 : lo[u];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kRankWidth; ++u) to += lo[u];
+    }
+    if (e < len) {
+        const int32_t v = vin[ck.x + e];
+        kout[to] = k;
+        vout[to] = v;
+        if (inv) inv[v] = to;
+    }
+}
+
 // The chunk sort into whichever buffers make the last pass end in keys_out / perm_out, then the passes.
 template <bool BODIES>
 static void sort_pairs(const SortSource &src, const SortSegs &g, uint64_t *keys_out, int32_t *perm_out, uint64_t *tmp_k,
@@ -266,6 +365,12 @@ static void sort_pairs(const SortSource &src, const SortSegs &g, uint64_t *keys_
     if (g.n <= 0) return;
     int passes = 0;
     while (((int64_t)kSortChunk << passes) < g.longest) ++passes;
+    if (passes > 0 && g.longest <= kRankChunks * kSortChunk && g.n <= kRankPairs) {
+        chunk_sort_kernel<BODIES><<<g.nchunks, kChunkThreads, 0, s>>>(src, g.chunks, g.n, tmp_k, tmp_v, nullptr);
+        rank_merge_kernel<<<g.nchunks * (kSortChunk / kRankThreads), kRankThreads, 0, s>>>(tmp_k, tmp_v, g.chunks, g.n,
+                                                                                        keys_out, perm_out, inv_out);
+        return;
+    }
     uint64_t *k = passes % 2 ? tmp_k : keys_out, *k2 = passes % 2 ? keys_out : tmp_k;
     int32_t *v = passes % 2 ? tmp_v : perm_out, *v2 = passes % 2 ? perm_out : tmp_v;
     chunk_sort_kernel<BODIES><<<g.nchunks, kChunkThreads, 0, s>>>(src, g.chunks, g.n, k, v, passes ? nullptr : inv_out);

@@ -56,24 +56,6 @@ __device__ inline int seg_of_sample(const Segs &g, int k)
 
 __device__ inline uint64_t prefix_of(uint64_t key, int L) { return key >> (63 - 3 * L); }
 
-// One step of a search for the first index in [lo, hi) where a predicate that
-// holds up to it fails: three probes, a quarter of the range left.  Searches over
-// sorted keys are chains of dependent loads (an L2 round trip each), so halving the
-// steps is worth the two extra loads.
-struct Quarter {
-    int m[3];
-};
-__device__ inline Quarter quarter_probes(int lo, int hi)
-{
-    const int len = hi - lo;
-    return Quarter{{lo + (len >> 2), lo + (len >> 1), lo + (int)((3 * (int64_t)len) >> 2)}};
-}
-__device__ inline void quarter_step(int &lo, int &hi, const Quarter &q, bool p0, bool p1, bool p2)
-{
-    const int l = p2 ? q.m[2] + 1 : p1 ? q.m[1] + 1 : p0 ? q.m[0] + 1 : lo;
-    hi = !p0 ? q.m[0] : !p1 ? q.m[1] : !p2 ? q.m[2] : hi;
-    lo = l;
-}
 // The run [a, b) of keys around position q of [lo, hi) that share its first L digits,
 // both ends searched at once.
 __device__ inline void prefix_run(const uint64_t *k, int lo, int q, int hi, int L, int &a, int &b)

@@ -110,6 +110,25 @@ __device__ inline uint32_t block_exclusive_scan(uint32_t v, uint32_t *sh, uint32
     return pre + x - v;
 }
 
+// One step of a search for the first index in [lo, hi) where a predicate that
+// holds up to it fails: three probes, a quarter of the range left.  Searches over
+// sorted keys are chains of dependent loads (an L2 round trip each), so halving the
+// steps is worth the two extra loads.
+struct Quarter {
+    int m[3];
+};
+__device__ inline Quarter quarter_probes(int lo, int hi)
+{
+    const int len = hi - lo;
+    return Quarter{{lo + (len >> 2), lo + (len >> 1), lo + (int)((3 * (int64_t)len) >> 2)}};
+}
+__device__ inline void quarter_step(int &lo, int &hi, const Quarter &q, bool p0, bool p1, bool p2)
+{
+    const int l = p2 ? q.m[2] + 1 : p1 ? q.m[1] + 1 : p0 ? q.m[0] + 1 : lo;
+    hi = !p0 ? q.m[0] : !p1 ? q.m[1] : !p2 ? q.m[2] : hi;
+    lo = l;
+}
+
 // Exclusive scan of `total` uint32 in place by one workgroup of 1024 threads, 16,384
 // entries a pass, the passes chained by a carry.  One CU's rate of lines touched
 // bounds it: a wave's 1,024 entries lie in four rows of 256, four entries a lane, so
