@@ -59,7 +59,8 @@ __device__ inline float wave_max(float v)
 // each such release writes back the XCD's L2.)
 
 // min x, max x, min y, max y, min z, max z of the workgroup, in v on thread 0.
-__device__ inline void block_extremes(float (&v)[6], float (*red)[4])
+template <int W>
+__device__ inline void block_extremes(float (&v)[6], float (*red)[W])
 {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
 #pragma unroll
@@ -108,18 +109,38 @@ __device__ inline bool fold_extremes(const float *__restrict__ x, const float *_
     return bad;
 }
 
-__global__ void __launch_bounds__(256) bbox_kernel(const float *__restrict__ x, const float *__restrict__ y,
-                                                   const float *__restrict__ z, int n, float *__restrict__ part,
-                                                   DeviceState *st)
+// The extremes v to the outputs, and the FP64 extent to the state.
+__device__ inline void store_extent(const float (&v)[6], DeviceState *st, float *minX, float *maxX, float *minY,
+                                    float *maxY, float *minZ, float *maxZ)
 {
-    __shared__ float red[6][4];
+    *minX = v[0]; *maxX = v[1]; *minY = v[2];
+    *maxY = v[3]; *minZ = v[4]; *maxZ = v[5];
+    double xs = fabs((double)v[1] - (double)v[0]);
+    double ys = fabs((double)v[3] - (double)v[2]);
+    double zs = fabs((double)v[5] - (double)v[4]);
+    double sp = xs > ys ? xs : ys;
+    sp = sp < zs ? zs : sp;
+    st->ext[0] = v[0]; st->ext[1] = v[2]; st->ext[2] = v[4]; st->ext[3] = sp;
+}
+
+// T threads; a launch of one workgroup (part == nullptr) also stores the result.
+template <int T>
+__global__ void __launch_bounds__(T) bbox_kernel(const float *__restrict__ x, const float *__restrict__ y,
+                                                 const float *__restrict__ z, int n, float *__restrict__ part,
+                                                 DeviceState *st, float *minX, float *maxX, float *minY, float *maxY,
+                                                 float *minZ, float *maxZ)
+{
+    __shared__ float red[6][T / 64];
     const int tid = threadIdx.x;
     float v[6] = {INFINITY, -INFINITY, INFINITY, -INFINITY, INFINITY, -INFINITY};
     const bool bad = fold_extremes(x, y, z, blockIdx.x * blockDim.x + tid, n, blockDim.x * gridDim.x, v);
     if (__ballot(bad) && (tid & 63) == 0) atomicOr(&st->err, kErrNonFinite);
     block_extremes(v, red);
-    if (tid == 0)
+    if (tid) return;
+    if (part)
         for (int k = 0; k < 6; ++k) part[6 * blockIdx.x + k] = v[k];
+    else
+        store_extent(v, st, minX, maxX, minY, maxY, minZ, maxZ);
 }
 
 __global__ void __launch_bounds__(256) bbox_fold_kernel(const float *__restrict__ part, int nparts, DeviceState *st,
@@ -136,16 +157,7 @@ __global__ void __launch_bounds__(256) bbox_fold_kernel(const float *__restrict_
         }
     }
     block_extremes(v, red);
-    if (threadIdx.x == 0) {
-        *minX = v[0]; *maxX = v[1]; *minY = v[2];
-        *maxY = v[3]; *minZ = v[4]; *maxZ = v[5];
-        double xs = fabs((double)v[1] - (double)v[0]);
-        double ys = fabs((double)v[3] - (double)v[2]);
-        double zs = fabs((double)v[5] - (double)v[4]);
-        double sp = xs > ys ? xs : ys;
-        sp = sp < zs ? zs : sp;
-        st->ext[0] = v[0]; st->ext[1] = v[2]; st->ext[2] = v[4]; st->ext[3] = sp;
-    }
+    if (threadIdx.x == 0) store_extent(v, st, minX, maxX, minY, maxY, minZ, maxZ);
 }
 
 // Keys of nbx_compute_keys (the build makes its own in the sort's first launch).
@@ -322,12 +334,19 @@ void launch_reset(nbx_context *c, hipStream_t s, int *mutex, float *x, float *y,
                                                             c->st);
 }
 
+// Up to this many bodies one workgroup folds them all (eight a thread, two rounds of loads).
+constexpr int kBoxOneGroup = 8192;
+
 void launch_bbox(nbx_context *c, hipStream_t s, const float *x, const float *y, const float *z,
                  float *minX, float *maxX, float *minY, float *maxY, float *minZ, float *maxZ, int n)
 {
+    if (n <= kBoxOneGroup) {
+        bbox_kernel<1024><<<1, 1024, 0, s>>>(x, y, z, n, nullptr, c->st, minX, maxX, minY, maxY, minZ, maxZ);
+        return;
+    }
     const int block = 256;
     int g = grid_for(n, block * 8, c->bbox_blocks);
-    bbox_kernel<<<g, block, 0, s>>>(x, y, z, n, c->bbox_part, c->st);
+    bbox_kernel<256><<<g, block, 0, s>>>(x, y, z, n, c->bbox_part, c->st, minX, maxX, minY, maxY, minZ, maxZ);
     bbox_fold_kernel<<<1, block, 0, s>>>(c->bbox_part, g, c->st, minX, maxX, minY, maxY, minZ, maxZ);
 }
 

@@ -206,23 +206,39 @@ __device__ inline int order_state(const OrderTables &o, uint64_t key, int state,
 // side, not one after another).  Thread 0 also sets *index past the top cells.
 // Every child's place in the group order is left relative to its parent's: {offset,
 // the parent's number among the top cells}, or {place, -1} under a root.
+//
+// SCAN: up to kWireScan entries, which every workgroup numbers for itself (workgroup 0
+// also stores the numbers, id[]); otherwise id[] holds the scanned flags.  At 2,000
+// and 32,768 bodies this adds 1.0 to 1.5 us and saves a launch of 4; at 150,001 (3,087
+// entries) it added 3.6.
+constexpr int kWireScan = 2048;
+template <bool SCAN>
 __global__ void __launch_bounds__(256) top_wire_kernel(
     Segs g, int nsamples, const uint64_t *__restrict__ skeys, const int32_t *__restrict__ perm, int *child,
-    int32_t *__restrict__ cell_level, const uint32_t *__restrict__ flag, const uint32_t *__restrict__ id,
+    int32_t *__restrict__ cell_level, const uint32_t *__restrict__ flag, uint32_t *__restrict__ id,
     const int32_t *__restrict__ ta, const int32_t *__restrict__ tb, int4 *__restrict__ sub, int sub_max,
     int base0, int m, int *index, int *__restrict__ start, int2 *__restrict__ top_place,
     int2 *__restrict__ sub_place, DeviceState *st)
 {
     __shared__ OrderTables tab;
+    __shared__ uint32_t s_id[SCAN ? kWireScan : 1], s_sum[4];
+    __shared__ int s_stop;
     order_tables_fill(tab);
+    if (threadIdx.x == 0) s_stop = latched(st);  // one read: this launch raises the latch itself
     __syncthreads();
-    if (latched(st)) return;
+    if (s_stop) return;
     const int total = nsamples * kLevels;
+    if (SCAN) {
+        scan_to_lds<kWireScan / 1024>(flag, total, s_id, s_sum);
+        if (blockIdx.x == 0)
+            for (int k = threadIdx.x; k < total; k += 256) id[k] = s_id[k];
+    }
+    const auto number = [&](int e) { return (int)(SCAN ? s_id[e] : id[e]); };
     const int gt = blockIdx.x * blockDim.x + threadIdx.x;
     const int t = gt >> 3;  // entry: one (level, sample) of the top table, or one root
     const int d = gt & 7;   // digit, slot
     if (gt == 0) {
-        const int ntop = (int)(id[total - 1] + flag[total - 1]);
+        const int ntop = number(total - 1) + (int)flag[total - 1];
         st->ntop = ntop;
         *index = base0 + ntop;
         if ((int64_t)base0 + ntop > m) atomicOr(&st->err, kErrCapacity);
@@ -232,7 +248,7 @@ __global__ void __launch_bounds__(256) top_wire_kernel(
         if (!flag[t]) return;
         L = t / nsamples;
         const int k = t - L * nsamples;
-        c = base0 + (int)id[t];
+        c = base0 + number(t);
         a = ta[t];
         b = tb[t];
         s = seg_of_sample(g, k);
@@ -268,7 +284,7 @@ __global__ void __launch_bounds__(256) top_wire_kernel(
         const int w = __shfl(cnt, o, 8);
         below += ((int)(dig >> (4 * o)) & 7) < ((int)(dig >> (4 * d)) & 7) ? w : 0;
     }
-    const int2 place = t < total ? make_int2(below, (int)id[t]) : make_int2(a + below, -1);
+    const int2 place = t < total ? make_int2(below, number(t)) : make_int2(a + below, -1);
     const int64_t slot = 8 * (int64_t)c + d;
     if (cnt == 0) {
         child[slot] = -1;
@@ -276,7 +292,7 @@ __global__ void __launch_bounds__(256) top_wire_kernel(
         child[slot] = perm[da];
     } else if (cnt > kSubtreeMax) {
         const int kk = samp_lo(g, s) + (da - lo + kSubtreeMax - 1) / kSubtreeMax;
-        const int tc = (int)id[(L + 1) * nsamples + kk];
+        const int tc = number((L + 1) * nsamples + kk);
         child[slot] = base0 + tc;
         top_place[tc] = place;
     } else {
@@ -566,16 +582,16 @@ __device__ inline int shared_digits(uint64_t a, uint64_t b)  // of two keys, 21 
     return x == 0 ? kKeyLevels : (__clzll((long long)x) - 1) / 3;
 }
 
-template <int T, int POOL, int BELOW>
+template <int T, int POOL, int BELOW, bool SCAN>
 __global__ void __launch_bounds__(T, 6) subtree_build_kernel(
     int m, const uint64_t *__restrict__ skeys, const int32_t *__restrict__ perm, int *__restrict__ child, int base0,
     const uint32_t *__restrict__ cbase, int32_t *__restrict__ cell_level, int *__restrict__ start,
-    const int4 *__restrict__ sub, int sub_max, int4 *__restrict__ subcells, DeviceState *st)
+    const int4 *__restrict__ sub, int sub_max, int4 *__restrict__ subcells, int *__restrict__ index, DeviceState *st)
 {
     constexpr bool REST = POOL == kBuildPool;
     constexpr int C = 4, W = T / 64;  // bodies per thread at most; waves
     static_assert(!REST || (C * T >= kSubtreeMax && build_bytes(0, kSubtreeMax) <= POOL), "the keys fit without the slots");
-    __shared__ int s_stop, s_cnt[C][W], s_deep[W];
+    __shared__ int s_stop, s_cnt[C][W], s_deep[W], s_sum[W];
     __shared__ __align__(16) unsigned char s_pool[POOL];
     if (threadIdx.x == 0) s_stop = latched(st);  // one read: this launch raises the latch itself
     __syncthreads();
@@ -583,10 +599,29 @@ __global__ void __launch_bounds__(T, 6) subtree_build_kernel(
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nsub = min(__hip_atomic_load(&st->nsub, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), sub_max);
     const int top = base0 + __hip_atomic_load(&st->ntop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    // SCAN: the cells of the subtrees [0, to), summed by the workgroup from the counts
+    const auto cells_before = [&](int to) {
+        int c = 0;
+        for (int j = tid; j < to; j += T) c += (int)cbase[j];
+        for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
+        if (lane == 0) s_sum[wave] = c;
+        __syncthreads();
+        c = 0;
+        for (int w = 0; w < W; ++w) c += s_sum[w];
+        __syncthreads();
+        return c;
+    };
+    if (SCAN && blockIdx.x == 0) {
+        const int64_t end = (int64_t)top + cells_before(nsub);
+        if (tid == 0) {
+            if (end > m) atomicOr(&st->err, kErrCapacity);
+            else *index = (int)end;
+        }
+    }
     for (int job = blockIdx.x; job < nsub; job += gridDim.x) {
         const int4 jb = sub[job];
-        const uint32_t cb0 = cbase[job], cb1 = cbase[job + 1];
-        const int base = top + (int)cb0, ks = (int)(cb1 - cb0);  // ids reserved by subtree_base_kernel
+        const uint32_t cb0 = SCAN ? cells_before(job) : cbase[job], cb1 = SCAN ? cb0 + cbase[job] : cbase[job + 1];
+        const int base = top + (int)cb0, ks = (int)(cb1 - cb0);  // the subtree's own ids
         const int a = jb.x, cnt = jb.y - jb.x, L0 = jb.z, slot = jb.w;
         const bool fits = ks >= 0 && ks < 65536 && cnt <= C * T && build_bytes(ks, cnt) <= POOL;
         if (fits ? BELOW > 0 && cnt <= 4 * kBuildSmallT && build_bytes(ks, cnt) <= BELOW : !REST) continue;
@@ -1257,16 +1292,27 @@ struct SysInfo {
     const double *ext;
 };
 
-template <bool BATCH>
+// SCAN: up to kLayoutRuns runs, whose totals (brun) every workgroup scans for itself
+// (workgroup 0 also stores the sums, bsum[]); otherwise bsum[] holds the scanned totals.
+// 0.6 us more at 2,000 and 32,768 bodies for a launch of 3.7; 2.4 more at 150,001.
+constexpr int kLayoutRuns = 96;
+template <bool BATCH, bool SCAN>
 __global__ void __launch_bounds__(256) frame_layout_kernel(
     int n, int nroot, const int *__restrict__ index, const int *__restrict__ child, const int32_t *__restrict__ pos,
     const int32_t *__restrict__ cell_level, const int *__restrict__ count, const int *__restrict__ start,
     const float4 *__restrict__ nodes4, float4 *__restrict__ fnode, int2 *__restrict__ fmeta,
-    const uint32_t *__restrict__ boff, const uint32_t *__restrict__ bsum, float4 *__restrict__ froot4,
-    int2 *__restrict__ frootm, int32_t *__restrict__ pblk, int32_t *__restrict__ bpar, float theta, float eps2,
-    SysInfo si, const DeviceState *st)
+    const uint32_t *__restrict__ boff, const uint32_t *__restrict__ brun, int runs, uint32_t *gsum,
+    float4 *__restrict__ froot4, int2 *__restrict__ frootm, int32_t *__restrict__ pblk, int32_t *__restrict__ bpar,
+    float theta, float eps2, SysInfo si, const DeviceState *st)
 {
-    if (latched(st)) return;
+    __shared__ uint32_t s_run[SCAN ? kLayoutRuns : 1], s_sum[4];
+    if (latched(st)) return;  // one value for the whole launch: nothing in it raises the latch
+    if (SCAN) {
+        scan_to_lds<1>(brun, runs, s_run, s_sum);
+        if (blockIdx.x == 0)
+            for (int k = threadIdx.x; k < runs; k += 256) gsum[k] = s_run[k];
+    }
+    const uint32_t *bsum = SCAN ? s_run : gsum;
     const int ncell = *index - n;
     const int64_t items = BATCH ? ncell : ncell + 1;
     const int64_t total = 8 * items;
@@ -1479,6 +1525,12 @@ static int job_grid(int nbodies)
 // 7.5M bodies in 512 systems; build: 30 and 37, 89 and 88, 207 and 177.
 constexpr int kSumTwoPools = 1 << 21, kBuildTwoPools = 1 << 22;
 
+// Up to this many bodies (some 250 subtrees) every workgroup of the build adds up the
+// cells of the subtrees before its own, instead of a launch that scans the counts: nothing
+// to 0.5 us more at 2,000 and 32,768 bodies for a launch of 3.9, 3.8 us more at 150,001 and
+// 4.3 for an ensemble of 96 systems with 100,000.
+constexpr int kBuildScan = 1 << 16;
+
 static void build_tree(Segs g, int nsamples, int base0, int m, TreeScratch &ts, DeviceState *st, hipStream_t s,
                        int n, const uint64_t *skeys, const int32_t *perm, const uint64_t *keys,
                        const int32_t *pos, const float4 *bodies4, float4 *nodes4, int *child, int *index,
@@ -1487,27 +1539,37 @@ static void build_tree(Segs g, int nsamples, int base0, int m, TreeScratch &ts, 
     const int tb = (32 * nsamples + 255) / 256;
     after_sort_kernel<<<tb + capped_grid(n), 256, 0, s>>>(g, nsamples, tb, skeys, ts.top_flag, ts.top_id, ts.top_a,
                                                           ts.top_b, ts.lcp, pos, bodies4, nodes4, st);
-    launch_exclusive_scan_u32(ts.top_id, nsamples * kLevels, ts.scan_tmp, s);
     const int wire = nsamples * kLevels + g.nseg;  // entries, 8 lanes each
-    top_wire_kernel<<<(8 * wire + 255) / 256, 256, 0, s>>>(g, nsamples, skeys, perm, child, cell_level, ts.top_flag,
-                                                        ts.top_id, ts.top_a, ts.top_b, ts.sub, ts.sub_max,
-                                                        base0, m, index, start, ts.top_place, ts.sub_place, st);
+    const auto wire_with = [&](auto kernel) {
+        kernel<<<(8 * wire + 255) / 256, 256, 0, s>>>(g, nsamples, skeys, perm, child, cell_level, ts.top_flag, ts.top_id,
+                                                      ts.top_a, ts.top_b, ts.sub, ts.sub_max, base0, m, index, start,
+                                                      ts.top_place, ts.sub_place, st);
+    };
+    if (nsamples * kLevels <= kWireScan) {
+        wire_with(top_wire_kernel<true>);
+    } else {
+        launch_exclusive_scan_u32(ts.top_id, nsamples * kLevels, ts.scan_tmp, s);
+        wire_with(top_wire_kernel<false>);
+    }
     subtree_cells_kernel<<<capped_grid(64 * (int64_t)ts.sub_max, 4096), 256, 0, s>>>(ts.sub, ts.sub_max, ts.lcp,
                                                                                      ts.cbase, st);
-    subtree_base_kernel<<<1, 1024, 0, s>>>(ts.cbase, ts.sub_max, base0, m, index, st);
-    if (locked)
-        subtree_insert_kernel<<<job_grid(g.n), 256, 0, s>>>(n, m, skeys, perm, keys, ts.lcp, child, base0,
-                                                                ts.cbase, cell_level, ts.sub, ts.sub_max,
-                                                                ts.subcells, st);
-    else if (g.n < kBuildTwoPools) {
-        subtree_build_kernel<256, kBuildPool, 0><<<job_grid(g.n), 256, 0, s>>>(m, skeys, perm, child, base0, ts.cbase, cell_level,
-                                                                         start, ts.sub, ts.sub_max, ts.subcells, st);
+    const bool scan = !locked && g.n <= kBuildScan;
+    if (!scan) subtree_base_kernel<<<1, 1024, 0, s>>>(ts.cbase, ts.sub_max, base0, m, index, st);
+    const int jobs = job_grid(g.n);
+    const auto build_with = [&](auto kernel, int threads) {
+        kernel<<<jobs, threads, 0, s>>>(m, skeys, perm, child, base0, ts.cbase, cell_level, start, ts.sub, ts.sub_max,
+                                        ts.subcells, index, st);
+    };
+    if (locked) {
+        subtree_insert_kernel<<<jobs, 256, 0, s>>>(n, m, skeys, perm, keys, ts.lcp, child, base0, ts.cbase, cell_level,
+                                                   ts.sub, ts.sub_max, ts.subcells, st);
+    } else if (scan) {
+        build_with(subtree_build_kernel<256, kBuildPool, 0, true>, 256);
+    } else if (g.n < kBuildTwoPools) {
+        build_with(subtree_build_kernel<256, kBuildPool, 0, false>, 256);
     } else {
-        subtree_build_kernel<256, kBuildPool, kBuildSmall><<<job_grid(g.n), 256, 0, s>>>(m, skeys, perm, child, base0, ts.cbase,
-                                                                         cell_level, start, ts.sub, ts.sub_max,
-                                                                         ts.subcells, st);
-        subtree_build_kernel<kBuildSmallT, kBuildSmall, 0><<<job_grid(g.n), kBuildSmallT, 0, s>>>(m, skeys, perm, child, base0, ts.cbase, cell_level,
-                                                                         start, ts.sub, ts.sub_max, ts.subcells, st);
+        build_with(subtree_build_kernel<256, kBuildPool, kBuildSmall, false>, 256);
+        build_with(subtree_build_kernel<kBuildSmallT, kBuildSmall, 0, false>, kBuildSmallT);
     }
 }
 
@@ -1599,15 +1661,29 @@ void launch_layout(nbx_context *c, hipStream_t s, int *sorted)
     launch_frame_layout(c, s);
 }
 
+// Blocks' children, their runs' totals scanned, then the records.  items: blocks at most.
+template <bool BATCH, class... Out>
+static void lay_out(hipStream_t s, int64_t items, int n, int nroot, const int *index, const int *child, const int32_t *pos,
+                    const int32_t *cell_level, const int *count, const int *start, const float4 *nodes4, float4 *fnode,
+                    int2 *fmeta, uint32_t *boff, uint32_t *bsum, uint32_t *brun, DeviceState *st, Out... out)
+{
+    const int runs = (int)((items + kOffRun - 1) / kOffRun);
+    const bool scan = runs <= kLayoutRuns;
+    frame_count_kernel<BATCH><<<runs, 256, 0, s>>>(n, index, child, boff, scan ? brun : bsum, st);
+    if (!scan) launch_scan_one_block(bsum, runs, s);
+    const auto with = [&](auto kernel) {
+        kernel<<<capped_grid(8 * items), 256, 0, s>>>(n, nroot, index, child, pos, cell_level, count, start, nodes4, fnode,
+                                                      fmeta, boff, brun, runs, bsum, out..., st);
+    };
+    if (scan) with(frame_layout_kernel<BATCH, true>);
+    else with(frame_layout_kernel<BATCH, false>);
+}
+
 void launch_frame_layout(nbx_context *c, hipStream_t s)
 {
-    SysInfo si{};
-    const int runs = (int)(((int64_t)c->m - c->n + 1 + kOffRun - 1) / kOffRun);
-    frame_count_kernel<false><<<runs, 256, 0, s>>>(c->n, c->index, c->child, c->boff, c->bsum, c->st);
-    launch_scan_one_block(c->bsum, runs, s);
-    frame_layout_kernel<false><<<capped_grid(8 * (int64_t)(c->m - c->n + 1)), 256, 0, s>>>(
-        c->n, 1, c->index, c->child, c->pos, c->cell_level, c->count, c->start, c->nodes4, c->fnode, c->fmeta, c->boff,
-        c->bsum, c->froot4, c->frootm, c->pblk, c->bpar, c->p.theta, layout_eps2(c->p), si, c->st);
+    lay_out<false>(s, (int64_t)c->m - c->n + 1, c->n, 1, c->index, c->child, c->pos, c->cell_level, c->count, c->start,
+                   c->nodes4, c->fnode, c->fmeta, c->boff, c->bsum, c->brun, c->st, c->froot4, c->frootm, c->pblk, c->bpar,
+                   c->p.theta, layout_eps2(c->p), SysInfo{});
     c->layout_theta = c->p.theta;
     c->layout_eps2 = layout_eps2(c->p);
 }
@@ -1632,13 +1708,9 @@ void launch_batch_layout(nbx_batch *b, hipStream_t s)
     Segs g{b->off, b->samp_off, b->S, b->N, 1};
     order_bodies(g, b->N + b->S, b->ts, b->st, s, b->skeys, b->child, b->count, b->start, b->cell_level, b->pblk,
                  b->perm, b->sorted, b->gorder);
-    SysInfo si{b->sys_of, b->theta, b->ext};
-    const int runs = (int)(((int64_t)b->m - b->N + kOffRun - 1) / kOffRun);
-    frame_count_kernel<true><<<runs, 256, 0, s>>>(b->N, b->index, b->child, b->boff, b->bsum, b->st);
-    launch_scan_one_block(b->bsum, runs, s);
-    frame_layout_kernel<true><<<capped_grid(8 * (int64_t)(b->m - b->N)), 256, 0, s>>>(
-        b->N, b->S, b->index, b->child, b->pos, b->cell_level, b->count, b->start, b->nodes4, b->fnode, b->fmeta, b->boff,
-        b->bsum, b->froot4, b->frootm, b->pblk, b->bpar, 0.f, layout_eps2(b->p), si, b->st);
+    lay_out<true>(s, (int64_t)b->m - b->N, b->N, b->S, b->index, b->child, b->pos, b->cell_level, b->count, b->start,
+                  b->nodes4, b->fnode, b->fmeta, b->boff, b->bsum, b->brun, b->st, b->froot4, b->frootm, b->pblk, b->bpar,
+                  0.f, layout_eps2(b->p), SysInfo{b->sys_of, b->theta, b->ext});
 }
 
 }  // namespace nbx

@@ -200,6 +200,40 @@ __device__ inline uint32_t scan_in_place(uint32_t *data, int total, uint32_t *sh
     return carry;
 }
 
+// Exclusive scan of src[0, total) into LDS by a workgroup of 256 threads, total <= 1024 V;
+// sh: 4 words.  Ends with a barrier; returns the total.  For arrays of a few thousand
+// entries that every workgroup of a launch scans for itself: 1 to 2 us, where a scan launched
+// before it costs 4 to 5.
+template <int V>
+__device__ inline uint32_t scan_to_lds(const uint32_t *__restrict__ src, int total, uint32_t *dst, uint32_t *sh)
+{
+    uint32_t v[V][4];
+    const int tid = threadIdx.x;
+#pragma unroll
+    for (int u = 0; u < V; ++u)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int k = 1024 * u + 4 * tid + i;
+            v[u][i] = k < total ? src[k] : 0u;
+        }
+    uint32_t carry = 0;
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+        if (1024 * u >= total) break;
+        uint32_t tot;
+        uint32_t ex = carry + block_exclusive_scan(v[u][0] + v[u][1] + v[u][2] + v[u][3], sh, &tot);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int k = 1024 * u + 4 * tid + i;
+            if (k < total) dst[k] = ex;
+            ex += v[u][i];
+        }
+        carry += tot;
+    }
+    __syncthreads();
+    return carry;
+}
+
 // First record of frame block b in the packed layout: the sum within its run of
 // kOffRun blocks plus the records of the runs before it.
 __device__ inline int frame_off(const uint32_t *__restrict__ boff, const uint32_t *__restrict__ bsum, int b)

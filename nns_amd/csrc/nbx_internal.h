@@ -138,6 +138,7 @@ struct nbx_context {
     int2 *fmeta = nullptr;       // [m_max + 8] child descriptors
     uint32_t *boff = nullptr;    // [m_max + 1] record offset of each block within its run of kOffRun
     uint32_t *bsum = nullptr;    // [m_max / kOffRun + 1] records before each run
+    uint32_t *brun = nullptr;    // [m_max / kOffRun + 1] records of each run
     float4 *froot4 = nullptr;    // root as a child of a virtual parent
     int2 *frootm = nullptr;
     int32_t *pblk = nullptr;     // [m_max] parent block of each block (-1: root)
@@ -221,6 +222,7 @@ struct nbx_batch {
     int2 *fmeta = nullptr;
     uint32_t *boff = nullptr;    // [M] record offset of each block within its run of kOffRun
     uint32_t *bsum = nullptr;    // [M / kOffRun + 1] records before each run
+    uint32_t *brun = nullptr;    // [M / kOffRun + 1] records of each run
     float4 *froot4 = nullptr;    // [S] roots
     int2 *frootm = nullptr;
     int32_t *pblk = nullptr, *bpar = nullptr;
