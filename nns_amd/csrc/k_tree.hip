@@ -867,6 +867,15 @@ __device__ inline void store_cell(const SumOut &o, int c, const CellSum &r, Devi
     o.nodes4[c] = make_float4(fx, fy, fz, fm);
 }
 
+// The single system's root, from its mass and moments.
+__device__ inline void store_root(double ms, double mx, double my, double mz, int cnt, DeviceState *st)
+{
+    if (cnt > 0 && !(ms > 0.0)) atomicOr(&st->err, kErrNonFinite);
+    const double gx = mx / ms, gy = my / ms, gz = mz / ms;
+    st->root64[0] = ms; st->root64[1] = gx; st->root64[2] = gy; st->root64[3] = gz;
+    st->root4 = make_float4((float)gx, (float)gy, (float)gz, (float)ms);
+}
+
 // lev: the cell's level when the caller has it (else -1).
 // B: slots whose loads go together; CURSOR: o.cursor (sum_cell).
 template <int B, bool CURSOR>
@@ -881,10 +890,7 @@ __device__ inline void summarise(const SumOut &o, int c, DeviceState *st, bool s
         store_cell(o, c, r, st);
         return;
     }
-    if (r.cnt > 0 && !(r.ms > 0.0)) atomicOr(&st->err, kErrNonFinite);
-    const double gx = r.mx / r.ms, gy = r.my / r.ms, gz = r.mz / r.ms;
-    st->root64[0] = r.ms; st->root64[1] = gx; st->root64[2] = gy; st->root64[3] = gz;
-    st->root4 = make_float4((float)gx, (float)gy, (float)gz, (float)r.ms);
+    store_root(r.ms, r.mx, r.my, r.mz, r.cnt, st);
 }
 
 // Subtree summary: workgroup w sums subtrees w, w + gridDim.x, ...: with as many
@@ -1061,31 +1067,31 @@ __global__ void __launch_bounds__(T, POOL == kSumSmall ? 8 : 4) subtree_summary_
 }
 
 // Top summary: the top cells level by level, deepest first, then the roots.  A
-// level's cells read only the level below.  A cell's sum gathers from up to 8
+// level's cells read only the levels below.  A cell's sum gathers from up to 8
 // children in unrelated cache lines, and one CU's address pipeline takes such
-// gathers a few lanes at a time, so a level of more than kTopNarrow cells is
-// spread over kTopBlocks workgroups (its cell i to workgroup i mod kTopBlocks)
-// that meet at a grid barrier after it; the narrower levels above it (a top cell's
-// parent is a top cell: a level never has more cells than the one below) and
-// the roots are summed by workgroup 0 alone, with workgroup barriers.
-// kTopBlocks workgroups of 256 threads fit on the device at once, so every
+// gathers a few lanes at a time, so while more than kTopItems - 64 cells are left, a
+// level is spread over kTopBlocks workgroups (its cell i to workgroup i mod kTopBlocks)
+// that meet at a grid barrier after it; the levels that are then left are summed by
+// workgroup 0 alone, in LDS.
+// kTopBlocks workgroups of 512 threads fit on the device at once, so every
 // workgroup reaches every barrier; the wait is bounded all the same: one that
 // runs out latches kErrStall, and every wave still finishes.
 constexpr int kTopBlocks = 64;
-constexpr int kTopNarrow = 64;
 constexpr int kTopSpin = 1 << 20;  // polls of one barrier wait (about a second)
 
-// Grid barrier number `phase` (1, 2, ...) of the launch.  Every thread makes its
-// stores visible device-wide (release), thread 0 arrives and waits until every
-// workgroup has, and every thread then acquires what they wrote.
+// Grid barrier number `phase` (1, 2, ...) of the launch.  Every wave waits until its
+// stores have reached the XCD's L2; thread 0 then makes them visible device-wide with its
+// arrival (one write-back of the L2, not one per wave), waits until every workgroup has
+// arrived, and acquires what they wrote for the whole CU.
 __device__ inline void top_barrier(DeviceState *st, int phase, bool &stalled)
 {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
     if (threadIdx.x == 0) {
         const int target = phase * (int)gridDim.x;
         __hip_atomic_fetch_add(&st->tsync, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-        for (int k = 0; !stalled && __hip_atomic_load(&st->tsync, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT) < target;
+        for (int k = 0; !stalled && __hip_atomic_load(&st->tsync, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target;
              ++k) {
             if (k == kTopSpin) {
                 atomicOr(&st->err, kErrStall);
@@ -1093,17 +1099,114 @@ __device__ inline void top_barrier(DeviceState *st, int phase, bool &stalled)
             }
             __builtin_amdgcn_s_sleep(2);
         }
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
     }
     __syncthreads();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+}
+
+// Few top cells and roots (items): all in the LDS of one workgroup.  The sums of
+// every item's children have their places there: those of subtrees and bodies are loaded up
+// front, all side by side, and an item that is summed puts its own into its parent's.
+// Eight lanes per item, of which four add one component each, in slot order.
+// (Level by level in memory, with four times as many write-backs of the L2 at a barrier:
+// 150,001 bodies 23 us, now 10; 1M: 49 and 23; 4M: 48 and 32; 7.5M in 512 systems: 100
+// and 76.)
+constexpr int kTopThreads = 512;
+constexpr int kTopItems = 448;
+struct TopLds {
+    double4 slot[8 * kTopItems];  // sums of the children
+    double4 rec[kTopItems];       // sums of the items
+    int cnt[8 * kTopItems];       // bodies of the children; slot 0 then the item's
+    int place[kTopItems];         // an item's place among its parent's children
+};
+template <bool CURSOR>
+__device__ inline void top_in_lds(TopLds &t, int *first, const SumOut &o, const Segs &g, int base0, int left,
+                                  int roots, const int *first_of_level, int from,
+                                  DeviceState *st)
+{
+    const int tid = threadIdx.x, s = tid & 7, items = left + roots;
+    const auto node_of = [&](int j) { return j < left ? base0 + j : seg_root(g, j - left); };
+    for (int k0 = tid; k0 < 8 * items; k0 += 4 * kTopThreads) {
+        int q[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int k = k0 + u * kTopThreads;
+            q[u] = k < 8 * items ? o.child[8 * (int64_t)node_of(k >> 3) + s] : -1;
+        }
+        double4 v[4];
+        int c[4], f[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            v[u] = make_double4(0.0, 0.0, 0.0, 0.0);
+            c[u] = 0;
+            f[u] = 0x7fffffff;
+            if (q[u] >= o.n && (q[u] < base0 || q[u] >= base0 + left)) {
+                v[u] = o.sum64[q[u]];
+                c[u] = o.count[q[u]];
+                if (!CURSOR) f[u] = o.start[q[u]];
+            } else if (q[u] >= 0 && q[u] < o.n) {
+                const float4 b = o.bodies4[q[u]];
+                const double m = (double)b.w;
+                v[u] = make_double4(m, __dmul_rn(m, (double)b.x), __dmul_rn(m, (double)b.y), __dmul_rn(m, (double)b.z));
+                c[u] = 1;
+                if (!CURSOR) f[u] = o.pos[q[u]];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int k = k0 + u * kTopThreads;
+            if (k >= 8 * items) break;
+            if (q[u] >= base0 && q[u] < base0 + left) t.place[q[u] - base0] = k;
+            t.slot[k] = v[u];
+            t.cnt[k] = c[u];
+            if (!CURSOR) first[k] = f[u];
+        }
+    }
+    __syncthreads();
+    for (int L = from; L >= 0; --L) {
+        const int a = L ? first_of_level[L] : left, b = L ? first_of_level[L + 1] : items;
+        if (a >= b) continue;
+        for (int j = a + (tid >> 3); j < b; j += kTopThreads / 8) {
+            int n1 = t.cnt[8 * j + s], lo = CURSOR ? 0 : first[8 * j + s];
+            for (int d = 1; d < 8; d <<= 1) {
+                n1 += __shfl_xor(n1, d, 8);
+                if (!CURSOR) lo = min(lo, __shfl_xor(lo, d, 8));
+            }
+            double sum = 0.0;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) sum = __dadd_rn(sum, ((const double *)&t.slot[8 * j + k])[s & 3]);
+            const int up = j < left ? t.place[j] : -1;
+            if (s < 4) {
+                ((double *)&t.rec[j])[s] = sum;
+                if (up >= 0) ((double *)&t.slot[up])[s] = sum;
+            } else if (s == 4) {
+                t.cnt[8 * j] = n1;  // this item's lanes have read it
+                if (up >= 0) t.cnt[up] = n1;
+                if (!CURSOR) {
+                    first[8 * j] = lo;
+                    if (up >= 0) first[up] = lo;
+                }
+            }
+        }
+        __syncthreads();
+    }
+    for (int j = tid; j < items; j += kTopThreads) {
+        const double4 r = t.rec[j];
+        if (j < left || g.batch)
+            store_cell(o, node_of(j), CellSum{r.x, r.y, r.z, r.w, t.cnt[8 * j], CURSOR ? 0 : first[8 * j]}, st);
+        else
+            store_root(r.x, r.y, r.z, r.w, t.cnt[8 * j], st);
+    }
 }
 
 template <bool CURSOR>
-__global__ void __launch_bounds__(256) top_summary_kernel(SumOut o, Segs g, int base0, int nsamples,
+__global__ void __launch_bounds__(kTopThreads) top_summary_kernel(SumOut o, Segs g, int base0, int nsamples,
                                                           const uint32_t *__restrict__ top_id, DeviceState *st)
 {
     __shared__ int s_first[kLevels + 1];
     __shared__ int s_stop;
+    __shared__ TopLds s_top;
+    __shared__ int s_low[CURSOR ? 1 : 8 * kTopItems];
     const int tid = threadIdx.x;
     if (tid == 0) s_stop = latched(st);  // one read for the whole workgroup
     // The top cells of level L are the ids base0 + [s_first[L], s_first[L + 1])
@@ -1118,24 +1221,23 @@ __global__ void __launch_bounds__(256) top_summary_kernel(SumOut o, Segs g, int 
     const bool stop = s_stop != 0;
     bool stalled = false;
     int L = kKeyLevels, phase = 0;
-    for (; L >= 1; --L) {
+    for (; L >= 1 && s_first[L + 1] > kTopItems - 64; --L) {
         const int cnt = s_first[L + 1] - s_first[L];
         if (cnt <= 0) continue;  // uniform: no barrier for an empty level
-        if (cnt <= kTopNarrow) break;
         if (!stop)
             for (int i = blockIdx.x + gridDim.x * tid; i < cnt; i += gridDim.x * blockDim.x)
                 summarise<4, CURSOR>(o, base0 + s_first[L] + i, st, false, 0, L);
         top_barrier(st, ++phase, stalled);
     }
     if (blockIdx.x == 0 && !stop) {
-        for (; L >= 1; --L) {
-            const int cnt = s_first[L + 1] - s_first[L];
-            if (cnt <= 0) continue;
-            for (int i = tid; i < cnt; i += blockDim.x) summarise<4, CURSOR>(o, base0 + s_first[L] + i, st, false, 0, L);
-            __syncthreads();
-        }
-        for (int s = tid; s < g.nseg; s += blockDim.x) summarise<4, CURSOR>(o, seg_root(g, s), st, !g.batch);
+        const int left = s_first[L + 1];
+        const bool roots = left + g.nseg <= kTopItems;
+        top_in_lds<CURSOR>(s_top, s_low, o, g, base0, left, roots ? g.nseg : 0, s_first, L, st);
+        __syncthreads();
+        if (!roots)  // every top cell is summed
+            for (int s = tid; s < g.nseg; s += blockDim.x) summarise<4, CURSOR>(o, seg_root(g, s), st, !g.batch);
     }
+    if (phase == 0) return;
     if (tid == 0) {  // the last workgroup out (every other one is past its last wait) resets the barrier
         const int out = __hip_atomic_fetch_add(&st->tdone, 1, __ATOMIC_ACQ_REL, __HIP_MEMORY_SCOPE_AGENT);
         if (out == (int)gridDim.x - 1) {
@@ -1584,7 +1686,7 @@ static void summarise_tree(Segs g, int base0, int nsamples, TreeScratch &ts, Dev
         subtree_summary_kernel<CURSOR, 256, kSumPool, kSumSmall><<<grid, 256, 0, s>>>(o, ts.sub, ts.sub_max, ts.subcells, st);
         subtree_summary_kernel<CURSOR, kSumSmallT, kSumSmall, 0><<<grid, kSumSmallT, 0, s>>>(o, ts.sub, ts.sub_max, ts.subcells, st);
     }
-    top_summary_kernel<CURSOR><<<kTopBlocks, 256, 0, s>>>(o, g, base0, nsamples, ts.top_id, st);
+    top_summary_kernel<CURSOR><<<kTopBlocks, kTopThreads, 0, s>>>(o, g, base0, nsamples, ts.top_id, st);
 }
 // base0: the first top cell's id; nsamples: the top table's samples.
 static void summarise_tree(Segs g, int base0, int nsamples, TreeScratch &ts, DeviceState *st, hipStream_t s,
