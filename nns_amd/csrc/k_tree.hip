@@ -1126,6 +1126,8 @@ __device__ inline void top_in_lds(TopLds &t, int *first, const SumOut &o, const 
 {
     const int tid = threadIdx.x, s = tid & 7, items = left + roots;
     const auto node_of = [&](int j) { return j < left ? base0 + j : seg_root(g, j - left); };
+    for (int j = tid; j < left; j += kTopThreads) t.place[j] = -1;  // below a root that is not an item
+    __syncthreads();
     for (int k0 = tid; k0 < 8 * items; k0 += 4 * kTopThreads) {
         int q[4];
 #pragma unroll
