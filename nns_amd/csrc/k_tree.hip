@@ -1077,6 +1077,13 @@ __global__ void __launch_bounds__(T, POOL == kSumSmall ? 8 : 4) subtree_summary_
 // workgroup reaches every barrier; the wait is bounded all the same: one that
 // runs out latches kErrStall, and every wave still finishes.
 constexpr int kTopBlocks = 64;
+// Up to kTopOneGroup bodies there are hardly ever many more top cells than fit, and
+// one workgroup sums them all; up to kTopFew bodies in a third of the LDS.  Workgroups that
+// need most of a CU's LDS hold up the kernels of other streams: three ensembles of 96
+// systems (100,000 bodies) side by side took 3 % longer a step with 64 workgroups of
+// 145 KB, 1.6 % with one, and as long as before with one of 52 KB.
+constexpr int kTopOneGroup = 1 << 19;
+constexpr int kTopSmall = 160, kTopLarge = 448, kTopFew = 1 << 17;
 constexpr int kTopSpin = 1 << 20;  // polls of one barrier wait (about a second)
 
 // Grid barrier number `phase` (1, 2, ...) of the launch.  Every wave waits until its
@@ -1112,15 +1119,15 @@ __device__ inline void top_barrier(DeviceState *st, int phase, bool &stalled)
 // 150,001 bodies 23 us, now 10; 1M: 49 and 23; 4M: 48 and 32; 7.5M in 512 systems: 100
 // and 76.)
 constexpr int kTopThreads = 512;
-constexpr int kTopItems = 448;
+template <int ITEMS>
 struct TopLds {
-    double4 slot[8 * kTopItems];  // sums of the children
-    double4 rec[kTopItems];       // sums of the items
-    int cnt[8 * kTopItems];       // bodies of the children; slot 0 then the item's
-    int place[kTopItems];         // an item's place among its parent's children
+    double4 slot[8 * ITEMS];  // sums of the children
+    double4 rec[ITEMS];       // sums of the items
+    int cnt[8 * ITEMS];       // bodies of the children; slot 0 then the item's
+    int place[ITEMS];         // an item's place among its parent's children
 };
-template <bool CURSOR>
-__device__ inline void top_in_lds(TopLds &t, int *first, const SumOut &o, const Segs &g, int base0, int left,
+template <bool CURSOR, int ITEMS>
+__device__ inline void top_in_lds(TopLds<ITEMS> &t, int *first, const SumOut &o, const Segs &g, int base0, int left,
                                   int roots, const int *first_of_level, int from,
                                   DeviceState *st)
 {
@@ -1201,14 +1208,14 @@ __device__ inline void top_in_lds(TopLds &t, int *first, const SumOut &o, const 
     }
 }
 
-template <bool CURSOR>
+template <bool CURSOR, int ITEMS>
 __global__ void __launch_bounds__(kTopThreads) top_summary_kernel(SumOut o, Segs g, int base0, int nsamples,
                                                           const uint32_t *__restrict__ top_id, DeviceState *st)
 {
     __shared__ int s_first[kLevels + 1];
     __shared__ int s_stop;
-    __shared__ TopLds s_top;
-    __shared__ int s_low[CURSOR ? 1 : 8 * kTopItems];
+    __shared__ TopLds<ITEMS> s_top;
+    __shared__ int s_low[CURSOR ? 1 : 8 * ITEMS];
     const int tid = threadIdx.x;
     if (tid == 0) s_stop = latched(st);  // one read for the whole workgroup
     // The top cells of level L are the ids base0 + [s_first[L], s_first[L + 1])
@@ -1223,7 +1230,7 @@ __global__ void __launch_bounds__(kTopThreads) top_summary_kernel(SumOut o, Segs
     const bool stop = s_stop != 0;
     bool stalled = false;
     int L = kKeyLevels, phase = 0;
-    for (; L >= 1 && s_first[L + 1] > kTopItems - 64; --L) {
+    for (; L >= 1 && s_first[L + 1] > (ITEMS * 7) / 8; --L) {
         const int cnt = s_first[L + 1] - s_first[L];
         if (cnt <= 0) continue;  // uniform: no barrier for an empty level
         if (!stop)
@@ -1233,7 +1240,7 @@ __global__ void __launch_bounds__(kTopThreads) top_summary_kernel(SumOut o, Segs
     }
     if (blockIdx.x == 0 && !stop) {
         const int left = s_first[L + 1];
-        const bool roots = left + g.nseg <= kTopItems;
+        const bool roots = left + g.nseg <= ITEMS;
         top_in_lds<CURSOR>(s_top, s_low, o, g, base0, left, roots ? g.nseg : 0, s_first, L, st);
         __syncthreads();
         if (!roots)  // every top cell is summed
@@ -1688,7 +1695,11 @@ static void summarise_tree(Segs g, int base0, int nsamples, TreeScratch &ts, Dev
         subtree_summary_kernel<CURSOR, 256, kSumPool, kSumSmall><<<grid, 256, 0, s>>>(o, ts.sub, ts.sub_max, ts.subcells, st);
         subtree_summary_kernel<CURSOR, kSumSmallT, kSumSmall, 0><<<grid, kSumSmallT, 0, s>>>(o, ts.sub, ts.sub_max, ts.subcells, st);
     }
-    top_summary_kernel<CURSOR><<<kTopBlocks, kTopThreads, 0, s>>>(o, g, base0, nsamples, ts.top_id, st);
+    if (g.n <= kTopFew)
+        top_summary_kernel<CURSOR, kTopSmall><<<1, kTopThreads, 0, s>>>(o, g, base0, nsamples, ts.top_id, st);
+    else
+        top_summary_kernel<CURSOR, kTopLarge><<<g.n <= kTopOneGroup ? 1 : kTopBlocks, kTopThreads, 0, s>>>(
+            o, g, base0, nsamples, ts.top_id, st);
 }
 // base0: the first top cell's id; nsamples: the top table's samples.
 static void summarise_tree(Segs g, int base0, int nsamples, TreeScratch &ts, DeviceState *st, hipStream_t s,

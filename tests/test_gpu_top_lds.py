@@ -26,7 +26,7 @@ def test_top_cells_around_the_limit(oracle, kind, n, locked):
     check_tree(bh, t)
 
 
-@pytest.mark.parametrize("sizes", [[2, 3000, 40000], [1100] * 300, [30] * 449, [1500] * 460])
+@pytest.mark.parametrize("sizes", [[2, 3000, 40000], [1100] * 100, [1100] * 300, [30] * 449, [1500] * 460])
 def test_roots_of_ensembles(oracle, sizes):
     import torch
     assert torch.cuda.is_available()
