@@ -46,12 +46,17 @@ class Slots:
         bh.rebuild()
         self.tag[k] = tag
 
-    def accel(self, k: int, x, y, z, m, tag=None):
-        """Builds slot k's tree for (x, y, z, m) and returns its accelerations (new tensors)."""
+    def walk(self, k: int, x, y, z, m, tag=None):
+        """Builds slot k's tree for (x, y, z, m) and returns its accelerations (the slot's own
+        arrays, which its next walk overwrites)."""
         bh, n = self.bh[k], self.n
         self.tree(k, x, y, z, m, tag)
         bh.forces()
-        return bh.arr["ax"][:n].clone(), bh.arr["ay"][:n].clone(), bh.arr["az"][:n].clone()
+        return bh.arr["ax"][:n], bh.arr["ay"][:n], bh.arr["az"][:n]
+
+    def accel(self, k: int, x, y, z, m, tag=None):
+        """Builds slot k's tree for (x, y, z, m) and returns its accelerations (new tensors)."""
+        return tuple(a.clone() for a in self.walk(k, x, y, z, m, tag))
 
     def vjp(self, k: int, ux, uy, uz):
         """(dL/dx, dL/dy, dL/dz, dL/dm) over slot k's current tree."""
@@ -85,7 +90,7 @@ class BarnesHutAccel(torch.autograd.Function):
 
 def _step(slots: Slots, k: int, s, m, dt: float, tag=None):
     x, y, z, vx, vy, vz = s
-    ax, ay, az = slots.accel(k, x, y, z, m, tag)
+    ax, ay, az = slots.walk(k, x, y, z, m, tag)
     vx = torch.add(vx, ax, alpha=dt)
     vy = torch.add(vy, ay, alpha=dt)
     vz = torch.add(vz, az, alpha=dt)
@@ -102,13 +107,13 @@ class Rollout(torch.autograd.Function):
         ckpt = []
         run = object()  # names this rollout's trees in the slots
         for k in range(steps):
-            if k % every == 0:
-                ckpt.append(tuple(t.clone() for t in s))
+            if k % every == 0:  # a step makes new tensors; only the inputs are not our own
+                ckpt.append(tuple(t.clone() for t in s) if k == 0 else s)
             s = _step(slots, k % every, s, m, dt, (run, k))
         ctx.slots, ctx.steps, ctx.dt, ctx.every, ctx.run = slots, steps, dt, every, run
         ctx.ckpt = ckpt
         ctx.save_for_backward(m)
-        return tuple(t.clone() for t in s)
+        return s if steps > 0 else tuple(t.clone() for t in s)
 
     @staticmethod
     def backward(ctx, gx, gy, gz, gvx, gvy, gvz):
