@@ -54,6 +54,12 @@
 
 namespace nbx {
 
+// eps^2 on the lanes of a frame's mask, infinite on the others.
+static __device__ __forceinline__ float frame_eps2(uint64_t mask, float eps2)
+{
+    return __builtin_amdgcn_inverse_ballot_w64(mask) ? eps2 : INFINITY;
+}
+
 // The walk of group g by the calling wave (all 64 lanes active), with the
 // wave's LDS stack s.  The launch's other arguments come from its job record
 // jb, read when the walk starts and again when it ends (the empty asm with a
@@ -85,18 +91,27 @@ static __device__ __forceinline__ void walk_group(int g, int lane, uint4 *s, con
     int64_t cnt = 0, nsteps = 0, nframes = 0;
     int work = 1;  // child steps of the walk (the root's and every frame's children)
 
-    // One child step: every lane of `mask` meets child q with descriptor
+    // One child step: every lane of the frame meets child q with descriptor
     // {tag, crit}; returns the lanes that open it.  A body's crit is -1, so it
-    // is always taken and never opened.
-    auto step = [&](const float4 q, const int tag, const float crit, const uint64_t mask) -> uint64_t {
+    // is always taken and never opened.  e2 (frame_eps2) is eps^2 on the frame's lanes
+    // and infinite on the others, which therefore open nothing and take a monopole of
+    // zero.  (An infinite crit, theta = 0, is opened by every body; lanes past the last
+    // body then open it too, and store nothing.)  The step is bound by the issue of its
+    // instructions, scalar ones and taken branches included: without the mask's two scalar
+    // operations, and with the push (one step in six) out of the way of the others, 1M
+    // bodies 1,778 -> 1,729 us, 4M 3,741 -> 3,665, 512 systems 11,636 -> 11,334.  Blocks
+    // fetched one frame ahead into vector registers and used through row broadcasts (DPP)
+    // made it 2,099 at 1M, one body of code per number of children 1,953.
+    auto step = [&](const float4 q, const int tag, const float crit, const float e2) -> uint64_t {
         const float dx = q.x - me.x;
         const float dy = q.y - me.y;
         const float dz = q.z - me.z;
-        const float d2 = fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, eps2)));  // |d|^2 + eps^2
-        const uint64_t ok = __ballot(crit < d2);                         // crit = crit_L + eps^2
-        uint64_t takem = mask & ok;
-        const uint64_t omask = mask & ~ok;
+        const float d2 = fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, e2)));  // |d|^2 + eps^2
+        const uint64_t ok = __ballot(crit < d2);                       // crit = crit_L + eps^2
+        uint64_t takem = ok;
+        const uint64_t omask = ~ok;
         if (COUNT) {
+            takem &= __ballot(e2 < INFINITY);
             if (__builtin_amdgcn_inverse_ballot_w64(takem)) cnt += ((tag & 15) == 0 && (tag >> 4) == p) ? 0 : 1;
         }
         if (!SOFT) takem &= __ballot(d2 > 0.f);
@@ -126,7 +141,7 @@ static __device__ __forceinline__ void walk_group(int g, int lane, uint4 *s, con
         const int2 rd = jb->frootm[sys];
         const int rt = __builtin_amdgcn_readfirstlane(rd.x);
         const float rc = __int_as_float(__builtin_amdgcn_readfirstlane(rd.y));
-        const uint64_t om = step(jb->froot4[sys], rt, rc, live);
+        const uint64_t om = step(jb->froot4[sys], rt, rc, frame_eps2(live, eps2));
         if (COUNT) nsteps += 1;
         if (om) {
             if (lane == 0) s[0] = make_uint4((unsigned)rt, 0u, (unsigned)om, (unsigned)(om >> 32));
@@ -154,6 +169,7 @@ static __device__ __forceinline__ void walk_group(int g, int lane, uint4 *s, con
         const int off = tag >> 4;  // the block's first record
         const uint64_t mask = ((uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)e.w) << 32) |
                               (uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)e.z);
+        const float e2 = frame_eps2(mask, eps2);
         work += nch;
         if (COUNT) {
             nsteps += nch;
@@ -183,8 +199,8 @@ static __device__ __forceinline__ void walk_group(int g, int lane, uint4 *s, con
             if (j >= nch) break;
             const int tj = __builtin_amdgcn_readfirstlane(d[j].x);
             const float cj = __int_as_float(__builtin_amdgcn_readfirstlane(d[j].y));
-            const uint64_t om = step(q[j], tj, cj, mask);
-            if (om) {
+            const uint64_t om = step(q[j], tj, cj, e2);
+            if (__builtin_expect(om != 0, !SOFT)) {
                 if (lane == 0) s[sp] = make_uint4((unsigned)tj, 0u, (unsigned)om, (unsigned)(om >> 32));
                 sp = __builtin_amdgcn_readfirstlane(sp + 1);
             }
@@ -339,8 +355,8 @@ static void launch_w(const ForceArgs &a, hipStream_t s, int waves)
 // block's trip to the L2, five child steps, the barrier).  Force kernel, one
 // wave per group against S waves: star + disk N = 2,000, 75 -> 18 us (S = 16);
 // 20,011-body sphere 338 -> 84 (16); 32,768-body disk 168 -> 37 (16); sphere
-// 65,536, 395 -> 161 (8); sphere 150,001 at theta 0.7, 240 -> 176 (8);
-// binary + disk 300,007 unsoftened at theta 0.3, 1089 -> 760 (4).
+// 65,536, 395 -> 161 (8); sphere 150,001 at theta 0.7, 240 -> 185 (8);
+// binary + disk 300,007 unsoftened at theta 0.3, 1089 -> 734 (4).
 // The register budget of eight waves per SIMD is worth a few reloads: with 94
 // scalar registers (seven waves) the same kernel was 5-15 % slower, with S = 16
 // 30 % (one workgroup per CU instead of two).
@@ -373,13 +389,13 @@ force_split_kernel(ForceJob jb, const float4 *__restrict__ fnode, const int2 *__
     float sx = 0.f, sy = 0.f, sz = 0.f;  // compensated totals of this wave
     float cx = 0.f, cy = 0.f, cz = 0.f;
     float px = 0.f, py = 0.f, pz = 0.f;
-    auto step = [&](const float4 q, const float crit, const uint64_t mask) -> uint64_t {
+    auto step = [&](const float4 q, const float crit, const float e2) -> uint64_t {  // as in walk_group
         const float dx = q.x - me.x;
         const float dy = q.y - me.y;
         const float dz = q.z - me.z;
-        const float d2 = fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, eps2)));
+        const float d2 = fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, e2)));
         const uint64_t ok = __ballot(crit < d2);
-        uint64_t takem = mask & ok;
+        uint64_t takem = ok;
         if (!SOFT) takem &= __ballot(d2 > 0.f);
         const float ri = __builtin_amdgcn_rsqf(SOFT || d2 > 0.f ? d2 : 1.f);
         float f = q.w * ri * (ri * ri);
@@ -387,11 +403,11 @@ force_split_kernel(ForceJob jb, const float4 *__restrict__ fnode, const int2 *__
         px = fmaf(f, dx, px);
         py = fmaf(f, dy, py);
         pz = fmaf(f, dz, pz);
-        return mask & ~ok;
+        return ~ok;
     };
     const int2 rd = jb.frootm[sys];
     const int rt = __builtin_amdgcn_readfirstlane(rd.x);
-    const uint64_t om = step(jb.froot4[sys], __int_as_float(__builtin_amdgcn_readfirstlane(rd.y)), live);
+    const uint64_t om = step(jb.froot4[sys], __int_as_float(__builtin_amdgcn_readfirstlane(rd.y)), frame_eps2(live, eps2));
     if (wave > 0) px = py = pz = 0.f;  // the root counts once
     int t = 0;
     const bool ok = split_walk<S>(L, wave, lane, make_uint4((unsigned)rt, 0u, (unsigned)om, (unsigned)(om >> 32)),
@@ -405,14 +421,15 @@ force_split_kernel(ForceJob jb, const float4 *__restrict__ fnode, const int2 *__
         asm volatile("" : "+v"(e.z), "+v"(e.w));
         const uint64_t mask = ((uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)e.w) << 32) |
                               (uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)e.z);
+        const float e2 = frame_eps2(mask, eps2);
         int k = 0;
         asm volatile("" : "+s"(k));  // a scalar count
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            if (j >= nch) break;
+            if (j > 0 && j >= nch) break;  // a frame has a child
             const int tj = __builtin_amdgcn_readfirstlane(d[j].x);
-            const uint64_t o = step(q[j], __int_as_float(__builtin_amdgcn_readfirstlane(d[j].y)), mask);
-            if (o) {
+            const uint64_t o = step(q[j], __int_as_float(__builtin_amdgcn_readfirstlane(d[j].y)), e2);
+            if (__builtin_expect(o != 0, !SOFT)) {
                 if (lane == 0) out[k] = make_uint4((unsigned)tj, 0u, (unsigned)o, (unsigned)(o >> 32));
                 k = __builtin_amdgcn_readfirstlane(k + 1);
             }
