@@ -298,7 +298,7 @@ vjp_kernel(VjpArgs v, int ngroups, const float4 *__restrict__ fnode, const int2 
         const int nch = tag & 15, off = tag >> 4;
         float4 q[8];
         int2 d[8];
-        load_block(fnode + off, fmeta + off, q, d);
+        load_block(fnode + off, fmeta + off, 0u, q, d);
         asm volatile("" : "+v"(e.z), "+v"(e.w));
         const uint64_t mask = ((uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)e.w) << 32) |
                               (uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)e.z);
@@ -353,12 +353,13 @@ vjp_split_kernel(VjpArgs v, const float4 *__restrict__ fnode, const int2 *__rest
         om = live & ~__ballot(rc < fmaf(dz, dz, fmaf(dy, dy, fmaf(dx, dx, eps2))));
     }
     const bool ok = split_walk<S>(L, wave, lane, make_uint4((unsigned)rt, 0u, (unsigned)om, (unsigned)(om >> 32)),
-                                  om != 0, [&](uint4 e, uint4 *out) -> int {
+                                  om != 0, [&](const uint4 *ep, uint4 *out) -> int {
+        uint4 e = *ep;
         const int tag = __builtin_amdgcn_readfirstlane((int)e.x);
         const int nch = tag & 15, off = tag >> 4;
         float4 q[8];
         int2 d[8];
-        load_block(fnode + off, fmeta + off, q, d);
+        load_block(fnode + off, fmeta + off, 0u, q, d);
         asm volatile("" : "+v"(e.z), "+v"(e.w));
         const uint64_t mask = ((uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)e.w) << 32) |
                               (uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)e.z);

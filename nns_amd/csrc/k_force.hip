@@ -10,7 +10,7 @@
 // through the scalar cache with three s_load_dwordx16 once per frame, and only
 // the block's own children are stepped through, with their data already in
 // SGPRs, so the only dependent memory access of a frame is that one load;
-// frames live in an LDS stack of {tag = first record << 4 | children, 0, lane
+// frames live in an LDS stack of {tag = first record << 4 | children, the tag again, lane
 // mask low, lane mask high}.
 //
 // Each lane applies its own opening test to a cell child (l/D < theta written
@@ -54,10 +54,16 @@
 
 namespace nbx {
 
-// eps^2 on the lanes of a frame's mask, infinite on the others.
+// eps^2 on the lanes of a frame's mask, infinite on the others; from the mask, or from
+// the lane's half of it (two vector instructions, no scalar ones).
 static __device__ __forceinline__ float frame_eps2(uint64_t mask, float eps2)
 {
     return __builtin_amdgcn_inverse_ballot_w64(mask) ? eps2 : INFINITY;
+}
+static __device__ __forceinline__ float frame_eps2(unsigned half, int lane, float eps2)
+{
+    const unsigned in = (unsigned)__builtin_amdgcn_sbfe((int)half, lane & 31, 1);  // all ones or zero
+    return __uint_as_float((in & __float_as_uint(eps2)) | (~in & __float_as_uint(INFINITY)));
 }
 
 // The walk of group g by the calling wave (all 64 lanes active), with the
@@ -97,11 +103,12 @@ static __device__ __forceinline__ void walk_group(int g, int lane, uint4 *s, con
     // and infinite on the others, which therefore open nothing and take a monopole of
     // zero.  (An infinite crit, theta = 0, is opened by every body; lanes past the last
     // body then open it too, and store nothing.)  The step is bound by the issue of its
-    // instructions, scalar ones and taken branches included: without the mask's two scalar
-    // operations, and with the push (one step in six) out of the way of the others, 1M
-    // bodies 1,778 -> 1,729 us, 4M 3,741 -> 3,665, 512 systems 11,636 -> 11,334.  Blocks
-    // fetched one frame ahead into vector registers and used through row broadcasts (DPP)
-    // made it 2,099 at 1M, one body of code per number of children 1,953.
+    // instructions, scalar ones and taken branches included.  Without the mask's two scalar
+    // operations, the push (one step in six) out of the way of the others and without an
+    // exec mask, offsets of 32 bits, half a mask per lane and one comparison to end the
+    // loop: 1M bodies 1,778 -> 1,600 us, 4M 3,741 -> 3,426, 512 systems 11,636 -> 10,350.
+    // Blocks fetched one frame ahead into vector registers and used through row broadcasts
+    // (DPP) made it 2,099 at 1M, one body of code per number of children 1,953.
     auto step = [&](const float4 q, const int tag, const float crit, const float e2) -> uint64_t {
         const float dx = q.x - me.x;
         const float dy = q.y - me.y;
@@ -144,75 +151,60 @@ static __device__ __forceinline__ void walk_group(int g, int lane, uint4 *s, con
         const uint64_t om = step(jb->froot4[sys], rt, rc, frame_eps2(live, eps2));
         if (COUNT) nsteps += 1;
         if (om) {
-            if (lane == 0) s[0] = make_uint4((unsigned)rt, 0u, (unsigned)om, (unsigned)(om >> 32));
+            if (lane == 0) s[0] = make_uint4((unsigned)rt, (unsigned)rt, (unsigned)om, (unsigned)(om >> 32));
             sp = 1;
         }
     }
-    // Frames run in tiles of kTile; the partials are folded after each tile.
-    // The frame loop has one exit, so the accumulators keep their registers
-    // from frame to frame (no copies between iterations).
-    constexpr int kTile = KAHAN ? 8 : 0x7fffffff;
-    bool overflow = false;
-    do {
-      for (int t = 0; t < kTile; ++t) {
-        if (sp <= 0) break;
-        // a frame pops one entry and pushes at most 8
-        if (sp > kForceStack - 7) {
-            overflow = true;
-            sp = 0;
-            break;
-        }
+    // The partials are folded every kTile frames (about 40 children).  The frame loop
+    // has one exit, so the accumulators keep their registers from frame to frame (no
+    // copies between iterations).
+    constexpr int kTile = 8;
+    int tile = kTile;
+    const unsigned *mine = reinterpret_cast<const unsigned *>(s) + (lane >> 5);
+    // A frame pops one entry and pushes at most 8: one comparison ends the loop when the
+    // stack is empty or has no room for that.
+    while ((unsigned)(sp - 1) < (unsigned)(kForceStack - 7)) {
         sp = __builtin_amdgcn_readfirstlane(sp - 1);
-        const uint4 e = s[sp];
-        const int tag = __builtin_amdgcn_readfirstlane((int)e.x);
-        const int nch = tag & 15;
-        const int off = tag >> 4;  // the block's first record
-        const uint64_t mask = ((uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)e.w) << 32) |
-                              (uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)e.z);
-        const float e2 = frame_eps2(mask, eps2);
+        // the lane's copy of the tag and its half of the mask
+        const unsigned *e = mine + 4 * sp;
+        const unsigned tag = (unsigned)__builtin_amdgcn_readfirstlane((int)e[0]), half = e[2];
+        const int nch = (int)(tag & 15u);
+        const unsigned at = tag & ~15u;  // bytes of the records before the block's first
+        const float e2 = frame_eps2(half, lane, eps2);
         work += nch;
         if (COUNT) {
             nsteps += nch;
             nframes += 1;
         }
-        const float4 *bq = fnode + off;
-        const int2 *bd = fmeta + off;
         float4 q[8];
         int2 d[8];
+        load_block(fnode, fmeta, at, q, d);
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-            q[j] = bq[j];
-            d[j] = bd[j];
-        }
-        // Every load of the block is issued before the first use: one wait per frame.
-        asm volatile("" ::"s"(q[0].x), "s"(q[0].y), "s"(q[0].z), "s"(q[0].w), "s"(q[1].x), "s"(q[1].y),
-                     "s"(q[1].z), "s"(q[1].w), "s"(q[2].x), "s"(q[2].y), "s"(q[2].z), "s"(q[2].w), "s"(q[3].x),
-                     "s"(q[3].y), "s"(q[3].z), "s"(q[3].w));
-        asm volatile("" ::"s"(q[4].x), "s"(q[4].y), "s"(q[4].z), "s"(q[4].w), "s"(q[5].x), "s"(q[5].y),
-                     "s"(q[5].z), "s"(q[5].w), "s"(q[6].x), "s"(q[6].y), "s"(q[6].z), "s"(q[6].w), "s"(q[7].x),
-                     "s"(q[7].y), "s"(q[7].z), "s"(q[7].w));
-        asm volatile("" ::"s"(d[0].x), "s"(d[0].y), "s"(d[1].x), "s"(d[1].y), "s"(d[2].x), "s"(d[2].y),
-                     "s"(d[3].x), "s"(d[3].y), "s"(d[4].x), "s"(d[4].y), "s"(d[5].x), "s"(d[5].y), "s"(d[6].x),
-                     "s"(d[6].y), "s"(d[7].x), "s"(d[7].y));
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            if (j >= nch) break;
+            if (j > 0 && j >= nch) break;  // a frame has a child
             const int tj = __builtin_amdgcn_readfirstlane(d[j].x);
             const float cj = __int_as_float(__builtin_amdgcn_readfirstlane(d[j].y));
             const uint64_t om = step(q[j], tj, cj, e2);
             if (__builtin_expect(om != 0, !SOFT)) {
-                if (lane == 0) s[sp] = make_uint4((unsigned)tj, 0u, (unsigned)om, (unsigned)(om >> 32));
+                // every lane stores the same: no exec mask to set and restore
+                s[sp] = make_uint4((unsigned)tj, (unsigned)tj, (unsigned)om, (unsigned)(om >> 32));
                 sp = __builtin_amdgcn_readfirstlane(sp + 1);
             }
         }
-      }
-        if (KAHAN) {  // fold the partials of the tile (about 40 children)
-            kahan_add(sx, cx, px); kahan_add(sy, cy, py); kahan_add(sz, cz, pz);
-            px = py = pz = 0.f;
+        if (KAHAN) {
+            tile = __builtin_amdgcn_readfirstlane(tile - 1);
+            if (__builtin_expect(tile == 0, 0)) {
+                kahan_add(sx, cx, px); kahan_add(sy, cy, py); kahan_add(sz, cz, pz);
+                px = py = pz = 0.f;
+                tile = kTile;
+            }
         }
-    } while (sp > 0);
+    }
+    if (KAHAN) {
+        kahan_add(sx, cx, px); kahan_add(sy, cy, py); kahan_add(sz, cz, pz);
+    }
     asm volatile("" ::: "memory");
-    if (overflow && lane == 0) atomicOr(jb->err, kErrStack);
+    if (sp > 0 && lane == 0) atomicOr(jb->err, kErrStack);
     if (!KAHAN) {
         sx = px; sy = py; sz = pz;
     }
@@ -355,8 +347,8 @@ static void launch_w(const ForceArgs &a, hipStream_t s, int waves)
 // block's trip to the L2, five child steps, the barrier).  Force kernel, one
 // wave per group against S waves: star + disk N = 2,000, 75 -> 18 us (S = 16);
 // 20,011-body sphere 338 -> 84 (16); 32,768-body disk 168 -> 37 (16); sphere
-// 65,536, 395 -> 161 (8); sphere 150,001 at theta 0.7, 240 -> 185 (8);
-// binary + disk 300,007 unsoftened at theta 0.3, 1089 -> 734 (4).
+// 65,536, 395 -> 149 (8); sphere 150,001 at theta 0.7, 240 -> 174 (8);
+// binary + disk 300,007 unsoftened at theta 0.3, 1089 -> 700 (4).
 // The register budget of eight waves per SIMD is worth a few reloads: with 94
 // scalar registers (seven waves) the same kernel was 5-15 % slower, with S = 16
 // 30 % (one workgroup per CU instead of two).
@@ -409,19 +401,17 @@ force_split_kernel(ForceJob jb, const float4 *__restrict__ fnode, const int2 *__
     const int rt = __builtin_amdgcn_readfirstlane(rd.x);
     const uint64_t om = step(jb.froot4[sys], __int_as_float(__builtin_amdgcn_readfirstlane(rd.y)), frame_eps2(live, eps2));
     if (wave > 0) px = py = pz = 0.f;  // the root counts once
-    int t = 0;
-    const bool ok = split_walk<S>(L, wave, lane, make_uint4((unsigned)rt, 0u, (unsigned)om, (unsigned)(om >> 32)),
-                                  om != 0, [&](uint4 e, uint4 *out) -> int {
-        const int tag = __builtin_amdgcn_readfirstlane((int)e.x);
-        const int nch = tag & 15, off = tag >> 4;
+    int t = 8;
+    const bool ok = split_walk<S>(L, wave, lane, make_uint4((unsigned)rt, (unsigned)rt, (unsigned)om, (unsigned)(om >> 32)),
+                                  om != 0, [&](const uint4 *e, uint4 *out) -> int {
+        // the lane's copy of the tag and its half of the mask
+        const unsigned *mine = reinterpret_cast<const unsigned *>(e) + (lane >> 5);
+        const unsigned tag = (unsigned)__builtin_amdgcn_readfirstlane((int)mine[0]), half = mine[2];
+        const int nch = (int)(tag & 15u);
         float4 q[8];
         int2 d[8];
-        load_block(fnode + off, fmeta + off, q, d);
-        // the mask after the block's loads: a wait for it in between would split them
-        asm volatile("" : "+v"(e.z), "+v"(e.w));
-        const uint64_t mask = ((uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)e.w) << 32) |
-                              (uint64_t)(unsigned)__builtin_amdgcn_readfirstlane((int)e.z);
-        const float e2 = frame_eps2(mask, eps2);
+        load_block(fnode, fmeta, tag & ~15u, q, d);
+        const float e2 = frame_eps2(half, lane, eps2);
         int k = 0;
         asm volatile("" : "+s"(k));  // a scalar count
 #pragma unroll
@@ -430,14 +420,17 @@ force_split_kernel(ForceJob jb, const float4 *__restrict__ fnode, const int2 *__
             const int tj = __builtin_amdgcn_readfirstlane(d[j].x);
             const uint64_t o = step(q[j], __int_as_float(__builtin_amdgcn_readfirstlane(d[j].y)), e2);
             if (__builtin_expect(o != 0, !SOFT)) {
-                if (lane == 0) out[k] = make_uint4((unsigned)tj, 0u, (unsigned)o, (unsigned)(o >> 32));
+                out[k] = make_uint4((unsigned)tj, (unsigned)tj, (unsigned)o, (unsigned)(o >> 32));  // from every lane
                 k = __builtin_amdgcn_readfirstlane(k + 1);
             }
         }
-        if (KAHAN && ++t == 8) {
-            kahan_add(sx, cx, px); kahan_add(sy, cy, py); kahan_add(sz, cz, pz);
-            px = py = pz = 0.f;
-            t = 0;
+        if (KAHAN) {
+            t = __builtin_amdgcn_readfirstlane(t - 1);
+            if (__builtin_expect(t == 0, 0)) {
+                kahan_add(sx, cx, px); kahan_add(sy, cy, py); kahan_add(sz, cz, pz);
+                px = py = pz = 0.f;
+                t = 8;
+            }
         }
         return k;
     });

@@ -51,7 +51,7 @@ static __device__ inline int row_inclusive_sum(int v)
 }
 
 // Walks every frame below `root` (walked itself when open; both the same in all
-// S waves).  frame(e, out) walks the frame of entry e = {tag, -, mask} with the
+// S waves).  frame(e, out) walks the frame of entry *e = {tag, tag, mask} with the
 // calling wave, writes the frames it opens to out[0 .. 8) and returns their
 // number.  Returns false (in every wave) if the stack bound was passed.  All
 // threads of the workgroup call it.
@@ -82,7 +82,7 @@ static __device__ __forceinline__ bool split_walk(SplitStack<S> &L, int wave, in
             } else {
                 e = &L.stk[sp - 1 - (wave - tot)];
             }
-            pushed = frame(*e, L.stage[P ^ 1][wave]);
+            pushed = frame(e, L.stage[P ^ 1][wave]);
         }
         if (lane == 0) L.cnt[P ^ 1][wave] = pushed;
         sp = tot >= S ? sp + tot - S : max(0, sp + tot - S);
@@ -92,11 +92,14 @@ static __device__ __forceinline__ bool split_walk(SplitStack<S> &L, int wave, in
     }
 }
 
-// A frame's block: eight records from the first, every load issued before the
-// first use (three scalar loads of 64 bytes, one wait).
-static __device__ __forceinline__ void load_block(const float4 *__restrict__ bq, const int2 *__restrict__ bd,
-                                                  float4 (&q)[8], int2 (&d)[8])
+// A frame's block: eight records from the first (`at`: bytes of the records before it
+// in fnode, the tag without its count), every load issued before the first use (three
+// scalar loads of 64 bytes, one wait).
+static __device__ __forceinline__ void load_block(const float4 *__restrict__ fnode, const int2 *__restrict__ fmeta,
+                                                  unsigned at, float4 (&q)[8], int2 (&d)[8])
 {
+    const float4 *bq = reinterpret_cast<const float4 *>(reinterpret_cast<const char *>(fnode) + at);
+    const int2 *bd = reinterpret_cast<const int2 *>(reinterpret_cast<const char *>(fmeta) + (at >> 1));
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
         q[j] = bq[j];
