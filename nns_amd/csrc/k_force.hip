@@ -479,10 +479,10 @@ static void launch_split(const ForceArgs &a, hipStream_t s, int S)
 // Waves per group.  As many as fill the device (256 CUs of 32 waves) about once,
 // 16 at most.  Each round costs a barrier and the hand-out of the frames, so once
 // the waves of one-wave groups fill the device by themselves the shared walk only
-// adds work: 4,096 groups (sphere of 262,144) 576 us with 4 waves per group
-// against 632 with one, 8,192 groups 1,129 against 1,031 (sphere) and 573 against
-// 600 (disk).  16 waves: 1,024 groups 176 us against 161 with 8; 313 groups 84
-// against 96.
+// adds work.  Force stage in us with one wave per group, 4 and 8: 2,560 groups, sphere
+// 419, 367, 348, disk 293, 192, 171; 4,096 groups 533, 521, 535 and 362, 261, 255; 5,120
+// groups 612, 641, 670 and 393, 352, 346; 8,192 groups 900, 1,018, 1,089 and 512, 515,
+// 539.  16 waves: 1,024 groups 176 us against 161 with 8; 313 groups 84 against 96.
 static int split_waves(int ngroups)
 {
     return ngroups <= 640 ? 16 : ngroups <= 2560 ? 8 : ngroups <= 5120 ? 4 : 1;

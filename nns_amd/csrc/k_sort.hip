@@ -8,8 +8,8 @@
 // passes of 8 bits were 24; up to 17 chunks are merged in one launch (rank_merge_kernel).
 // Keys and permutation on one MI355X, radix -> merge:
 // N = 2,000, 95 -> 16 us; 20,011, 127 -> 31; 150,001, 132 -> 71; 1,000,003, 172 -> 127;
-// 4,194,304, 388 -> 370 (and its Morton keys are made on the way, 37 us less); 8.4 M,
-// 737 -> 753.  Chunks of 8,192 pairs take 36 us against 29 at N = 8,192 and 131
+// 4,194,304, 388 -> 308 (and its Morton keys are made on the way, 37 us less); 8.4 M by
+// radix 737, 8.0 M merged 595.  Chunks of 8,192 pairs take 36 us against 29 at N = 8,192 and 131
 // against 127 at 1M (one workgroup per CU instead of three), chunks of 2,048 139.
 //
 // Segments: the pairs of one system, or of each system of an ensemble, sorted
@@ -177,20 +177,41 @@ __global__ void __launch_bounds__(kChunkThreads) chunk_sort_kernel(SortSource sr
     }
 }
 
-// First i in [lo, hi] with i == hi or A[i] > B[d - 1 - i]: how many of the first d
-// merged pairs come from A.  One wave, 64 probes per round.
-__device__ inline int merge_split(const uint64_t *__restrict__ A, const uint64_t *__restrict__ B, int na, int nb, int d,
-                                  int lane)
+// Steps of a split's rounds in a pass over runs of R, as powers of two of five bits each,
+// the first lowest: 64 probes from a multiple of a step reach over the run, or over
+// the step before.  From kMergeGrid pairs on, whose passes are bound by what they
+// fetch; 0 (probes spread evenly) below: there the lines that all tiles probe at the
+// same time, 16 KB apart, cost more than they save.  Sort of 64-bit keys, spread and at
+// multiples: 1M pairs 126 and 133 us, 1.5M 163 and 156, 2M 182 and 161, 4,194,304
+// 370 and 308, 8M 728 and 595.
+constexpr int kMergeGrid = 5 << 18;
+static uint32_t merge_steps(int n, int64_t R)
 {
+    if (n < kMergeGrid) return 0;
+    return R <= 64 << 6 ? 6 : R <= 64 << 11 ? 11 | 6 << 5 : R <= 64 << 17 ? 17 | 11 << 5 | 6 << 10 : 23 | 17 << 5 | 11 << 10 | 6 << 15;
+}
+
+// First i in [lo, hi] with i == hi or A[i] > B[d - 1 - i]: how many of the first d
+// merged pairs come from A.  One wave, 64 probes per round, a step apart and, with
+// steps, at multiples of it: from steps of 2,048 up (d is a multiple of that but
+// for the last tile) the tiles of a merge probe the same lines, and the 66 lines of
+// the round of 64 are the only ones that a tile fetches for itself.  Spread evenly,
+// the probes fetch as much again as the pairs.
+__device__ inline int merge_split(const uint64_t *__restrict__ A, const uint64_t *__restrict__ B, int na, int nb, int d,
+                                  uint32_t steps, int lane)
+{
+    const bool grid = steps != 0;
     int lo = max(0, d - nb), hi = min(d, na);
     while (lo < hi) {
-        const int step = (hi - lo + 63) >> 6;
-        const int i = lo + lane * step;
+        const int step = grid ? 1 << (steps & 31) : (hi - lo + 63) >> 6;
+        const int base = grid ? lo & -step : lo;
+        steps >>= 5;
+        const int i = max(lo, base + lane * step);
         const bool ok = i < hi && A[i] <= B[d - 1 - i];
         const int c = __popcll(__ballot(ok));  // the probes that hold are the first c
         // the answer lies past probe c - 1 and not past probe c
-        const int nlo = c ? lo + (c - 1) * step + 1 : lo;
-        hi = min(hi, lo + c * step);
+        const int nlo = c ? max(lo, base + (c - 1) * step) + 1 : lo;
+        hi = min(hi, max(lo, base + c * step));
         lo = nlo;
     }
     return lo;
@@ -198,11 +219,11 @@ __device__ inline int merge_split(const uint64_t *__restrict__ A, const uint64_t
 
 // Output tile `sub` of a chunk in the pass that merges runs of R into runs of 2 R.
 // Bound by its round trips (the split search, the tile's load, the merge in LDS:
-// 8 us) while the tiles fit the device at once, then by HBM: 35 us for 4M pairs, 100 MB.
+// 8 us) while the tiles fit the device at once, then by HBM: 25 us for 4M pairs, 100 MB.
 __global__ void __launch_bounds__(kMergeThreads) merge_pass_kernel(const uint64_t *__restrict__ kin,
                                                                    const int32_t *__restrict__ vin,
                                                                    const int4 *__restrict__ chunks, int n, int R,
-                                                                   uint64_t *__restrict__ kout,
+                                                                   uint32_t steps, uint64_t *__restrict__ kout,
                                                                    int32_t *__restrict__ vout,
                                                                    int32_t *__restrict__ inv)
 {
@@ -221,7 +242,7 @@ __global__ void __launch_bounds__(kMergeThreads) merge_pass_kernel(const uint64_
     const int na = min(R, ck.y - p), nb = (int)min((int64_t)R, max((int64_t)0, (int64_t)ck.y - p - R));
     const uint64_t *A = kin + p, *B = kin + p + na;
     if (wave < 2) {
-        const int i = merge_split(A, B, na, nb, o0 - p + (wave ? cnt : 0), lane);
+        const int i = merge_split(A, B, na, nb, o0 - p + (wave ? cnt : 0), steps, lane);
         if (lane == 0) s_split[wave] = i;
     }
     __syncthreads();
@@ -376,7 +397,8 @@ static void sort_pairs(const SortSource &src, const SortSegs &g, uint64_t *keys_
     chunk_sort_kernel<BODIES><<<g.nchunks, kChunkThreads, 0, s>>>(src, g.chunks, g.n, k, v, passes ? nullptr : inv_out);
     for (int p = 0; p < passes; ++p) {
         merge_pass_kernel<<<g.nchunks * (kSortChunk / kMergeTile), kMergeThreads, 0, s>>>(
-            k, v, g.chunks, g.n, kSortChunk << p, k2, v2, p == passes - 1 ? inv_out : nullptr);
+            k, v, g.chunks, g.n, kSortChunk << p, merge_steps(g.n, (int64_t)kSortChunk << p), k2, v2,
+            p == passes - 1 ? inv_out : nullptr);
         std::swap(k, k2);
         std::swap(v, v2);
     }
