@@ -8,8 +8,8 @@
 // passes of 8 bits were 24; up to 17 chunks are merged in one launch (rank_merge_kernel).
 // Keys and permutation on one MI355X, radix -> merge:
 // N = 2,000, 95 -> 16 us; 20,011, 127 -> 31; 150,001, 132 -> 71; 1,000,003, 172 -> 127;
-// 4,194,304, 388 -> 308 (and its Morton keys are made on the way, 37 us less); 8.4 M by
-// radix 737, 8.0 M merged 595.  Chunks of 8,192 pairs take 36 us against 29 at N = 8,192 and 131
+// 4,194,304, 388 -> 285 (and its Morton keys are made on the way, 37 us less); 8.4 M by
+// radix 737, 8.0 M merged 545.  Chunks of 8,192 pairs take 36 us against 29 at N = 8,192 and 131
 // against 127 at 1M (one workgroup per CU instead of three), chunks of 2,048 139.
 //
 // Segments: the pairs of one system, or of each system of an ensemble, sorted
@@ -182,8 +182,8 @@ __global__ void __launch_bounds__(kChunkThreads) chunk_sort_kernel(SortSource sr
 // the step before.  From kMergeGrid pairs on, whose passes are bound by what they
 // fetch; 0 (probes spread evenly) below: there the lines that all tiles probe at the
 // same time, 16 KB apart, cost more than they save.  Sort of 64-bit keys, spread and at
-// multiples: 1M pairs 126 and 133 us, 1.5M 163 and 156, 2M 182 and 161, 4,194,304
-// 370 and 308, 8M 728 and 595.
+// multiples (tiles in launch order): 1M pairs 126 and 133 us, 1.5M 163 and 156, 2M 182
+// and 161, 4,194,304 370 and 308, 8M 728 and 595.
 constexpr int kMergeGrid = 5 << 18;
 static uint32_t merge_steps(int n, int64_t R)
 {
@@ -219,11 +219,15 @@ __device__ inline int merge_split(const uint64_t *__restrict__ A, const uint64_t
 
 // Output tile `sub` of a chunk in the pass that merges runs of R into runs of 2 R.
 // Bound by its round trips (the split search, the tile's load, the merge in LDS:
-// 8 us) while the tiles fit the device at once, then by HBM: 25 us for 4M pairs, 100 MB.
+// 8 us) while the tiles fit the device at once, then by HBM: 23 us for 4M pairs, 100 MB.
+// Large merges (steps) give each XCD consecutive tiles, whose pairs and splits share
+// lines of its L2 (block b runs on XCD b mod 8): sort of 1.5M pairs 156 -> 147 us,
+// 4,194,304 308 -> 285, 8M 597 -> 545.
 __global__ void __launch_bounds__(kMergeThreads) merge_pass_kernel(const uint64_t *__restrict__ kin,
                                                                    const int32_t *__restrict__ vin,
                                                                    const int4 *__restrict__ chunks, int n, int R,
-                                                                   uint32_t steps, uint64_t *__restrict__ kout,
+                                                                   uint32_t steps, int ntiles,
+                                                                   uint64_t *__restrict__ kout,
                                                                    int32_t *__restrict__ vout,
                                                                    int32_t *__restrict__ inv)
 {
@@ -233,8 +237,11 @@ __global__ void __launch_bounds__(kMergeThreads) merge_pass_kernel(const uint64_
     __shared__ int s_split[2];
     const int t = threadIdx.x, lane = t & 63;
     const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
-    const int4 ck = chunk_of(chunks, n, blockIdx.x / kSub);
-    const int o0 = ck.x + ck.z * kSortChunk + (int)(blockIdx.x % kSub) * kMergeTile;
+    const int b = blockIdx.x;
+    const int tile = steps ? (b & 7) * (int)(gridDim.x >> 3) + (b >> 3) : b;
+    if (tile >= ntiles) return;
+    const int4 ck = chunk_of(chunks, n, tile / kSub);
+    const int o0 = ck.x + ck.z * kSortChunk + tile % kSub * kMergeTile;
     if (o0 >= ck.y) return;
     const int cnt = min(kMergeTile, ck.y - o0);
     const int64_t rel = o0 - ck.x;
@@ -396,8 +403,9 @@ static void sort_pairs(const SortSource &src, const SortSegs &g, uint64_t *keys_
     int32_t *v = passes % 2 ? tmp_v : perm_out, *v2 = passes % 2 ? perm_out : tmp_v;
     chunk_sort_kernel<BODIES><<<g.nchunks, kChunkThreads, 0, s>>>(src, g.chunks, g.n, k, v, passes ? nullptr : inv_out);
     for (int p = 0; p < passes; ++p) {
-        merge_pass_kernel<<<g.nchunks * (kSortChunk / kMergeTile), kMergeThreads, 0, s>>>(
-            k, v, g.chunks, g.n, kSortChunk << p, merge_steps(g.n, (int64_t)kSortChunk << p), k2, v2,
+        const int ntiles = g.nchunks * (kSortChunk / kMergeTile);
+        merge_pass_kernel<<<(ntiles + 7) / 8 * 8, kMergeThreads, 0, s>>>(
+            k, v, g.chunks, g.n, kSortChunk << p, merge_steps(g.n, (int64_t)kSortChunk << p), ntiles, k2, v2,
             p == passes - 1 ? inv_out : nullptr);
         std::swap(k, k2);
         std::swap(v, v2);
