@@ -64,12 +64,13 @@ FLOP_PER_INTERACTION = 20  # GPU Gems 3 convention
 
 def stage_bytes(n, m, c):
     """Algorithmic HBM bytes of the non-force stages for n bodies, m nodes and c
-    cells: reset 44m + 16(m - n); bbox 12n; build = keys 36n + 8 radix passes of
-    24n + lcp, tree and key-ordered bodies 32n + 40c; centre of mass 16(n + c) +
-    80c; sort stage (sorted[], frame layout, group order) 8n + 56c + 24n + 8n +
-    4 radix passes of 24n; update 60n."""
-    return {"reset": 44 * m + 16 * (m - n), "bbox": 12 * n, "build": 36 * n + 8 * 24 * n + 32 * n + 40 * c,
-            "com": 16 * (n + c) + 80 * c, "sort": 8 * n + 56 * c + 24 * n + 8 * n + 4 * 24 * n, "update": 60 * n}
+    cells: reset 44m + 16(m - n); bbox 12n; build = keys and float4 bodies 40n +
+    sorted chunks of 4096 pairs 12n + log2(n / 4096) merges of 24n + lcp, tree and
+    key-ordered bodies 45n + 40c; centre of mass 16(n + c) + 80c; sort stage
+    (sorted[], frame layout, group order) 8n + 56c + 24n + 4n + 44c; update 60n."""
+    merges = max(0, -(-n // 4096) - 1).bit_length()
+    return {"reset": 44 * m + 16 * (m - n), "bbox": 12 * n, "build": (40 + 12 + 24 * merges + 45) * n + 40 * c,
+            "com": 16 * (n + c) + 80 * c, "sort": 8 * n + 56 * c + 24 * n + 4 * n + 44 * c, "update": 60 * n}
 
 
 def parse():

@@ -219,7 +219,7 @@ __device__ inline int merge_split(const uint64_t *__restrict__ A, const uint64_t
 
 // Output tile `sub` of a chunk in the pass that merges runs of R into runs of 2 R.
 // Bound by its round trips (the split search, the tile's load, the merge in LDS:
-// 8 us) while the tiles fit the device at once, then by HBM: 23 us for 4M pairs, 100 MB.
+// 8 us) while the tiles fit the device at once, then by HBM: 22 us for 4M pairs, 100 MB (the last pass, with inv, 79).
 // Large merges (steps) give each XCD consecutive tiles, whose pairs and splits share
 // lines of its L2 (block b runs on XCD b mod 8): sort of 1.5M pairs 156 -> 147 us,
 // 4,194,304 308 -> 285, 8M 597 -> 545.
