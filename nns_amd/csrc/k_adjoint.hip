@@ -399,13 +399,13 @@ vjp_split_kernel(VjpArgs v, const float4 *__restrict__ fnode, const int2 *__rest
     }
 }
 
-// Clears the gradient sums and the log's counters.
+// Clears the gradient sums and the log's counters (of a small system more than its sums).
 __global__ void __launch_bounds__(256) vjp_clear_kernel(double *__restrict__ p, int64_t count, int *__restrict__ next,
                                                         int nnext)
 {
-    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x;
-    for (int64_t k = t; k < count; k += (int64_t)blockDim.x * gridDim.x) p[k] = 0.0;
-    if (t < nnext) next[t] = 0;
+    const int64_t t = blockIdx.x * (int64_t)blockDim.x + threadIdx.x, stride = (int64_t)blockDim.x * gridDim.x;
+    for (int64_t k = t; k < count; k += stride) p[k] = 0.0;
+    for (int64_t k = t; k < nnext; k += stride) next[k] = 0;
 }
 
 // ---- sums of the log, node by node: binned form
