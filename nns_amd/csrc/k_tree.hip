@@ -1069,22 +1069,27 @@ __global__ void __launch_bounds__(T, POOL == kSumSmall ? 8 : 4) subtree_summary_
 // Top summary: the top cells level by level, deepest first, then the roots.  A
 // level's cells read only the levels below.  A cell's sum gathers from up to 8
 // children in unrelated cache lines, and one CU's address pipeline takes such
-// gathers a few lanes at a time, so while more than kTopItems - 64 cells are left, a
-// level is spread over kTopBlocks workgroups (its cell i to workgroup i mod kTopBlocks)
-// that meet at a grid barrier after it; the levels that are then left are summed by
-// workgroup 0 alone, in LDS.
-// kTopBlocks workgroups of 512 threads fit on the device at once, so every
-// workgroup reaches every barrier; the wait is bounded all the same: one that
+// gathers a few lanes at a time, so while more are left than fit there,
+// the levels are spread over kTopBlocks workgroups (a level's cell i to workgroup i mod
+// kTopBlocks) that meet at a grid barrier after each (top_levels_kernel); the rest is
+// summed by one workgroup alone, in LDS (top_summary_kernel).
+// The workgroups of a grid barrier must all be on the device at once.  Those of
+// top_levels_kernel hold no LDS to speak of and 256 threads, so 64 fit any partition of an MI355X
+// (32 CUs at least) twice over, beside other kernels and launches of their own kind; the
+// LDS part, whose workgroup takes a CU for itself, is a launch of its own (a step of 1M
+// bodies 2,036 us, with both in one launch 2,034).  The wait is bounded all the same: one that
 // runs out latches kErrStall, and every wave still finishes.
-constexpr int kTopBlocks = 64;
+constexpr int kTopBlocks = 64, kTopLevelThreads = 256;
 // Up to kTopOneGroup bodies there are hardly ever many more top cells than fit, and
 // one workgroup sums them all; up to kTopFew bodies in a third of the LDS.  Workgroups that
 // need most of a CU's LDS hold up the kernels of other streams: three ensembles of 96
-// systems (100,000 bodies) side by side took 3 % longer a step with 64 workgroups of
-// 145 KB, 1.6 % with one, and as long as before with one of 52 KB.
+// systems (100,000 bodies) side by side took 1.6 % longer a step with one of 145 KB
+// and as long as before with one of 52 KB.
 constexpr int kTopOneGroup = 1 << 19;
 constexpr int kTopSmall = 160, kTopLarge = 448, kTopFew = 1 << 17;
 constexpr int kTopSpin = 1 << 20;  // polls of one barrier wait (about a second)
+// Top cells that the LDS part takes with room for `items`; the others leave some to the roots.
+constexpr int top_lds_cells(int items) { return items * 7 / 8; }
 
 // Grid barrier number `phase` (1, 2, ...) of the launch.  Every wave waits until its
 // stores have reached the XCD's L2; thread 0 then makes them visible device-wide with its
@@ -1208,43 +1213,41 @@ __device__ inline void top_in_lds(TopLds<ITEMS> &t, int *first, const SumOut &o,
     }
 }
 
-template <bool CURSOR, int ITEMS>
-__global__ void __launch_bounds__(kTopThreads) top_summary_kernel(SumOut o, Segs g, int base0, int nsamples,
-                                                          const uint32_t *__restrict__ top_id, DeviceState *st)
+// The top cells of level L are the ids base0 + [first[L], first[L + 1]) (the scanned,
+// level-major top table).  Called by the whole workgroup; ends with a barrier.
+__device__ inline void top_levels(int *first, const uint32_t *top_id, int nsamples, const DeviceState *st)
+{
+    const int tid = threadIdx.x;
+    if (tid <= kLevels)
+        first[tid] = tid < kLevels ? (int)top_id[tid * nsamples]
+                                   : __hip_atomic_load(&st->ntop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+}
+
+// The levels below those that the LDS part takes with room for kTopLarge items.
+template <bool CURSOR>
+__global__ void __launch_bounds__(kTopLevelThreads) top_levels_kernel(SumOut o, int base0, int nsamples,
+                                                                      const uint32_t *__restrict__ top_id,
+                                                                      DeviceState *st)
 {
     __shared__ int s_first[kLevels + 1];
     __shared__ int s_stop;
-    __shared__ TopLds<ITEMS> s_top;
-    __shared__ int s_low[CURSOR ? 1 : 8 * ITEMS];
     const int tid = threadIdx.x;
     if (tid == 0) s_stop = latched(st);  // one read for the whole workgroup
-    // The top cells of level L are the ids base0 + [s_first[L], s_first[L + 1])
-    // (the scanned, level-major top table); every workgroup reads the same.
-    if (tid <= kLevels)
-        s_first[tid] = tid < kLevels ? (int)top_id[tid * nsamples]
-                                     : __hip_atomic_load(&st->ntop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    __syncthreads();
+    top_levels(s_first, top_id, nsamples, st);
     // Latched before this launch: every workgroup reads it so and skips the sums,
     // but still meets every barrier (a latch raised by this launch's own sums may
     // be seen by some workgroups only).
     const bool stop = s_stop != 0;
     bool stalled = false;
-    int L = kKeyLevels, phase = 0;
-    for (; L >= 1 && s_first[L + 1] > (ITEMS * 7) / 8; --L) {
+    int phase = 0;
+    for (int L = kKeyLevels; L >= 1 && s_first[L + 1] > top_lds_cells(kTopLarge); --L) {
         const int cnt = s_first[L + 1] - s_first[L];
         if (cnt <= 0) continue;  // uniform: no barrier for an empty level
         if (!stop)
             for (int i = blockIdx.x + gridDim.x * tid; i < cnt; i += gridDim.x * blockDim.x)
                 summarise<4, CURSOR>(o, base0 + s_first[L] + i, st, false, 0, L);
         top_barrier(st, ++phase, stalled);
-    }
-    if (blockIdx.x == 0 && !stop) {
-        const int left = s_first[L + 1];
-        const bool roots = left + g.nseg <= ITEMS;
-        top_in_lds<CURSOR>(s_top, s_low, o, g, base0, left, roots ? g.nseg : 0, s_first, L, st);
-        __syncthreads();
-        if (!roots)  // every top cell is summed
-            for (int s = tid; s < g.nseg; s += blockDim.x) summarise<4, CURSOR>(o, seg_root(g, s), st, !g.batch);
     }
     if (phase == 0) return;
     if (tid == 0) {  // the last workgroup out (every other one is past its last wait) resets the barrier
@@ -1254,6 +1257,36 @@ __global__ void __launch_bounds__(kTopThreads) top_summary_kernel(SumOut o, Segs
             __hip_atomic_store(&st->tdone, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         }
     }
+}
+
+// One workgroup.  WIDE: also the levels below those that fit (without a launch of
+// top_levels_kernel before).
+template <bool CURSOR, int ITEMS, bool WIDE>
+__global__ void __launch_bounds__(kTopThreads) top_summary_kernel(SumOut o, Segs g, int base0, int nsamples,
+                                                          const uint32_t *__restrict__ top_id, DeviceState *st)
+{
+    static_assert(WIDE || ITEMS == kTopLarge, "top_levels_kernel leaves off at kTopLarge");
+    __shared__ int s_first[kLevels + 1];
+    __shared__ int s_stop;
+    __shared__ TopLds<ITEMS> s_top;
+    __shared__ int s_low[CURSOR ? 1 : 8 * ITEMS];
+    const int tid = threadIdx.x;
+    if (tid == 0) s_stop = latched(st);  // one read for the whole workgroup
+    top_levels(s_first, top_id, nsamples, st);
+    if (s_stop) return;
+    int L = kKeyLevels;
+    for (; L >= 1 && s_first[L + 1] > top_lds_cells(ITEMS); --L) {
+        if (!WIDE) continue;
+        for (int i = s_first[L] + tid; i < s_first[L + 1]; i += kTopThreads)
+            summarise<4, CURSOR>(o, base0 + i, st, false, 0, L);
+        __syncthreads();
+    }
+    const int left = s_first[L + 1];
+    const bool roots = left + g.nseg <= ITEMS;
+    top_in_lds<CURSOR>(s_top, s_low, o, g, base0, left, roots ? g.nseg : 0, s_first, L, st);
+    __syncthreads();
+    if (!roots)  // every top cell is summed
+        for (int s = tid; s < g.nseg; s += kTopThreads) summarise<4, CURSOR>(o, seg_root(g, s), st, !g.batch);
 }
 
 // ------------------------------------------------------------------ layout
@@ -1695,11 +1728,14 @@ static void summarise_tree(Segs g, int base0, int nsamples, TreeScratch &ts, Dev
         subtree_summary_kernel<CURSOR, 256, kSumPool, kSumSmall><<<grid, 256, 0, s>>>(o, ts.sub, ts.sub_max, ts.subcells, st);
         subtree_summary_kernel<CURSOR, kSumSmallT, kSumSmall, 0><<<grid, kSumSmallT, 0, s>>>(o, ts.sub, ts.sub_max, ts.subcells, st);
     }
-    if (g.n <= kTopFew)
-        top_summary_kernel<CURSOR, kTopSmall><<<1, kTopThreads, 0, s>>>(o, g, base0, nsamples, ts.top_id, st);
-    else
-        top_summary_kernel<CURSOR, kTopLarge><<<g.n <= kTopOneGroup ? 1 : kTopBlocks, kTopThreads, 0, s>>>(
-            o, g, base0, nsamples, ts.top_id, st);
+    if (g.n <= kTopFew) {
+        top_summary_kernel<CURSOR, kTopSmall, true><<<1, kTopThreads, 0, s>>>(o, g, base0, nsamples, ts.top_id, st);
+    } else if (g.n <= kTopOneGroup) {
+        top_summary_kernel<CURSOR, kTopLarge, true><<<1, kTopThreads, 0, s>>>(o, g, base0, nsamples, ts.top_id, st);
+    } else {
+        top_levels_kernel<CURSOR><<<kTopBlocks, kTopLevelThreads, 0, s>>>(o, base0, nsamples, ts.top_id, st);
+        top_summary_kernel<CURSOR, kTopLarge, false><<<1, kTopThreads, 0, s>>>(o, g, base0, nsamples, ts.top_id, st);
+    }
 }
 // base0: the first top cell's id; nsamples: the top table's samples.
 static void summarise_tree(Segs g, int base0, int nsamples, TreeScratch &ts, DeviceState *st, hipStream_t s,
