@@ -66,6 +66,11 @@ static __device__ __forceinline__ float frame_eps2(unsigned half, int lane, floa
     return __uint_as_float((in & __float_as_uint(eps2)) | (~in & __float_as_uint(INFINITY)));
 }
 
+// m ri^3 of a monopole, exactly 0 where ri is 0 (the lanes outside a frame's mask), also of a
+// mass that is past FP32: v_mul_legacy_f32 rounds as v_mul_f32 does, but 0 times anything is 0.
+extern "C" __device__ float nbx_mul_legacy(float, float) __asm("llvm.amdgcn.fmul.legacy");
+static __device__ __forceinline__ float weight(float m, float ri) { return nbx_mul_legacy(m, ri) * (ri * ri); }
+
 // The walk of group g by the calling wave (all 64 lanes active), with the
 // wave's LDS stack s.  The launch's other arguments come from its job record
 // jb, read when the walk starts and again when it ends (the empty asm with a
@@ -127,7 +132,7 @@ static __device__ __forceinline__ void walk_group(int g, int lane, uint4 *s, con
             // lanes and zeroed by one select for those that do not take the child:
             // no exec-mask branch, fewer scalar instructions per step
             const float ri = __builtin_amdgcn_rsqf(d2);
-            float f = q.w * ri * (ri * ri);
+            float f = weight(q.w, ri);
             f = __builtin_amdgcn_inverse_ballot_w64(takem) ? f : 0.f;
             px = fmaf(f, dx, px);
             py = fmaf(f, dy, py);
@@ -135,7 +140,7 @@ static __device__ __forceinline__ void walk_group(int g, int lane, uint4 *s, con
         } else if (__builtin_amdgcn_inverse_ballot_w64(takem)) {  // exec = takem: no select, skipped when empty
             asm volatile("");  // keeps the branch (no if-conversion into selects of the partials)
             const float ri = __builtin_amdgcn_rsqf(d2);
-            const float f = q.w * ri * (ri * ri);
+            const float f = weight(q.w, ri);
             px = fmaf(f, dx, px);
             py = fmaf(f, dy, py);
             pz = fmaf(f, dz, pz);
@@ -390,7 +395,7 @@ force_split_kernel(ForceJob jb, const float4 *__restrict__ fnode, const int2 *__
         uint64_t takem = ok;
         if (!SOFT) takem &= __ballot(d2 > 0.f);
         const float ri = __builtin_amdgcn_rsqf(SOFT || d2 > 0.f ? d2 : 1.f);
-        float f = q.w * ri * (ri * ri);
+        float f = weight(q.w, ri);
         f = __builtin_amdgcn_inverse_ballot_w64(takem) ? f : 0.f;
         px = fmaf(f, dx, px);
         py = fmaf(f, dy, py);
