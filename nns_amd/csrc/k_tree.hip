@@ -599,10 +599,10 @@ __global__ void __launch_bounds__(T, 6) subtree_build_kernel(
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int nsub = min(__hip_atomic_load(&st->nsub, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT), sub_max);
     const int top = base0 + __hip_atomic_load(&st->ntop, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    // SCAN: the cells of the subtrees [0, to), summed by the workgroup from the counts
-    const auto cells_before = [&](int to) {
+    // SCAN: the cells of the subtrees [from, to), summed by the workgroup from the counts
+    const auto cells_of = [&](int from, int to) {
         int c = 0;
-        for (int j = tid; j < to; j += T) c += (int)cbase[j];
+        for (int j = from + tid; j < to; j += T) c += (int)cbase[j];
         for (int o = 32; o > 0; o >>= 1) c += __shfl_xor(c, o);
         if (lane == 0) s_sum[wave] = c;
         __syncthreads();
@@ -612,15 +612,22 @@ __global__ void __launch_bounds__(T, 6) subtree_build_kernel(
         return c;
     };
     if (SCAN && blockIdx.x == 0) {
-        const int64_t end = (int64_t)top + cells_before(nsub);
+        const int64_t end = (int64_t)top + cells_of(0, nsub);
         if (tid == 0) {
             if (end > m) atomicOr(&st->err, kErrCapacity);
             else *index = (int)end;
         }
     }
-    for (int job = blockIdx.x; job < nsub; job += gridDim.x) {
+    // SCAN: the cells before a job, kept from job to job, so that a workgroup reads every count once
+    uint32_t before = SCAN && (int)blockIdx.x < nsub ? (uint32_t)cells_of(0, blockIdx.x) : 0u;
+    const auto next_of = [&](int job) {
+        const int next = job + (int)gridDim.x;
+        if (SCAN && next < nsub) before += (uint32_t)cells_of(job, next);
+        return next;
+    };
+    for (int job = blockIdx.x; job < nsub; job = next_of(job)) {
         const int4 jb = sub[job];
-        const uint32_t cb0 = SCAN ? cells_before(job) : cbase[job], cb1 = SCAN ? cb0 + cbase[job] : cbase[job + 1];
+        const uint32_t cb0 = SCAN ? before : cbase[job], cb1 = SCAN ? cb0 + cbase[job] : cbase[job + 1];
         const int base = top + (int)cb0, ks = (int)(cb1 - cb0);  // the subtree's own ids
         const int a = jb.x, cnt = jb.y - jb.x, L0 = jb.z, slot = jb.w;
         const bool fits = ks >= 0 && ks < 65536 && cnt <= C * T && build_bytes(ks, cnt) <= POOL;
@@ -1669,11 +1676,13 @@ static int job_grid(int nbodies)
 // 7.5M bodies in 512 systems; build: 30 and 37, 89 and 88, 207 and 177.
 constexpr int kSumTwoPools = 1 << 21, kBuildTwoPools = 1 << 22;
 
-// Up to this many bodies (some 250 subtrees) every workgroup of the build adds up the
-// cells of the subtrees before its own, instead of a launch that scans the counts: nothing
-// to 0.5 us more at 2,000 and 32,768 bodies for a launch of 3.9, 3.8 us more at 150,001 and
-// 4.3 for an ensemble of 96 systems with 100,000.
-constexpr int kBuildScan = 1 << 16;
+// Up to this many bodies (some 250 subtrees) and systems (up to eight subtrees each, however
+// small) every workgroup of the build adds up the cells of the subtrees before its
+// own, instead of a launch that scans the counts: nothing to 0.5 us more at 2,000 and 32,768
+// bodies for a launch of 3.9, 3.8 us more at 150,001 and 4.3 for an ensemble of 96 systems
+// with 100,000.  Each workgroup reads all counts about once, so without the line of the
+// systems 8,192 of 8 bodies would read some 15,000 counts in each of 1,024 workgroups.
+constexpr int kBuildScan = 1 << 16, kBuildScanSystems = 192;
 
 static void build_tree(Segs g, int nsamples, int base0, int m, TreeScratch &ts, DeviceState *st, hipStream_t s,
                        int n, const uint64_t *skeys, const int32_t *perm, const uint64_t *keys,
@@ -1697,7 +1706,7 @@ static void build_tree(Segs g, int nsamples, int base0, int m, TreeScratch &ts, 
     }
     subtree_cells_kernel<<<capped_grid(64 * (int64_t)ts.sub_max, 4096), 256, 0, s>>>(ts.sub, ts.sub_max, ts.lcp,
                                                                                      ts.cbase, st);
-    const bool scan = !locked && g.n <= kBuildScan;
+    const bool scan = !locked && g.n <= kBuildScan && g.nseg <= kBuildScanSystems;
     if (!scan) subtree_base_kernel<<<1, 1024, 0, s>>>(ts.cbase, ts.sub_max, base0, m, index, st);
     const int jobs = job_grid(g.n);
     const auto build_with = [&](auto kernel, int threads) {
