@@ -1311,7 +1311,7 @@ __global__ void __launch_bounds__(kTopThreads) top_summary_kernel(SumOut o, Segs
 // and centre of mass (the FP64 sums of a single child are exact copies), and
 // crit_L + eps^2 falls with L, so a body accepts some cell of the chain exactly
 // when it accepts the bottom one, and meets the same monopole once either way.  fnode
-// keeps the data of the child itself.
+// keeps the data of the child itself (walk_record).
 // Single system: block 0 is the root (slots child[0..7]), block i >= 1 is cell
 // n + i - 1.  Ensemble: block i is cell n + i, the roots being blocks 0..S-1.
 // froot4 / frootm describe each root as a child of a virtual parent.  The
@@ -1435,6 +1435,15 @@ __device__ inline int2 chain_bottom_from(int c, int4 a, int4 b, int lev, int n, 
     }
 }
 
+// A cell's record for the walk, its centre of mass brought into FP32's range (masses that nearly
+// cancel can put it past that).  Its monopole is then 0 at every body, d^2 being infinite, and 0
+// times the distance stays 0 on all of the wave's lanes, also those that do not meet the cell.
+__device__ inline float4 walk_record(const float4 q)
+{
+    constexpr float M = 3.402823466e38f;
+    return make_float4(fminf(fmaxf(q.x, -M), M), fminf(fmaxf(q.y, -M), M), fminf(fmaxf(q.z, -M), M), q.w);
+}
+
 // Ensemble: the system of a cell from its first sorted position (sorting leaves every
 // system's bodies in the system's own positions, so sys_of holds for both orders).
 struct SysInfo {
@@ -1513,7 +1522,7 @@ __global__ void __launch_bounds__(256) frame_layout_kernel(
             th = theta;
         }
         if (k < total && item < nroot && s == 0) {
-            froot4[item] = BATCH ? nodes4[node] : st->root4;
+            froot4[item] = walk_record(BATCH ? nodes4[node] : st->root4);
             frootm[item] = chain_bottom<BATCH>(node, n, child, cell_level, true, span, th, eps2, boff, bsum);
             pblk[item] = -1;
         }
@@ -1526,7 +1535,7 @@ __global__ void __launch_bounds__(256) frame_layout_kernel(
             fmeta[slot] = make_int2(ps << 4, body_crit);
             bpar[ps] = (int)item;
         } else {
-            fnode[slot] = cnode;
+            fnode[slot] = walk_record(cnode);
             fmeta[slot] = chain_bottom_from<BATCH>(ch, ca, cb, clev, n, child, cell_level, span, th, eps2, boff, bsum);
             pblk[block_of<BATCH>(ch, n)] = (int)item;
         }
