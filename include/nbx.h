@@ -252,8 +252,10 @@ int nbx_step(nbx_context *ctx, const nbx_arrays *a, void *stream, float *stage_m
 int nbx_copy_buffer(nbx_context *ctx, int which, void *host_dst, int64_t count, void *stream);
 
 /* Times the force kernel at 2, 4 and 8 waves per block on the current tree (after nbx_sort)
- * and keeps the fastest for this context's later nbx_compute_forces calls.  *waves_out
- * (nullable) receives the choice.  Synchronises the stream. */
+ * and keeps the fastest for this context's later nbx_compute_forces calls.  Up to 5,120
+ * groups of 64 bodies, where the waves of a block share a group and the setting has no
+ * effect, nothing is timed and it stays.  *waves_out (nullable) receives the choice.
+ * Synchronises the stream. */
 int nbx_autotune(nbx_context *ctx, void *stream, int *waves_out);
 
 /* ---- differentiation (no counterpart in the reference) ----------------------------- */

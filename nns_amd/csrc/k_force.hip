@@ -493,6 +493,8 @@ static int split_waves(int ngroups)
     return ngroups <= 640 ? 16 : ngroups <= 2560 ? 8 : ngroups <= 5120 ? 4 : 1;
 }
 
+bool walk_shared(int ngroups) { return split_waves(ngroups) > 1; }
+
 template <bool BATCH>
 static void dispatch(const ForceArgs &a, hipStream_t s, bool kahan, int waves)
 {

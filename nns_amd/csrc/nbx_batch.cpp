@@ -306,6 +306,12 @@ int nbx_batch_autotune(nbx_batch *b, void *stream, int *waves_out)
     nbx::launch_batch_build(b, s);
     nbx::launch_batch_summarize(b, s);
     nbx::launch_batch_layout(b, s);
+    if (nbx::walk_shared(b->ngroups)) {  // no choice to make: the setting stays
+        if (hipStreamSynchronize(s) != hipSuccess) return bfail(b, NBX_ERR_HIP, "hipStreamSynchronize");
+        drop_graph(b);
+        if (waves_out) *waves_out = b->force_waves;
+        return finish(b);
+    }
     const int cand[3] = {2, 4, 8};
     float best = 1e30f;
     int pick = b->force_waves;
@@ -370,6 +376,14 @@ int nbx_autotune(nbx_context *c, void *stream, int *waves_out)
     }
     hipSetDevice(c->device);
     hipStream_t s = (hipStream_t)stream;
+    if (nbx::walk_shared((c->n + 63) / 64)) {  // no choice to make: the setting stays
+        if (hipStreamSynchronize(s) != hipSuccess) {
+            c->last_error = "hipStreamSynchronize failed";
+            return NBX_ERR_HIP;
+        }
+        if (waves_out) *waves_out = c->force_waves;
+        return NBX_OK;
+    }
     const int cand[3] = {2, 4, 8};
     float best = 1e30f;
     int pick = c->force_waves;

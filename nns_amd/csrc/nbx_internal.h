@@ -315,6 +315,9 @@ constexpr int kGroupLevels = 10;
 // group, the child steps and frames of its walk.
 void launch_force(nbx_context *c, hipStream_t s, float *ax, float *ay, float *az, float g, int64_t *counts,
                   int64_t *walk = nullptr);
+// Whether a launch of that many groups shares each among the waves of a workgroup, whose number
+// then follows from the groups, not from force_waves.
+bool walk_shared(int ngroups);
 void launch_force_waves(nbx_context *c, hipStream_t s, float *ax, float *ay, float *az, float g, int waves);
 
 // batched form (k_basic.hip, k_sort.hip, k_tree.hip, k_force.hip)
