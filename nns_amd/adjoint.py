@@ -2,7 +2,7 @@
 
 * ``BarnesHutAccel`` -- torch.autograd.Function: accelerations of bodies at
   (x, y, z) with masses m; its backward is ``nbx_force_vjp`` on the tree of the
-  same positions (rebuilt if the context has walked another tree since).
+  same positions, which it builds again (the slot may have walked another since).
 * ``Rollout`` -- K steps of the reference's integrator (v += dt a; x += d dt v,
   3D/CUDA/CUDA_NBody/src/Kernels.cu:581-600, here with d = 1) as one autograd
   node.  Its backward is the discrete adjoint of that map,

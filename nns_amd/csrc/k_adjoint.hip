@@ -737,10 +737,14 @@ static int sort_passes(int64_t id_max)
 }
 
 // Waves per group of the walk (the force launch's rule, with more work per frame
-// and so a later end): sphere of 20,011 (313 groups) 216 us with 16 waves, 254 with 8,
-// 838 with one; 65,536 (1,024) 425, 423, 1035; 262,144 (4,096) 1750 with 16, 1595
-// with 8, 1622 with 4, 1956 with one; 524,288 (8,192) 3327 with 8, 3204 with 4, 3386
-// with one; 1,048,576 (16,384) 6826 with 4, 6680 with one (whole VJP).
+// and so a later end).  Whole product, us: a sphere and a binary + disk at theta 0.5, with
+//   16 and 8 waves:  480 groups 236, 277; 121, 143.   640 groups 321, 341; 155, 165.   1,024
+//                    groups 426, 439; 213, 220 (at theta 0.8 the sphere 212, 210)
+//   8 and 4 waves:   4,096 groups 1,581, 1,586; 741, 786.   5,120 groups 2,035, 2,008; 984,
+//                    1,008.   8,192 groups 3,292, 3,187; 1,556, 1,528
+//   4 and 1 wave:    8,192 groups 3,187, 3,310; 1,528, 1,746.   12,288 groups 4,915, 4,963;
+//                    2,397, 2,434.   16,384 groups 6,826, 6,680 (sphere)
+// Between 640 and 1,024 groups 16 waves and 8 differ by no more than 6 %.
 static int vjp_split(int ngroups)
 {
     return ngroups <= 640 ? 16 : ngroups <= 5120 ? 8 : ngroups <= 10240 ? 4 : 1;

@@ -349,11 +349,11 @@ static void launch_w(const ForceArgs &a, hipStream_t s, int waves)
 // groups of an XCD are consecutive.  Every wave sums its own frames as above,
 // the compensated totals of the waves are added in wave order.  Bound by the
 // length of the longest group's chain of rounds (about 1,500 clocks each: the
-// block's trip to the L2, five child steps, the barrier).  Force kernel, one
-// wave per group against S waves: star + disk N = 2,000, 75 -> 18 us (S = 16);
-// 20,011-body sphere 338 -> 84 (16); 32,768-body disk 168 -> 37 (16); sphere
-// 65,536, 395 -> 149 (8); sphere 150,001 at theta 0.7, 240 -> 174 (8);
-// binary + disk 300,007 unsoftened at theta 0.3, 1089 -> 700 (4).
+// block's trip to the L2, five child steps, the barrier).  Forces with one
+// wave per group against S waves: star + disk N = 2,000, 69 -> 17 us (S = 16);
+// 20,011-body sphere 295 -> 73 (16); 32,768-body disk 149 -> 35 (16); sphere
+// 65,536, 337 -> 148 (8); sphere 150,001 at theta 0.7, 197 -> 161 (8);
+// binary + disk 294,912 unsoftened at theta 0.3, 966 -> 668 (4).
 // The register budget of eight waves per SIMD is worth a few reloads: with 94
 // scalar registers (seven waves) the same kernel was 5-15 % slower, with S = 16
 // 30 % (one workgroup per CU instead of two).
@@ -484,10 +484,16 @@ static void launch_split(const ForceArgs &a, hipStream_t s, int S)
 // Waves per group.  As many as fill the device (256 CUs of 32 waves) about once,
 // 16 at most.  Each round costs a barrier and the hand-out of the frames, so once
 // the waves of one-wave groups fill the device by themselves the shared walk only
-// adds work.  Force stage in us with one wave per group, 4 and 8: 2,560 groups, sphere
-// 419, 367, 348, disk 293, 192, 171; 4,096 groups 533, 521, 535 and 362, 261, 255; 5,120
-// groups 612, 641, 670 and 393, 352, 346; 8,192 groups 900, 1,018, 1,089 and 512, 515,
-// 539.  16 waves: 1,024 groups 176 us against 161 with 8; 313 groups 84 against 96.
+// adds work.  Where that is depends on the bodies, which the rule does not see: the
+// walks of a disk differ more in length than those of a sphere, and sharing them pays for
+// longer.  Each line lies where a sphere starts to lose, or shortly past it where disks gain
+// more (the last).  Computing the forces, us: a sphere at theta 0.5, a binary + disk at
+// theta 0.5 and one at 0.3 unsoftened, with
+//   16 and 8 waves:  640 groups 116, 117; 49, 52; 80, 93.   800 groups 142, 138; 59, 61; 97, 105
+//   8 and 4 waves:   2,560 groups 341, 364; 166, 187; 336, 391.   3,584 groups 470, 470; 224,
+//                    232; 459, 494.   4,096 groups 535, 516; 250, 256; 499, 558
+//   4 and 1 wave:    4,608 groups 585, 608; 308, 387; 668, 966.   5,120 groups 636, 618; 342,
+//                    390; 746, 956.   6,144 groups 756, 704; 369, 453; 801, 1,068
 static int split_waves(int ngroups)
 {
     return ngroups <= 640 ? 16 : ngroups <= 2560 ? 8 : ngroups <= 5120 ? 4 : 1;

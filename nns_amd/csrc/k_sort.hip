@@ -297,9 +297,14 @@ __global__ void __launch_bounds__(kMergeThreads) merge_pass_kernel(const uint64_
 // 64 keys each, and the others search between them, four chunks side by side.  Bound by
 // the chain of loads, about 7 us per four chunks, where each doubling of the runs costs a
 // launch of 8 us; every wave meets every chunk, so the work grows with the square of the
-// chunks.  Sort of n pairs, merge passes and this: n = 8,192, 29.4 and 28.9 us;
-// 20,000, 44 and 30; 36,864, 53 and 35; 69,632 (17 chunks), 61 and 48; 150,000, 84 and
-// 114; an ensemble of 7.5M pairs in chunks by at most 16, 419 and 673.
+// chunks, and a last chunk that is not full takes longer (a sixth of it filled, below).  Sort of
+// n pairs, merge passes and this, the last chunk full and not: 2 chunks, 29.8 and 29.1 us, 28.6
+// and 30.4; 4 chunks, 37.6 and 30.0, 37.4 and 31.2; 12 chunks, 53.5 and 40.3, 53.6 and 46.3;
+// 16 chunks, 53.8 and 45.9, 53.8 and 54.2; 17 chunks, 60.9 and 48.7, 60.3 and 56.9; 18 chunks,
+// 61.4 and 53.8, 61.7 and 62.4; 22 chunks, 62.0 and 60.3, 61.9 and 71.2; 26 chunks, 62.7 and
+// 66.4, 62.1 and 78.2.  The line
+// lies below the first count from which on a chunk that is not full only loses.  An ensemble of
+// 7.5M pairs in chunks by at most 16, 419 and 673.
 constexpr int kRankThreads = 256, kRankWidth = 4;
 constexpr int kRankChunks = 17, kRankPairs = 1 << 17;
 

@@ -14,11 +14,12 @@
 //      from the sorted keys by searches (one thread per sample of
 //      kSubtreeMax bodies) and wired with their child ranges;
 //   2. every child range of a top cell with 2..kSubtreeMax bodies is a subtree
-//      built by ONE wave from the shared-digit counts of neighbouring keys:
-//      cell ids from a prefix sum, parents from previous-smaller-value queries,
-//      one plain store per child slot (subtree_build_kernel).  Every subtree's
-//      exact cell count is known first (from the shared-digit counts), and one
-//      scan of the counts gives each its block of cell ids.
+//      built by one workgroup from the shared-digit counts of neighbouring keys:
+//      cell ids from a prefix sum, parents from searches over the keys in LDS, the
+//      child slots filled in LDS and copied out (subtree_build_kernel).  Every subtree's
+//      exact cell count is known first (from the shared-digit counts), and their
+//      sums give each its block of cell ids: by a scan of its own, or up to kBuildScan
+//      bodies summed by the build's workgroups.
 //      The lock-based insertion (compare-and-swap on child slots, -2 = locked,
 //      at workgroup scope; subtree_insert_kernel) builds the same cells when
 //      nbx_params.build_locked is set;
@@ -316,11 +317,11 @@ __global__ void __launch_bounds__(256) top_wire_kernel(
 // builds reject counts 0); subtree_base_kernel turns the counts into the
 // exclusive sum cbase[] (cbase[nsub] the total) and sets *index past the last
 // subtree cell, so subtree j owns the ids from base0 + ntop + cbase[j] (after
-// the top cells).  Each build workgroup reads its base instead of taking it from
-// one shared counter: the device-scope atomics of a shared counter are
-// serialised, one per subtree.  A build that counts other than cbase[j + 1] -
-// cbase[j] cells for its subtree latches kErrCapacity and leaves it unbuilt, so
-// no two subtrees can share an id.
+// the top cells).  (Where the build sums the counts itself, cbase[] keeps them and the
+// build does the rest.)  Each build workgroup reads or sums its base instead of taking it
+// from one shared counter: the device-scope atomics of a shared counter are
+// serialised, one per subtree.  A build that counts other than its subtree's number of
+// cells latches kErrCapacity and leaves it unbuilt, so no two subtrees can share an id.
 __global__ void __launch_bounds__(256) subtree_cells_kernel(const int4 *__restrict__ sub, int sub_max,
                                                             const uint8_t *__restrict__ lcp,
                                                             uint32_t *__restrict__ cbase, const DeviceState *st)

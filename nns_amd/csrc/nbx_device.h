@@ -244,21 +244,6 @@ __device__ inline int frame_off(const uint32_t *__restrict__ boff, const uint32_
 // ---------------------------------------------------------------- tree
 static __device__ inline int digit_at(uint64_t key, int level) { return (int)((key >> (60 - 3 * level)) & 7u); }
 
-static __device__ inline int ld_slot(const int *p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-static __device__ inline void st_slot(int *p, int v)
-{
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-static __device__ inline int cas_slot(int *p, int expect, int desired)
-{
-    __hip_atomic_compare_exchange_strong(p, &expect, desired, __ATOMIC_RELAXED, __ATOMIC_RELAXED,
-                                         __HIP_MEMORY_SCOPE_AGENT);
-    return expect;  // value found (== the expected value on success)
-}
-
 static __device__ inline int latched(const DeviceState *st)
 {
     return __hip_atomic_load(&st->err, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

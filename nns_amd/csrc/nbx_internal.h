@@ -24,7 +24,6 @@ constexpr int kSortTile = kSortThreads * kSortItems;
 // A cell at level L is opened at most once per path and pushes at most 8 children,
 // so the stack never holds more than 8 + 7*21 = 155 entries.
 constexpr int kForceStack = 160;
-constexpr int kRootRef = 0x7fffffff;
 
 // Device-side error latch bits (mapped to NBX_ERR_* on the host).
 constexpr int kErrCapacity = 1;
