@@ -1085,7 +1085,7 @@ __global__ void __launch_bounds__(T, POOL == kSumSmall ? 8 : 4) subtree_summary_
 // top_levels_kernel hold no LDS to speak of and 256 threads, so 64 fit any partition of an MI355X
 // (32 CUs at least) twice over, beside other kernels and launches of their own kind; the
 // LDS part, whose workgroup takes a CU for itself, is a launch of its own (a step of 1M
-// bodies 2,036 us, with both in one launch 2,034).  The wait is bounded all the same: one that
+// bodies 2,022 us, with both in one launch 2,014).  The wait is bounded all the same: one that
 // runs out latches kErrStall, and every wave still finishes.
 constexpr int kTopBlocks = 64, kTopLevelThreads = 256;
 // Up to kTopOneGroup bodies there are hardly ever many more top cells than fit, and
@@ -1129,8 +1129,8 @@ __device__ inline void top_barrier(DeviceState *st, int phase, bool &stalled)
 // front, all side by side, and an item that is summed puts its own into its parent's.
 // Eight lanes per item, of which four add one component each, in slot order.
 // (Level by level in memory, with four times as many write-backs of the L2 at a barrier:
-// 150,001 bodies 23 us, now 10; 1M: 49 and 23; 4M: 48 and 32; 7.5M in 512 systems: 100
-// and 76.)
+// 150,001 bodies 23 us, now 11; with the levels before it 1M: 49, now 12 + 16; 4M: 48, now
+// 23 + 14; 7.5M in 512 systems: 100, now 61 + 20.)
 constexpr int kTopThreads = 512;
 template <int ITEMS>
 struct TopLds {
